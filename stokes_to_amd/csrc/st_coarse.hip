@@ -1,0 +1,811 @@
+// Kernels of the multigrid levels that are not marched plane by plane: the levels below
+// 128 cells a side under a finer one, every 2D level and the small 3D grids, and the
+// fused cycle of the coarsest levels.
+//
+// These levels fit the caches, and what bounds a pass on them is the number of vector
+// instructions (a wave64 instruction holds a CDNA SIMD for four cycles) and the latency
+// of one dependent chain, not bytes.  So nodes are addressed by a 32-bit offset from
+// per-field scalar bases, index splits are shifts (every level side is a power of two)
+// and each lane does useful work (a colour pass has one lane per pair of cells, one of
+// each colour).  The arithmetic is that of the per-node kernels of st_kernels.hip in
+// the same order (st_box.h).
+//
+// Against the kernels with 64-bit indices, a lane per node and range tests per access,
+// us per launch in FP64 / FP32: colour pass 64^3 23.7 / 17.2 -> 9.9 / 7.8, 32^3 9.5 / 8.3
+// -> 4.6 / 4.3, 16^3 8.9 / 7.8 -> 4.4 / 4.2, 2D 256^2 FP32 6.9 -> 5.7 (finest level),
+// 64^2 6.4 -> 3.6; residual and restriction 32^3 7.4 + 4.9 -> 7.8 in one launch, 64^2 FP32
+// 4.3 + 3.6 -> 3.9.  About 3 us of each is the launch and one trip to memory.
+#include "st_box.h"
+#include "st_kernels.h"
+
+namespace st {
+
+namespace {
+
+// value at a 32-bit element offset from a uniform base
+template <typename T> __device__ __forceinline__ T at(const T *p, unsigned i)
+{
+    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + i * (unsigned)sizeof(T));
+}
+template <typename T> __device__ __forceinline__ void put(T *p, unsigned i, T v)
+{
+    *reinterpret_cast<T *>(reinterpret_cast<char *>(p) + i * (unsigned)sizeof(T)) = v;
+}
+
+// accessor of a cell (i, j, k all below the level's side) in the node layout: at most
+// one offset is negative; below the grid it reads the own node and F, p are 0; the
+// only node past the box that a cell's rows name is i + 2 (in the last cell plane)
+template <typename TS, int DIM, bool M> struct CellAcc {
+    typedef typename Cvt<TS>::C C;
+    static constexpr bool MASK = M;
+    const uint8_t *fl;
+    const TS *x, *b, *al;
+    long S, sI, sJ;
+    unsigned q, qi, qj, qk;  // own node; the node below along each axis (own at the edge)
+    bool li, lj, lk, hi;     // first cell along an axis, last along i
+
+    __device__ __forceinline__ CellAcc(const Lvl &g, const uint8_t *f, const TS *a, const TS *bb, const TS *xx, int i,
+                                       int j, int k)
+        : fl(f), x(xx), b(bb), al(a), S(g.S), sI((long)g.Py * g.Pz), sJ(g.Pz)
+    {
+        q = ((unsigned)i * (unsigned)g.Py + (unsigned)j) * (unsigned)g.Pz + (unsigned)k;
+        li = i == 0;
+        lj = j == 0;
+        lk = k == 0;
+        hi = i == g.nx - 1;
+        qi = li ? q : q - (unsigned)sI;
+        qj = lj ? q : q - (unsigned)sJ;
+        qk = lk ? q : q - 1u;
+    }
+    // lane part and uniform part of the offset of a neighbour
+    __device__ __forceinline__ unsigned lane(int di, int dj, int dk) const
+    { return di < 0 ? qi : (dj < 0 ? qj : (dk < 0 ? qk : q)); }
+    __device__ __forceinline__ long uni(int di, int dj, int dk) const
+    { return (di > 0 ? di * sI : 0) + (dj > 0 ? dj * sJ : 0) + (dk > 0 ? dk : 0); }
+    __device__ __forceinline__ bool out(int di, int dj, int dk) const
+    { return (di < 0 && li) || (dj < 0 && lj) || (dk < 0 && lk) || (di > 1 && hi); }
+
+    __device__ __forceinline__ int F(int di, int dj, int dk) const
+    {
+        if (di > 1) {  // one plane short of i + 2 in the last cell plane, and discarded
+            const int f = at(fl + sI, hi ? q : q + (unsigned)sI);
+            return hi ? 0 : f;
+        }
+        const int f = at(fl + uni(di, dj, dk), lane(di, dj, dk));
+        return out(di, dj, dk) ? 0 : f;
+    }
+    __device__ __forceinline__ C X(int f, int di, int dj, int dk) const
+    {
+        // i + 2 of u_x in the last cell plane lies in u_y's first plane: in bounds, and it
+        // enters only the divergence of the cell i + 1, whose flag is 0 there
+        const C v = Cvt<TS>::ld(at(x + f * S + uni(di, dj, dk), lane(di, dj, dk)));
+        return ((f == 0 || !MASK) && out(di, dj, dk)) ? C(0) : v;
+    }
+    __device__ __forceinline__ C B(int f, int di, int dj, int dk) const
+    { return Cvt<TS>::ld(at(b + f * S + uni(di, dj, dk), q)); }
+    __device__ __forceinline__ C AL(int d, int di, int dj, int dk) const
+    { return Cvt<TS>::ld(at(al + d * S + uni(di, dj, dk), q)); }
+};
+
+// accessor of any node of the box: offsets in -1..1 per axis, 0 outside the box
+template <typename TS, int DIM, bool M> struct NodeAcc {
+    typedef typename Cvt<TS>::C C;
+    static constexpr bool MASK = M;
+    const uint8_t *fl;
+    const TS *x, *al;
+    long S;
+    unsigned q, im, ip, jm, jp, km, kp;  // steps to the neighbours (0 at the edge)
+    bool li, lj, lk, hi, hj, hk;
+
+    __device__ __forceinline__ NodeAcc(const Lvl &g, const uint8_t *f, const TS *a, const TS *xx, int i, int j, int k)
+        : fl(f), x(xx), al(a), S(g.S)
+    {
+        const unsigned sI = (unsigned)g.Py * (unsigned)g.Pz, sJ = (unsigned)g.Pz;
+        q = (unsigned)i * sI + (unsigned)j * sJ + (unsigned)k;
+        li = i == 0; lj = j == 0; lk = k == 0;
+        hi = i == g.nx; hj = j == g.ny; hk = (DIM == 2) || k >= g.nz;
+        im = li ? 0u : sI; ip = hi ? 0u : sI;
+        jm = lj ? 0u : sJ; jp = hj ? 0u : sJ;
+        km = lk ? 0u : 1u; kp = hk ? 0u : 1u;
+    }
+    __device__ __forceinline__ unsigned node(int di, int dj, int dk) const
+    {
+        return q + (di > 0 ? ip : 0u) + (dj > 0 ? jp : 0u) + (dk > 0 ? kp : 0u) - (di < 0 ? im : 0u) -
+               (dj < 0 ? jm : 0u) - (dk < 0 ? km : 0u);
+    }
+    __device__ __forceinline__ bool out(int di, int dj, int dk) const
+    {
+        return (di < 0 && li) || (dj < 0 && lj) || (dk < 0 && lk) || (di > 0 && hi) || (dj > 0 && hj) || (dk > 0 && hk);
+    }
+    __device__ __forceinline__ int F(int di, int dj, int dk) const
+    {
+        const int f = at(fl, node(di, dj, dk));
+        return out(di, dj, dk) ? 0 : f;
+    }
+    __device__ __forceinline__ C X(int f, int di, int dj, int dk) const
+    {
+        const C v = Cvt<TS>::ld(at(x + f * S, node(di, dj, dk)));
+        return ((f == 0 || !MASK) && out(di, dj, dk)) ? C(0) : v;
+    }
+    __device__ __forceinline__ C AL(int d, int di, int dj, int dk) const
+    { return Cvt<TS>::ld(at(al + d * S, node(di, dj, dk))); }
+};
+
+}  // namespace
+
+// ------------------------------------------------------------ colour pass
+
+// One colour of the smoother, xin -> xout, one lane per pair of cells along the fastest
+// axis: the lane solves the block of the pair's colour cell and copies what the colour
+// does not own (the other cell's p, and its faces on the domain boundary).  lg: log2 of
+// the level side.  ZERO: xin is zero and not read.
+template <typename TS, int DIM, bool ZERO, bool MASK>
+__global__ void __launch_bounds__(256) k_box(Lvl g, int lg, const uint8_t *__restrict__ fl, const TS *__restrict__ al,
+                                             const TS *__restrict__ b, const TS *__restrict__ xin,
+                                             TS *__restrict__ xout, int color, float omega)
+{
+    typedef typename Cvt<TS>::C C;
+    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (1u << (DIM * lg - 1))) return;
+    const int m = (1 << lg) - 1;
+    const int pr = (int)(t & (unsigned)(m >> 1)) * 2;  // even cell of the pair along the fastest axis
+    int i, j, k, oj, ok;                               // the colour cell; (i, oj, ok) the other one
+    if (DIM == 3) {
+        j = oj = (int)(t >> (lg - 1)) & m;
+        i = (int)(t >> (2 * lg - 1));
+        k = pr + ((i + j + color) & 1);
+        ok = 2 * pr + 1 - k;
+    } else {
+        i = (int)(t >> (lg - 1));
+        j = pr + ((i + color) & 1);
+        oj = 2 * pr + 1 - j;
+        k = ok = 0;
+    }
+    const CellAcc<TS, DIM, MASK> a(g, fl, al, b, xin, i, j, k);
+    C pn, u0[3], u1[3];
+    box_cell<C, DIM, ZERO>(a, omega, pn, u0, u1);
+    const long st[3] = {a.sI, a.sJ, 1};
+    // copy-through first (its loads are independent of the solve)
+    const unsigned qo = a.q + (DIM == 3 ? (unsigned)(ok - k) : (unsigned)(oj - j));
+    auto cp = [&](int f, long off) {
+        TS v;
+        if (ZERO) v = Cvt<TS>::st(C(0));
+        else v = at(xin + f * g.S + off, qo);
+        put(xout + f * g.S + off, qo, v);
+    };
+    cp(0, 0);
+    if (i == 0) cp(1, 0);
+    if (i == g.nx - 1) cp(1, st[0]);
+    if (oj == 0) cp(2, 0);
+    if (oj == g.ny - 1) cp(2, st[1]);
+    if (DIM == 3) {
+        if (ok == 0) cp(3, 0);
+        if (ok == g.nz - 1) cp(3, st[2]);
+    }
+    put(xout, a.q, Cvt<TS>::st(pn));
+#pragma unroll
+    for (int d = 0; d < DIM; d++) {
+        put(xout + (1 + d) * g.S, a.q, Cvt<TS>::st(u0[d]));
+        put(xout + (1 + d) * g.S + st[d], a.q, Cvt<TS>::st(u1[d]));
+    }
+}
+
+// ------------------------------------------------------ operator, residual
+
+// node of a linear index over the padded box (rows of Pz)
+template <int DIM> __device__ __forceinline__ void box_node(const Lvl &g, unsigned n, int &i, int &j, int &k)
+{
+    if (DIM == 3) {
+        const unsigned t = n / (unsigned)g.Pz;
+        k = (int)(n - t * (unsigned)g.Pz);
+        i = (int)(t / (unsigned)g.Py);
+        j = (int)(t - (unsigned)i * (unsigned)g.Py);
+    } else {
+        i = (int)(n / (unsigned)g.Py);
+        j = (int)(n - (unsigned)i * (unsigned)g.Py);
+        k = 0;
+    }
+}
+
+// y = A x, one node per lane (these levels have no row padding)
+template <typename TS, int DIM>
+__global__ void __launch_bounds__(256) k_apply(Lvl g, const uint8_t *__restrict__ fl, const TS *__restrict__ al,
+                                               const TS *__restrict__ x, TS *__restrict__ y)
+{
+    typedef typename Cvt<TS>::C C;
+    const unsigned n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= (unsigned)g.S) return;
+    int i, j, k;
+    box_node<DIM>(g, n, i, j, k);
+    const NodeAcc<TS, DIM, true> a(g, fl, al, x, i, j, k);
+    const BoxSten<C, DIM, NodeAcc<TS, DIM, true>> s{a};
+    put(y, n, Cvt<TS>::st(s.cell()));
+    put(y + g.S, n, Cvt<TS>::st(s.template face<0>(0, 0, 0)));
+    put(y + 2 * g.S, n, Cvt<TS>::st(s.template face<1>(0, 0, 0)));
+    if (DIM == 3) put(y + 3 * g.S, n, Cvt<TS>::st(s.template face<2>(0, 0, 0)));
+}
+
+// r = b - A x (without r: the norm only), and the block's partial sum of |r|^2
+template <typename TS, int DIM>
+__global__ void __launch_bounds__(256) k_residual(Lvl g, const uint8_t *__restrict__ fl, const TS *__restrict__ al,
+                                                  const TS *__restrict__ b, const TS *__restrict__ x, TS *r,
+                                                  double *part)
+{
+    typedef typename Cvt<TS>::C C;
+    __shared__ double sh[4];
+    const unsigned n = blockIdx.x * blockDim.x + threadIdx.x;
+    double acc = 0.0;
+    if (n < (unsigned)g.S) {
+        int i, j, k;
+        box_node<DIM>(g, n, i, j, k);
+        const NodeAcc<TS, DIM, true> a(g, fl, al, x, i, j, k);
+        const BoxSten<C, DIM, NodeAcc<TS, DIM, true>> s{a};
+        C v[4];
+        v[0] = Cvt<TS>::ld(at(b, n)) - s.cell();
+        v[1] = Cvt<TS>::ld(at(b + g.S, n)) - s.template face<0>(0, 0, 0);
+        v[2] = Cvt<TS>::ld(at(b + 2 * g.S, n)) - s.template face<1>(0, 0, 0);
+        if (DIM == 3) v[3] = Cvt<TS>::ld(at(b + 3 * g.S, n)) - s.template face<2>(0, 0, 0);
+#pragma unroll
+        for (int f = 0; f <= DIM; f++) {
+            if (r) put(r + f * g.S, n, Cvt<TS>::st(v[f]));
+            acc += (double)v[f] * v[f];
+        }
+    }
+    if (part) {
+        for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
+        if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = acc;
+        __syncthreads();
+        if (threadIdx.x == 0) part[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
+    }
+}
+
+// ----------------------------------------------------------- prolongation
+
+// xf += P ec on the free DOFs (pressure correction scaled by 1/2).  A lane takes the
+// two fine nodes over one coarse entry of the fastest axis, whose coarse values they
+// share; V2: rows start on even entries, and the pair moves in one access per field.
+template <typename T> struct alignas(2 * sizeof(T)) Two {
+    T v[2];
+};
+template <typename TS, int DIM, bool V2>
+__global__ void __launch_bounds__(256) k_prolong(Lvl gf, Lvl gc, const uint8_t *__restrict__ flf,
+                                                 const TS *__restrict__ ec, TS *__restrict__ xf)
+{
+    typedef typename Cvt<TS>::C C;
+    const unsigned m = (unsigned)(DIM == 3 ? gc.nz : gc.ny) + 1u;  // coarse entries of a row
+    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned row = t / m, e = t - row * m;                    // fine row: i (2D) or i, j
+    if (row >= (unsigned)(DIM == 3 ? gf.Px * gf.Py : gf.Px)) return;
+    const unsigned i = DIM == 3 ? row / (unsigned)gf.Py : row, j = DIM == 3 ? row - i * (unsigned)gf.Py : 2u * e;
+    const unsigned rowlen = (unsigned)(DIM == 3 ? gf.nz : gf.ny) + 1u, pitch = (unsigned)(DIM == 3 ? gf.Pz : gf.Py);
+    const unsigned q = row * pitch + 2u * e;
+    const unsigned qc = DIM == 3 ? ((i >> 1) * (unsigned)gc.Py + (j >> 1)) * (unsigned)gc.Pz + e
+                                 : (i >> 1) * (unsigned)gc.Py + e;
+    const bool two = 2u * e + 1u < rowlen;  // the last entry of a row is alone
+    const long sc[3] = {(long)gc.Py * gc.Pz, (long)gc.Pz, 1};
+    constexpr int fast = DIM - 1;  // axis of the pair
+    int fb[2];
+    if (V2) {
+        const Two<uint8_t> w = *reinterpret_cast<const Two<uint8_t> *>(flf + q);
+        fb[0] = w.v[0];
+        fb[1] = two ? w.v[1] : 0;
+    } else {
+        fb[0] = at(flf, q);
+        fb[1] = two ? (int)at(flf, q + 1u) : 0;
+    }
+    const unsigned co[3] = {i, j, 2u * e};
+#pragma unroll
+    for (int f = 0; f <= DIM; f++) {
+        C c0 = Cvt<TS>::ld(at(ec + f * gc.S, qc)), c1;
+        if (f == 0) {
+            c0 = C(0.5) * c0;
+            c1 = c0;
+        } else if (f - 1 == fast) {
+            c1 = c0 + Cvt<TS>::ld(at(ec + f * gc.S, two ? qc + 1u : qc));
+            c1 *= C(0.5);
+        } else {
+            const bool odd = co[f - 1] & 1u;
+            const C h = Cvt<TS>::ld(at(ec + f * gc.S, odd ? qc + (unsigned)sc[f - 1] : qc));
+            if (odd) {
+                c0 = c0 + h;
+                c0 *= C(0.5);
+            }
+            c1 = c0;
+        }
+        // loads before the flag tests: a lane waits once
+        TS *xp = xf + f * gf.S;
+        const bool on0 = (fb[0] >> f) & 1, on1 = (fb[1] >> f) & 1;
+        if (V2) {
+            Two<TS> w = *reinterpret_cast<const Two<TS> *>(xp + q);
+            if (on0) w.v[0] = Cvt<TS>::st(Cvt<TS>::ld(w.v[0]) + c0);
+            if (on1) w.v[1] = Cvt<TS>::st(Cvt<TS>::ld(w.v[1]) + c1);
+            if (on0 || on1) *reinterpret_cast<Two<TS> *>(xp + q) = w;
+        } else {
+            const unsigned q1 = two ? q + 1u : q;
+            const TS w0 = at(xp, q), w1 = at(xp, q1);
+            if (on0) put(xp, q, Cvt<TS>::st(Cvt<TS>::ld(w0) + c0));
+            if (on1) put(xp, q1, Cvt<TS>::st(Cvt<TS>::ld(w1) + c1));
+        }
+    }
+}
+
+// ------------------------------------------------- residual + restriction
+
+// Coarse right-hand side R (b - A x) in one launch: a workgroup evaluates the fine
+// residual on the (2 CI + 1) x (2 CJ + 1) x (2 CK + 1) nodes under its CI x CJ x CK
+// coarse nodes into LDS (rounded to the storage type, as a stored residual is) and
+// restricts from there with restrict_body's sums.  The residual never reaches memory
+// and one launch of each level's cycle is saved; 1.3-1.5 of the residual rows are
+// evaluated twice, which on these levels is cheaper than a launch.
+template <int DIM> struct RrTile {  // NT: one lane per residual node
+    static constexpr int CI = DIM == 3 ? 2 : 4, CJ = DIM == 3 ? 4 : 16, CK = DIM == 3 ? 8 : 1;
+    static constexpr int FI = 2 * CI + 1, FJ = 2 * CJ + 1, FK = DIM == 3 ? 2 * CK + 1 : 1, N = FI * FJ * FK;
+    static constexpr int NT = (N + 63) / 64 * 64;
+};
+
+// row f of the restriction at a free coarse DOF (else 0) from the residual r of field f
+// around the fine node of the coarse node, strides sI, sJ, sK: the sums of restrict_body
+// in its order (along the face normal, then the two axes across in (i, j, k) order)
+template <typename TS, int DIM>
+__device__ __forceinline__ typename Cvt<TS>::C restrict_from(const TS *r, int f, int sI, int sJ, int sK, bool free)
+{
+    typedef typename Cvt<TS>::C C;
+    if (!free) return C(0);
+    C s = C(0);
+    if (f == 0) {
+        for (int a = 0; a < 2; a++)
+            for (int b = 0; b < 2; b++)
+                for (int c = 0; c < (DIM == 3 ? 2 : 1); c++) s += Cvt<TS>::ld(r[a * sI + b * sJ + c * sK]);
+        return s * ((DIM == 3) ? C(0.25) : C(0.5));
+    }
+    const int so = f == 1 ? sI : (f == 2 ? sJ : sK), su = f == 1 ? sJ : sI, sv = f == 3 ? sJ : sK;
+    for (int on = -1; on <= 1; on++) {
+        const C w = (on == 0) ? C(1) : C(0.5);
+        for (int a = 0; a < 2; a++)
+            for (int b = 0; b < (DIM == 3 ? 2 : 1); b++) s += w * Cvt<TS>::ld(r[on * so + a * su + b * sv]);
+    }
+    return s * ((DIM == 3) ? C(0.5) : C(1.0));
+}
+
+template <typename TS, int DIM, bool MASK>
+__global__ void __launch_bounds__(RrTile<DIM>::NT) k_resid_restrict(Lvl gf, Lvl gc, const uint8_t *__restrict__ flf,
+                                                          const TS *__restrict__ al, const TS *__restrict__ b,
+                                                          const TS *__restrict__ x, const uint8_t *__restrict__ flc,
+                                                          TS *__restrict__ bc)
+{
+    typedef typename Cvt<TS>::C C;
+    typedef RrTile<DIM> T;
+    __shared__ TS sr[DIM + 1][T::N];
+    const int K0 = blockIdx.x * T::CK, J0 = blockIdx.y * T::CJ, I0 = blockIdx.z * T::CI;
+    if (const int t = threadIdx.x; t < T::N) {
+        const int c = t % T::FK, r = t / T::FK;
+        const int i = 2 * I0 - 1 + r / T::FJ, j = 2 * J0 - 1 + r % T::FJ, k = DIM == 3 ? 2 * K0 - 1 + c : 0;
+        C v[4] = {C(0), C(0), C(0), C(0)};
+        if (i >= 0 && j >= 0 && k >= 0 && i <= gf.nx && j <= gf.ny && (DIM == 2 || k <= gf.nz)) {
+            const NodeAcc<TS, DIM, MASK> a(gf, flf, al, x, i, j, k);
+            const BoxSten<C, DIM, NodeAcc<TS, DIM, MASK>> s{a};
+            v[0] = Cvt<TS>::ld(at(b, a.q)) - s.cell();
+            v[1] = Cvt<TS>::ld(at(b + gf.S, a.q)) - s.template face<0>(0, 0, 0);
+            v[2] = Cvt<TS>::ld(at(b + 2 * gf.S, a.q)) - s.template face<1>(0, 0, 0);
+            if (DIM == 3) v[3] = Cvt<TS>::ld(at(b + 3 * gf.S, a.q)) - s.template face<2>(0, 0, 0);
+        }
+#pragma unroll
+        for (int f = 0; f <= DIM; f++) sr[f][t] = Cvt<TS>::st(v[f]);
+    }
+    __syncthreads();
+    constexpr int NC = T::CI * T::CJ * T::CK;
+    for (int t = threadIdx.x; t < NC * (DIM + 1); t += T::NT) {
+        const int f = t / NC, n = t % NC;
+        const int dK = n % T::CK, dJ = (n / T::CK) % T::CJ, dI = n / (T::CK * T::CJ);
+        const int I = I0 + dI, J = J0 + dJ, K = K0 + dK;
+        if (I > gc.nx || J > gc.ny || (DIM == 3 && K > gc.nz)) continue;
+        const unsigned qc = ((unsigned)I * (unsigned)gc.Py + (unsigned)J) * (unsigned)gc.Pz + (unsigned)K;
+        const C s = restrict_from<TS, DIM>(
+            &sr[f][((2 * dI + 1) * T::FJ + (2 * dJ + 1)) * T::FK + (DIM == 3 ? 2 * dK + 1 : 0)], f, T::FJ * T::FK, T::FK,
+            DIM == 3 ? 1 : 0, (at(flc, qc) >> f) & 1);
+        put(bc + f * gc.S, qc, Cvt<TS>::st(s));
+    }
+}
+
+// ------------------------------------------------ fused coarsest levels
+
+namespace {
+
+// One level of the fused cycle in LDS, side N known to the compiler.  Every field is a
+// box of (N + 2)^DIM nodes, indices -1 .. N per axis: the zero entries at -1 stand for
+// everything outside the level (the entry after N along an axis is the -1 of the next
+// row or plane; after the last plane of u_x comes u_y's, after the flags a spare plane).
+template <typename TS, int DIM, int N> struct TLvl {
+    static constexpr int P = N + 2, SK = DIM == 3 ? 1 : 0, SJ = DIM == 3 ? P : 1, SI = SJ * P;
+    static constexpr int NODES = SI * P, NF = DIM + 1;
+    static constexpr int VEC = NF * NODES;
+    static constexpr bool LAST = N == 2;          // coarsest: only b and x are kept
+    TS x[VEC], b[VEC];
+    TS al[LAST ? 1 : DIM * NODES], r[LAST ? 1 : VEC];
+    uint8_t fl[(NODES + SI + 15) / 16 * 16];
+    __device__ static constexpr int id(int i, int j, int k) { return (i + 1) * SI + (j + 1) * SJ + (DIM == 3 ? (k + 1) * SK : 0); }
+};
+
+template <typename TS, int DIM, int N, bool M> struct LdsAcc {
+    typedef typename Cvt<TS>::C C;
+    static constexpr bool MASK = M;
+    typedef TLvl<TS, DIM, N> L;
+    const L &l;
+    int q;
+    __device__ __forceinline__ int o(int di, int dj, int dk) const { return q + di * L::SI + dj * L::SJ + dk * L::SK; }
+    __device__ __forceinline__ int F(int di, int dj, int dk) const { return l.fl[o(di, dj, dk)]; }
+    __device__ __forceinline__ C X(int f, int di, int dj, int dk) const { return Cvt<TS>::ld(l.x[f * L::NODES + o(di, dj, dk)]); }
+    __device__ __forceinline__ C B(int f, int di, int dj, int dk) const { return Cvt<TS>::ld(l.b[f * L::NODES + o(di, dj, dk)]); }
+    __device__ __forceinline__ C AL(int d, int di, int dj, int dk) const { return Cvt<TS>::ld(l.al[d * L::NODES + o(di, dj, dk)]); }
+};
+
+constexpr int TAIL_NT = 512;  // 256 registers a lane: the FP64 block solve fits them
+
+// the node t of the (N + 1)^DIM nodes of a level
+template <int DIM, int N> __device__ __forceinline__ void node_of(int t, int &i, int &j, int &k)
+{
+    if (DIM == 3) {
+        k = t % (N + 1);
+        j = (t / (N + 1)) % (N + 1);
+        i = t / ((N + 1) * (N + 1));
+    } else {
+        k = 0;
+        j = t % (N + 1);
+        i = t / (N + 1);
+    }
+}
+template <int DIM, int N> constexpr int n_nodes() { return (N + 1) * (N + 1) * (DIM == 3 ? N + 1 : 1); }
+
+// one colour pass in place: every lane reads what it needs, then every lane writes (the
+// first pass of the way down reads the zeros the launch starts with)
+template <typename TS, int DIM, int N, bool MASK>
+__device__ __forceinline__ void tail_color(TLvl<TS, DIM, N> &l, int color, float omega)
+{
+    typedef typename Cvt<TS>::C C;
+    typedef TLvl<TS, DIM, N> L;
+    constexpr int NP = (DIM == 3 ? N * N * N : N * N) / 2, H = N / 2;
+    static_assert(NP <= TAIL_NT, "one colour cell per lane");
+    const int t = threadIdx.x;
+    int q = 0;
+    C pn, u0[3], u1[3];
+    if (t < NP) {
+        int i, j, k;
+        const int pr = 2 * (t % H);
+        if (DIM == 3) {
+            j = (t / H) % N;
+            i = t / (H * N);
+            k = pr + ((i + j + color) & 1);
+        } else {
+            i = t / H;
+            j = pr + ((i + color) & 1);
+            k = 0;
+        }
+        q = L::id(i, j, k);
+        const LdsAcc<TS, DIM, N, MASK> a{l, q};
+        box_cell<C, DIM, false>(a, omega, pn, u0, u1);
+    }
+    __syncthreads();
+    if (t < NP) {
+        l.x[q] = Cvt<TS>::st(pn);
+        const int st[3] = {L::SI, L::SJ, L::SK};
+#pragma unroll
+        for (int d = 0; d < DIM; d++) {
+            l.x[(1 + d) * L::NODES + q] = Cvt<TS>::st(u0[d]);
+            l.x[(1 + d) * L::NODES + q + st[d]] = Cvt<TS>::st(u1[d]);
+        }
+    }
+    __syncthreads();
+}
+
+template <typename TS, int DIM, int N, bool MASK>
+__device__ __forceinline__ void tail_smooth(TLvl<TS, DIM, N> &l, int nu, int first, float omega)
+{
+#pragma unroll 1
+    for (int s = 0; s < 2 * nu; s++) tail_color<TS, DIM, N, MASK>(l, first ^ (s & 1), omega);
+}
+
+// r = b - A x on the nodes of the level
+template <typename TS, int DIM, int N, bool MASK>
+__device__ __forceinline__ void tail_residual(TLvl<TS, DIM, N> &l)
+{
+    typedef typename Cvt<TS>::C C;
+    typedef TLvl<TS, DIM, N> L;
+    for (int t = threadIdx.x; t < n_nodes<DIM, N>(); t += TAIL_NT) {
+        int i, j, k;
+        node_of<DIM, N>(t, i, j, k);
+        const LdsAcc<TS, DIM, N, MASK> a{l, L::id(i, j, k)};
+        const BoxSten<C, DIM, LdsAcc<TS, DIM, N, MASK>> s{a};
+        l.r[a.q] = Cvt<TS>::st(a.B(0, 0, 0, 0) - s.cell());
+        l.r[L::NODES + a.q] = Cvt<TS>::st(a.B(1, 0, 0, 0) - s.template face<0>(0, 0, 0));
+        l.r[2 * L::NODES + a.q] = Cvt<TS>::st(a.B(2, 0, 0, 0) - s.template face<1>(0, 0, 0));
+        if (DIM == 3) l.r[3 * L::NODES + a.q] = Cvt<TS>::st(a.B(3, 0, 0, 0) - s.template face<2>(0, 0, 0));
+    }
+    __syncthreads();
+}
+
+// c.b = R l.r: one (field, coarse node) per lane
+template <typename TS, int DIM, int N>
+__device__ __forceinline__ void tail_restrict(const TLvl<TS, DIM, N> &l, TLvl<TS, DIM, N / 2> &c)
+{
+    typedef typename Cvt<TS>::C C;
+    typedef TLvl<TS, DIM, N> L;
+    typedef TLvl<TS, DIM, N / 2> K_;
+    constexpr int NN = n_nodes<DIM, N / 2>();
+    for (int t = threadIdx.x; t < NN * (DIM + 1); t += TAIL_NT) {
+        const int f = t / NN;
+        int I, J, K;
+        node_of<DIM, N / 2>(t % NN, I, J, K);
+        const int qc = K_::id(I, J, K), q = L::id(2 * I, 2 * J, 2 * K);
+        const C s = restrict_from<TS, DIM>(l.r + f * L::NODES + q, f, L::SI, L::SJ, L::SK, (c.fl[qc] >> f) & 1);
+        c.b[f * K_::NODES + qc] = Cvt<TS>::st(s);
+    }
+    __syncthreads();
+}
+
+// l.x += P c.x on the free DOFs
+template <typename TS, int DIM, int N>
+__device__ __forceinline__ void tail_prolong(TLvl<TS, DIM, N> &l, const TLvl<TS, DIM, N / 2> &c)
+{
+    typedef typename Cvt<TS>::C C;
+    typedef TLvl<TS, DIM, N> L;
+    typedef TLvl<TS, DIM, N / 2> K_;
+    for (int t = threadIdx.x; t < n_nodes<DIM, N>(); t += TAIL_NT) {
+        int co[3];
+        node_of<DIM, N>(t, co[0], co[1], co[2]);
+        const int q = L::id(co[0], co[1], co[2]), qc = K_::id(co[0] >> 1, co[1] >> 1, co[2] >> 1);
+        const int fb = l.fl[q], st[3] = {K_::SI, K_::SJ, K_::SK};
+        if (fb & 1) l.x[q] = Cvt<TS>::st(Cvt<TS>::ld(l.x[q]) + C(0.5) * Cvt<TS>::ld(c.x[qc]));
+#pragma unroll
+        for (int d = 0; d < DIM; d++) {
+            if (!((fb >> (1 + d)) & 1)) continue;
+            const TS *e0 = c.x + (1 + d) * K_::NODES + qc;
+            C e = Cvt<TS>::ld(e0[0]);
+            if (co[d] & 1) {
+                e += Cvt<TS>::ld(e0[st[d]]);
+                e *= C(0.5);
+            }
+            TS &v = l.x[(1 + d) * L::NODES + q];
+            v = Cvt<TS>::st(Cvt<TS>::ld(v) + e);
+        }
+    }
+    __syncthreads();
+}
+
+// level data from the node layout of device memory (levels below 64 a side: pitch N + 1)
+template <typename TS, int DIM, int N>
+__device__ __forceinline__ void tail_load(TLvl<TS, DIM, N> &l, const uint8_t *fl, const TS *al, const TS *b)
+{
+    typedef TLvl<TS, DIM, N> L;
+    constexpr int NN = n_nodes<DIM, N>();
+    for (int t = threadIdx.x; t < NN; t += TAIL_NT) {
+        int i, j, k;
+        node_of<DIM, N>(t, i, j, k);
+        const int q = L::id(i, j, k);
+        l.fl[q] = fl[t];
+        if constexpr (!L::LAST)
+            for (int d = 0; d < DIM; d++) l.al[d * L::NODES + q] = al[d * NN + t];
+        if (b)
+            for (int f = 0; f <= DIM; f++) l.b[f * L::NODES + q] = b[f * NN + t];
+    }
+}
+
+template <typename TS, int DIM, int N> struct TailPool {
+    TLvl<TS, DIM, N> l;
+    TailPool<TS, DIM, N / 2> next;
+};
+template <typename TS, int DIM> struct TailPool<TS, DIM, 2> {
+    TLvl<TS, DIM, 2> l;
+};
+
+template <typename TS, int DIM, int N, int LEV>
+__device__ __forceinline__ void tail_load_all(TailPool<TS, DIM, N> &p, const TailArgs<TS> &a, const TS *b)
+{
+    tail_load<TS, DIM, N>(p.l, a.fl[LEV], a.al[LEV], b);
+    if constexpr (N > 2) tail_load_all<TS, DIM, N / 2, LEV + 1>(p.next, a, nullptr);
+}
+
+// DOFs of the coarsest level (2 cells a side) in the compact list's order
+template <int DIM> struct TailDofs {
+    static constexpr int PL = DIM == 3 ? 2 : 1;             // nodes along k
+    static constexpr int NCELL = 4 * PL, NFACE = 6 * PL;    // per direction (i and j: 3 x 2 x PL; k: 2 x 2 x 3)
+    static constexpr int ND = NCELL + DIM * NFACE;
+    static constexpr int LPR = 8, NCOL = (ND + LPR - 1) / LPR;  // lanes per row, columns per lane
+};
+// position of the compact DOF c in the coarsest level's LDS box
+template <typename TS, int DIM> __device__ __forceinline__ int tail_dof(int c)
+{
+    typedef TLvl<TS, DIM, 2> L;
+    typedef TailDofs<DIM> D;
+    const int f = c < D::NCELL ? 0 : 1 + (c - D::NCELL) / D::NFACE;
+    const int m = c < D::NCELL ? c : (c - D::NCELL) % D::NFACE;
+    const int nk = DIM == 3 ? 2 + (f == 3) : 1, nj = 2 + (f == 2);
+    return f * L::NODES + L::id(m / (nk * nj), (m / nk) % nj, m % nk);
+}
+
+// rows of the coarsest inverse held by a lane: LPR lanes per row, columns lane, lane + LPR, ..
+template <typename TS, int DIM>
+__device__ __forceinline__ void tail_coarse(TLvl<TS, DIM, 2> &l, const double *mrow, const int *mcol, int row, int nd)
+{
+    typedef typename Cvt<TS>::C C;
+    typedef TailDofs<DIM> D;
+    double s = 0.0;
+#pragma unroll
+    for (int c = 0; c < D::NCOL; c++) s += mrow[c] * (double)Cvt<TS>::ld(l.b[mcol[c]]);
+#pragma unroll
+    for (int o = D::LPR / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, D::LPR);
+    if (row < nd && (threadIdx.x & (D::LPR - 1)) == 0) l.x[tail_dof<TS, DIM>(row)] = Cvt<TS>::st((C)s);
+    __syncthreads();
+}
+
+template <typename TS, int DIM, int N, bool MASK>
+__device__ __forceinline__ void tail_cycle(TailPool<TS, DIM, N> &p, int nu_pre, int nu_post, float om,
+                                           const double *mrow, const int *mcol, int row, int nd)
+{
+    if constexpr (N == 2) {
+        tail_coarse<TS, DIM>(p.l, mrow, mcol, row, nd);
+    } else {
+        // way down, then way up: one loop, so that the passes of a level are compiled once
+        // (the launch runs on one CU, and fetching its instructions is a good part of it)
+#pragma unroll 1
+        for (int up = 0; up < 2; up++) {
+            if (up) tail_prolong<TS, DIM, N>(p.l, p.next.l);
+            tail_smooth<TS, DIM, N, MASK>(p.l, up ? nu_post : nu_pre, up, om);
+            if (!up) {
+                tail_residual<TS, DIM, N, MASK>(p.l);
+                tail_restrict<TS, DIM, N>(p.l, p.next.l);
+                tail_cycle<TS, DIM, N / 2, false>(p.next, nu_pre, nu_post, om, mrow, mcol, row, nd);
+            }
+        }
+    }
+}
+
+}  // namespace
+
+// The V-cycle from a level of N cells a side (8 in 3D; 32, or the grid itself, in 2D)
+// down to the coarsest one and back in one workgroup, every buffer in LDS.  x is
+// updated in place (a pass holds its results in registers over a barrier), so a level
+// needs x, b, alpha and r only and a 32^2 level fits in FP64; sides, pitches and loop
+// counts are compile-time constants, and the coarsest inverse is read into registers
+// while the levels are staged.  Per cycle, first level 8^3: 28 us FP64, 25 us FP32
+// (81 us both with 64-bit index arithmetic, run-time sides and the rows of a cell
+// evaluated one by one); from 32^2: 38 / 30 us (65 us from 16^2, and ten launches of
+// 3-7 us for the 32^2 level).  One workgroup is a chain of ~20 passes of ~1 us each.
+template <typename TS, int DIM, int N, bool MASK>
+__global__ void __launch_bounds__(TAIL_NT) k_tail(TailArgs<TS> a, const TS *__restrict__ b0, TS *__restrict__ x0)
+{
+    typedef TailPool<TS, DIM, N> Pool;
+    typedef TailDofs<DIM> D;
+    static_assert(sizeof(Pool) <= 160 * 1024, "the levels of the fused cycle fit in LDS");
+    static_assert(D::ND * D::LPR <= TAIL_NT, "a row of the coarsest inverse per group of lanes");
+    __shared__ __align__(16) unsigned char mem[sizeof(Pool) / 16 * 16 + 16];
+    Pool &p = *reinterpret_cast<Pool *>(mem);
+    const int nd = a.nd;
+    double mrow[D::NCOL];
+    int mcol[D::NCOL];
+    const int row = threadIdx.x / D::LPR;
+#pragma unroll
+    for (int c = 0; c < D::NCOL; c++) {
+        const int col = (int)(threadIdx.x & (D::LPR - 1)) + c * D::LPR;
+        const bool on = row < nd && col < nd;
+        mrow[c] = on ? a.minv[(long)row * nd + col] : 0.0;
+        mcol[c] = on ? tail_dof<TS, DIM>(col) : 0;
+    }
+    for (int q = threadIdx.x; q < (int)(sizeof(mem) / 16); q += TAIL_NT)
+        reinterpret_cast<uint4 *>(mem)[q] = make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
+    tail_load_all<TS, DIM, N, 0>(p, a, b0);
+    __syncthreads();
+    tail_cycle<TS, DIM, N, MASK>(p, a.nu_pre, a.nu_post, a.omega, mrow, mcol, row, nd);
+    constexpr int NN = n_nodes<DIM, N>();
+    for (int t = threadIdx.x; t < NN; t += TAIL_NT) {
+        int i, j, k;
+        node_of<DIM, N>(t, i, j, k);
+        const int q = TLvl<TS, DIM, N>::id(i, j, k);
+        for (int f = 0; f <= DIM; f++) x0[f * NN + t] = p.l.x[f * TLvl<TS, DIM, N>::NODES + q];
+    }
+}
+
+// ============================================================== launchers
+
+static int lg2(int n) { return __builtin_ctz((unsigned)n); }
+
+template <typename TS>
+void launch_box(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b, const TS *xin, TS *xout, int color,
+                float omega, bool zero, bool inner, hipStream_t s)
+{
+    const int lg = lg2(g.nx);
+    const unsigned np = 1u << (g.dim * lg - 1);
+    // one wave per workgroup on the smallest levels, so that every wave has a CU
+    const unsigned bs = np <= (1u << 16) ? 64 : 256;
+    const dim3 gr((np + bs - 1) / bs), bl(bs);
+#define ST_BOX(D, Z, M) hipLaunchKernelGGL((k_box<TS, D, Z, M>), gr, bl, 0, s, g, lg, fl, al, b, xin, xout, color, omega)
+    if (g.dim == 3) {
+        if (zero) ST_BOX(3, true, false);  // reads no x
+        else if (inner) ST_BOX(3, false, false);
+        else ST_BOX(3, false, true);
+    } else {
+        if (zero) ST_BOX(2, true, false);
+        else if (inner) ST_BOX(2, false, false);
+        else ST_BOX(2, false, true);
+    }
+#undef ST_BOX
+}
+
+template <typename TS>
+void launch_resid_restrict(const Lvl &gf, const Lvl &gc, const uint8_t *flf, const TS *al, const TS *b, const TS *x,
+                           const uint8_t *flc, TS *bc, bool inner, hipStream_t s)
+{
+    auto up = [](int n, int c) { return (unsigned)((n + c) / c); };  // n + 1 coarse nodes in tiles of c
+    const dim3 g3(up(gc.nz, RrTile<3>::CK), up(gc.ny, RrTile<3>::CJ), up(gc.nx, RrTile<3>::CI));
+    const dim3 g2(1, up(gc.ny, RrTile<2>::CJ), up(gc.nx, RrTile<2>::CI));
+#define ST_RR(D, M, GR) \
+    hipLaunchKernelGGL((k_resid_restrict<TS, D, M>), GR, dim3(RrTile<D>::NT), 0, s, gf, gc, flf, al, b, x, flc, bc)
+    if (gf.dim == 3) {
+        if (inner) ST_RR(3, false, g3);
+        else ST_RR(3, true, g3);
+    } else {
+        if (inner) ST_RR(2, false, g2);
+        else ST_RR(2, true, g2);
+    }
+#undef ST_RR
+}
+
+template <typename TS>
+void launch_node_apply(const Lvl &g, const uint8_t *fl, const TS *al, const TS *x, TS *y, hipStream_t s)
+{
+    const dim3 gr((unsigned)((g.S + 255) / 256)), bl(256);
+    if (g.dim == 3) hipLaunchKernelGGL((k_apply<TS, 3>), gr, bl, 0, s, g, fl, al, x, y);
+    else hipLaunchKernelGGL((k_apply<TS, 2>), gr, bl, 0, s, g, fl, al, x, y);
+}
+template <typename TS>
+void launch_node_residual(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b, const TS *x, TS *r, double *part,
+                          hipStream_t s)
+{
+    const dim3 gr((unsigned)((g.S + 255) / 256)), bl(256);
+    if (g.dim == 3) hipLaunchKernelGGL((k_residual<TS, 3>), gr, bl, 0, s, g, fl, al, b, x, r, part);
+    else hipLaunchKernelGGL((k_residual<TS, 2>), gr, bl, 0, s, g, fl, al, b, x, r, part);
+}
+
+template <typename TS>
+void launch_prolong(const Lvl &gf, const Lvl &gc, const uint8_t *flf, const TS *ec, TS *xf, hipStream_t s)
+{
+    const long rows = gf.dim == 3 ? (long)gf.Px * gf.Py : gf.Px, m = (gf.dim == 3 ? gc.nz : gc.ny) + 1;
+    const dim3 gr((unsigned)((rows * m + 255) / 256)), bl(256);
+    if (gf.dim == 2) hipLaunchKernelGGL((k_prolong<TS, 2, false>), gr, bl, 0, s, gf, gc, flf, ec, xf);
+    else if (gf.Pz % 2 == 0) hipLaunchKernelGGL((k_prolong<TS, 3, true>), gr, bl, 0, s, gf, gc, flf, ec, xf);
+    else hipLaunchKernelGGL((k_prolong<TS, 3, false>), gr, bl, 0, s, gf, gc, flf, ec, xf);
+}
+
+template <typename TS>
+void launch_vcycle_tail(const TailArgs<TS> &a, int dim, int n, const TS *b0, TS *x0, bool inner, hipStream_t s)
+{
+#define ST_TAIL(D, N, M) hipLaunchKernelGGL((k_tail<TS, D, N, M>), dim3(1), dim3(TAIL_NT), 0, s, a, b0, x0)
+    if (dim == 3) {
+        if (inner) ST_TAIL(3, 8, false);
+        else ST_TAIL(3, 8, true);
+    } else if (n == 32) {
+        if (inner) ST_TAIL(2, 32, false);
+        else ST_TAIL(2, 32, true);
+    } else if (n == 16) {  // these sides start the cycle only as the grid itself
+        ST_TAIL(2, 16, true);
+    } else {
+        ST_TAIL(2, 8, true);
+    }
+#undef ST_TAIL
+}
+
+#define INST_C(T)                                                                                                  \
+    template void launch_box<T>(const Lvl &, const uint8_t *, const T *, const T *, const T *, T *, int, float, bool, \
+                                bool, hipStream_t);                                                                     \
+    template void launch_resid_restrict<T>(const Lvl &, const Lvl &, const uint8_t *, const T *, const T *,       \
+                                           const T *, const uint8_t *, T *, bool, hipStream_t);                   \
+    template void launch_node_apply<T>(const Lvl &, const uint8_t *, const T *, const T *, T *, hipStream_t);      \
+    template void launch_node_residual<T>(const Lvl &, const uint8_t *, const T *, const T *, const T *, T *,     \
+                                          double *, hipStream_t);                                                 \
+    template void launch_prolong<T>(const Lvl &, const Lvl &, const uint8_t *, const T *, T *, hipStream_t);      \
+    template void launch_vcycle_tail<T>(const TailArgs<T> &, int, int, const T *, T *, bool, hipStream_t);
+INST_C(double)
+INST_C(float)
+INST_C(bf16)
+
+}  // namespace st

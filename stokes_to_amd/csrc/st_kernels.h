@@ -10,32 +10,37 @@ struct AlphaParams {
     double amax, amin, q, power, scale;
 };
 
-// the V-cycle below and including level l0 in one launch (levels small enough for
-// one workgroup): pre-smoothing, residual and restriction down to the coarsest
-// level, its dense solve, then prolongation and post-smoothing back to l0
 constexpr int ST_MAX_LEVELS = 12;
-constexpr long ST_TAIL_MAX_CELLS = 512;  // 8^3: one cell per thread of the workgroup
-// (kept in device memory: the kernel indexes it by level; b and x of level 0 are
-// the caller's vectors when l0 = 0, the level buffers b[l], x[l] otherwise)
-constexpr int ST_TAIL_LDS_BYTES = 150 * 1024;  // LDS pool of the LDS-resident variant
-struct TailLds {  // byte offsets of the level buffers in the LDS pool
-    int fl[ST_MAX_LEVELS], al[ST_MAX_LEVELS], b[ST_MAX_LEVELS], x[ST_MAX_LEVELS], t[ST_MAX_LEVELS],
-        r[ST_MAX_LEVELS];
-    int bs, bytes, ok;
-};
+// the coarsest levels of a V-cycle in one launch (st_coarse.hip): flags and alpha of the
+// first of them and the ones below, by value, so that their loads wait for no pointer
+constexpr int ST_TAIL_LEVELS = 5;
 template <typename TS> struct TailArgs {
-    int l0, L, nu_pre, nu_post, nd, dim;
+    int nu_pre, nu_post, nd;
     float omega;
-    TailLds lds;
-    Lvl g[ST_MAX_LEVELS];
-    const uint8_t *fl[ST_MAX_LEVELS];
-    const TS *al[ST_MAX_LEVELS];
-    TS *b[ST_MAX_LEVELS], *x[ST_MAX_LEVELS], *t[ST_MAX_LEVELS], *r[ST_MAX_LEVELS];
-    const long *dofs;
+    const uint8_t *fl[ST_TAIL_LEVELS];
+    const TS *al[ST_TAIL_LEVELS];
     const double *minv;
 };
+// inner (here and below): the level lies under the finest one, so every fixed DOF has a
+// zero right-hand side and a zero x (st_box.h)
+// n: side of the first level, 8 in 3D and 8, 16 or 32 in 2D; b0, x0: its right-hand side
+// and solution
 template <typename TS>
-void launch_vcycle_tail(const TailArgs<TS> *dev_args, int dim, const TS *b0, TS *x0, int nd, bool lds, hipStream_t);
+void launch_vcycle_tail(const TailArgs<TS> &a, int dim, int n, const TS *b0, TS *x0, bool inner, hipStream_t);
+// smoother colour pass of a level that is not marched, one lane per pair of cells
+template <typename TS>
+void launch_box(const Lvl &, const uint8_t *, const TS *al, const TS *b, const TS *xin, TS *xout, int color,
+                float omega, bool zero, bool inner, hipStream_t);
+// y = A x and r = b - A x (partials of |r|^2 per 256 nodes) of such a level
+template <typename TS>
+void launch_node_apply(const Lvl &, const uint8_t *, const TS *al, const TS *x, TS *y, hipStream_t);
+template <typename TS>
+void launch_node_residual(const Lvl &, const uint8_t *, const TS *al, const TS *b, const TS *x, TS *r, double *part,
+                          hipStream_t);
+// bc = R (b - A x): residual and restriction of such a level in one launch
+template <typename TS>
+void launch_resid_restrict(const Lvl &gf, const Lvl &gc, const uint8_t *flf, const TS *al, const TS *b, const TS *x,
+                           const uint8_t *flc, TS *bc, bool inner, hipStream_t);
 
 template <typename TS> void launch_apply(const Lvl &, const uint8_t *, const TS *, const TS *, TS *, hipStream_t);
 template <typename TS>
@@ -44,7 +49,7 @@ void launch_residual(const Lvl &, const uint8_t *, const TS *, const TS *b, cons
 unsigned residual_blocks(const Lvl &);
 template <typename TS>
 void launch_smooth(const Lvl &, const uint8_t *, const TS *, const TS *b, const TS *xin, TS *xout, int color,
-                   float omega, bool zero, hipStream_t);
+                   float omega, bool zero, bool inner, hipStream_t);
 template <typename TS>
 void launch_restrict(const Lvl &gf, const Lvl &gc, const uint8_t *flc, const TS *rf, TS *bc, hipStream_t);
 template <typename TS>
@@ -55,9 +60,7 @@ void launch_coarsen(const Lvl &gf, const Lvl &gc, const uint8_t *flf, const TF *
 template <typename TS>
 void launch_probe(const Lvl &, const uint8_t *, const TS *, const long *dofs, int nd, int closed, double *A,
                   hipStream_t);
-void launch_gauss_jordan(int n, double *A, int *perm, int *info, hipStream_t);
-template <typename TS>
-void launch_coarse_solve(int nd, const long *dofs, const double *Minv, const TS *b, TS *x, hipStream_t);
+void launch_gauss_jordan(int n, double *A, int *info, hipStream_t);  // n <= 64
 template <typename TS>
 void launch_pack(const Lvl &, const double *abi, TS *pad, int fixed_only, const uint8_t *fl, double scale,
                  hipStream_t);

@@ -184,194 +184,6 @@ __device__ __forceinline__ double block_sum(double v, double *sh)
     return s;
 }
 
-// ------------------------------------------------------------- operator
-
-template <typename TS, int DIM>
-__global__ void __launch_bounds__(256) k_apply(Lvl g, const uint8_t *fl, const TS *al, const TS *x, TS *y)
-{
-    long n = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= g.S) return;
-    int i, j, k;
-    node_ijk(g, n, i, j, k);
-    Sten<TS, DIM> s{g, fl, x, al, -1};
-    y[n] = Cvt<TS>::st(s.Acell(i, j, k));
-    y[g.S + n] = Cvt<TS>::st(s.template Aface<0>(i, j, k));
-    y[2 * g.S + n] = Cvt<TS>::st(s.template Aface<1>(i, j, k));
-    if (DIM == 3) y[3 * g.S + n] = Cvt<TS>::st(s.template Aface<2>(i, j, k));
-}
-
-// r = b - A x at node n; returns the node's contribution to |r|^2
-template <typename TS, int DIM>
-__device__ __forceinline__ double residual_body(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b,
-                                                const TS *x, TS *r, long n)
-{
-    if (n >= g.S) return 0.0;
-    int i, j, k;
-    node_ijk(g, n, i, j, k);
-    Sten<TS, DIM> s{g, fl, x, al, -1};
-    typedef typename Cvt<TS>::C C;
-    C v0 = Cvt<TS>::ld(b[n]) - s.Acell(i, j, k);
-    C v1 = Cvt<TS>::ld(b[g.S + n]) - s.template Aface<0>(i, j, k);
-    C v2 = Cvt<TS>::ld(b[2 * g.S + n]) - s.template Aface<1>(i, j, k);
-    if (r) {  // without r: the norm only
-        r[n] = Cvt<TS>::st(v0);
-        r[g.S + n] = Cvt<TS>::st(v1);
-        r[2 * g.S + n] = Cvt<TS>::st(v2);
-    }
-    double acc = (double)v0 * v0 + (double)v1 * v1 + (double)v2 * v2;
-    if (DIM == 3) {
-        C v3 = Cvt<TS>::ld(b[3 * g.S + n]) - s.template Aface<2>(i, j, k);
-        if (r) r[3 * g.S + n] = Cvt<TS>::st(v3);
-        acc += (double)v3 * v3;
-    }
-    return acc;
-}
-
-// r = b - A x, optional partial sums of r^2 (FP64) per block
-template <typename TS, int DIM>
-__global__ void __launch_bounds__(256) k_residual(Lvl g, const uint8_t *fl, const TS *al, const TS *b,
-                                                  const TS *x, TS *r, double *part)
-{
-    __shared__ double sh[16];
-    const double acc = residual_body<TS, DIM>(g, fl, al, b, x, r, (long)blockIdx.x * blockDim.x + threadIdx.x);
-    if (part) {
-        double t = block_sum(acc, sh);
-        if (threadIdx.x == 0) part[blockIdx.x] = t;
-    }
-}
-
-// --------------------------------------------------------------- smoother
-
-// One colour of the red-black box-Vanka smoother (the reference smooths the same
-// cell blocks [6 faces + cell] with batched LU, ST/StokeLike.cu:41-372,
-// CX/DescentSmoother.cu:31-53).  For a cell c of the colour the local block of A is
-//   [K  b_f ; m_c b_f^T  1 - m_c],  K = E - (1 - m_c) b_f b_f^T,
-//   E = blockdiag_d [[a_lo + (1-m_c) m_lo, -m_lo m_hi], [-m_lo m_hi, a_hi + (1-m_c) m_hi]],
-//   b_f = (-m_lo, m_hi) per axis.
-// In a free cell the cross-axis couplings of curl-curl and grad-div cancel (vol = free
-// mask) and K = E; the block is solved through the scalar Schur complement.  In a
-// fixed cell the curl-curl couplings remain as the rank-one term, p is decoupled
-// (dp = r_p) and the velocity solve is Sherman-Morrison on E.  Both are the exact
-// block inverse (equal to LU of the probed block).  xin -> xout (ping-pong); DOFs not
-// owned by a cell of the colour are copied.  ZERO: xin is identically zero.
-template <typename TS, int DIM, bool ZERO>
-__device__ __forceinline__ void smooth_cell(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b,
-                                            const TS *xin, TS *xout, int color, float omega, int i, int j, int k)
-{
-    typedef typename Cvt<TS>::C C;
-    Sten<TS, DIM> s{g, fl, xin, al, -1};
-    const long q = s.id(i, j, k);
-    const long S = g.S;
-    const long st[3] = {(long)g.Py * g.Pz, (long)g.Pz, 1};
-    if (((i + j + k) & 1) != color) {
-        xout[q] = ZERO ? Cvt<TS>::st(C(0)) : xin[q];
-        if (i == 0) xout[S + q] = ZERO ? Cvt<TS>::st(C(0)) : xin[S + q];
-        if (i == g.nx - 1) xout[S + q + st[0]] = ZERO ? Cvt<TS>::st(C(0)) : xin[S + q + st[0]];
-        if (j == 0) xout[2 * S + q] = ZERO ? Cvt<TS>::st(C(0)) : xin[2 * S + q];
-        if (j == g.ny - 1) xout[2 * S + q + st[1]] = ZERO ? Cvt<TS>::st(C(0)) : xin[2 * S + q + st[1]];
-        if (DIM == 3) {
-            if (k == 0) xout[3 * S + q] = ZERO ? Cvt<TS>::st(C(0)) : xin[3 * S + q];
-            if (k == g.nz - 1) xout[3 * S + q + st[2]] = ZERO ? Cvt<TS>::st(C(0)) : xin[3 * S + q + st[2]];
-        }
-        return;
-    }
-    const int fb = fl[q];
-    const C mc = (fb & 1) ? C(1) : C(0);
-    const C NE = (DIM == 3) ? C(4) : C(2);
-    C rp = Cvt<TS>::ld(b[q]);
-    if (!ZERO) rp -= s.Acell(i, j, k);
-    C beta = C(0), tb = C(0);  // b^T E^-1 b, b^T E^-1 r_u
-    C a0[3], a1[3], of[3], r0[3], r1[3], m0[3], m1[3];
-#pragma unroll
-    for (int d = 0; d < DIM; d++) {
-        const int di = (d == 0), dj = (d == 1), dk = (d == 2);
-        const long qh = q + st[d];
-        const int fl_lo = fb, fl_hi = fl[qh];
-        m0[d] = ((fl_lo >> (1 + d)) & 1) ? C(1) : C(0);
-        m1[d] = ((fl_hi >> (1 + d)) & 1) ? C(1) : C(0);
-        // free cells adjacent to the two faces: (c - e_d, c) and (c, c + e_d)
-        C c_lo = (C)(s.F(i - di, j - dj, k - dk) & 1);
-        C c_hi = (C)(s.F(i + di, j + dj, k + dk) & 1);
-        C al0 = Cvt<TS>::ld(al[(long)d * S + q]);
-        C al1 = Cvt<TS>::ld(al[(long)d * S + qh]);
-        a0[d] = m0[d] * (c_lo + mc + NE) + al0 + (C(1) - m0[d]) + (C(1) - mc) * m0[d];
-        a1[d] = m1[d] * (mc + c_hi + NE) + al1 + (C(1) - m1[d]) + (C(1) - mc) * m1[d];
-        of[d] = -m0[d] * m1[d];
-        C rl = Cvt<TS>::ld(b[(long)(1 + d) * S + q]);
-        C rh = Cvt<TS>::ld(b[(long)(1 + d) * S + qh]);
-        if (!ZERO) {
-            if (d == 0) { rl -= s.template Aface<0>(i, j, k); rh -= s.template Aface<0>(i + 1, j, k); }
-            if (d == 1) { rl -= s.template Aface<1>(i, j, k); rh -= s.template Aface<1>(i, j + 1, k); }
-            if (d == 2) { rl -= s.template Aface<2>(i, j, k); rh -= s.template Aface<2>(i, j, k + 1); }
-        }
-        r0[d] = rl;
-        r1[d] = rh;
-        const C id = C(1) / (a0[d] * a1[d] - of[d] * of[d]);
-        // b_f = (-m0, m1), b_c = mc * b_f
-        const C kb0 = id * (a1[d] * (-m0[d]) - of[d] * m1[d]);
-        const C kb1 = id * (-of[d] * (-m0[d]) + a0[d] * m1[d]);
-        const C kr0 = id * (a1[d] * rl - of[d] * rh);
-        const C kr1 = id * (-of[d] * rl + a0[d] * rh);
-        beta += (-m0[d]) * kb0 + m1[d] * kb1;
-        tb += (-m0[d]) * kr0 + m1[d] * kr1;
-    }
-    const C Sc = (mc != C(0)) ? -beta : C(1);
-    const C dp = (Sc != C(0)) ? (rp - mc * tb) / Sc : C(0);
-    const C gm = (mc != C(0)) ? dp : (dp - tb) / (C(1) - beta);
-    const C om = (C)omega;
-    const C p0 = ZERO ? C(0) : Cvt<TS>::ld(xin[q]);
-    xout[q] = Cvt<TS>::st(p0 + om * dp);
-#pragma unroll
-    for (int d = 0; d < DIM; d++) {
-        const long qh = q + st[d];
-        const C id = C(1) / (a0[d] * a1[d] - of[d] * of[d]);
-        const C e0 = r0[d] + m0[d] * gm;   // r - b_f g, b_f = (-m0, m1)
-        const C e1 = r1[d] - m1[d] * gm;
-        const C u0 = ZERO ? C(0) : Cvt<TS>::ld(xin[(long)(1 + d) * S + q]);
-        const C u1 = ZERO ? C(0) : Cvt<TS>::ld(xin[(long)(1 + d) * S + qh]);
-        xout[(long)(1 + d) * S + q] = Cvt<TS>::st(u0 + om * id * (a1[d] * e0 - of[d] * e1));
-        xout[(long)(1 + d) * S + qh] = Cvt<TS>::st(u1 + om * id * (-of[d] * e0 + a0[d] * e1));
-    }
-}
-
-// one thread per cell t (k fastest)
-template <typename TS, int DIM, bool ZERO>
-__device__ __forceinline__ void smooth_body(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b,
-                                            const TS *xin, TS *xout, int color, float omega, long t)
-{
-    const long ncell = (long)g.nx * g.ny * g.nz;
-    if (t >= ncell) return;
-    const int k = (int)(t % g.nz);
-    const long tt = t / g.nz;
-    smooth_cell<TS, DIM, ZERO>(g, fl, al, b, xin, xout, color, omega, (int)(tt / g.ny), (int)(tt % g.ny), k);
-}
-
-// The pass from x = 0 in 3D with one thread per pair of cells (k, k+1), k even: the
-// pair holds one cell of each colour, so every lane runs the block solve of its
-// colour cell (one thread per cell leaves half the lanes idle through it)
-template <typename TS>
-__global__ void __launch_bounds__(256) k_smooth0_pairs(Lvl g, const uint8_t *fl, const TS *al, const TS *b,
-                                                       TS *xout, int color, float omega)
-{
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int hz = g.nz / 2;
-    if (t >= (long)g.nx * g.ny * hz) return;
-    const int kp = (int)(t % hz);
-    const long tt = t / hz;
-    const int j = (int)(tt % g.ny), i = (int)(tt / g.ny);
-    const int k0 = 2 * kp;
-    const int km = (((i + j + k0) & 1) == color) ? k0 : k0 + 1;
-    smooth_cell<TS, 3, true>(g, fl, al, b, (const TS *)nullptr, xout, color, omega, i, j, km);
-    smooth_cell<TS, 3, true>(g, fl, al, b, (const TS *)nullptr, xout, color, omega, i, j, 2 * k0 + 1 - km);
-}
-
-template <typename TS, int DIM, bool ZERO>
-__global__ void __launch_bounds__(256) k_smooth(Lvl g, const uint8_t *fl, const TS *al, const TS *b,
-                                                const TS *xin, TS *xout, int color, float omega)
-{
-    smooth_body<TS, DIM, ZERO>(g, fl, al, b, xin, xout, color, omega, (long)blockIdx.x * blockDim.x + threadIdx.x);
-}
-
 // ------------------------------------------------------------- transfers
 
 // coarse rhs from the fine residual: R = (4/2^dim) P^T on velocity, (2/2^dim)
@@ -425,43 +237,6 @@ template <typename TS, int DIM>
 __global__ void __launch_bounds__(256) k_restrict(Lvl gf, Lvl gc, const uint8_t *flc, const TS *rf, TS *bc)
 {
     restrict_body<TS, DIM>(gf, gc, flc, rf, bc, (long)blockIdx.x * blockDim.x + threadIdx.x);
-}
-
-// xf += P ec on free fine DOFs (pressure correction scaled by 1/2: unit spacing)
-template <typename TS, int DIM>
-__device__ __forceinline__ void prolong_body(const Lvl &gf, const Lvl &gc, const uint8_t *flf, const TS *ec, TS *xf,
-                                             long n)
-{
-    typedef typename Cvt<TS>::C C;
-    if (n >= gf.S) return;
-    int i, j, k;
-    node_ijk(gf, n, i, j, k);
-    const int fb = flf[n];
-    if (!fb) return;
-    Sten<TS, DIM> c{gc, nullptr, ec, nullptr, -1};
-    const int kz = (DIM == 3) ? 2 : 1;
-    if (fb & 1) xf[n] = Cvt<TS>::st(Cvt<TS>::ld(xf[n]) + C(0.5) * c.X(0, i >> 1, j >> 1, k / kz));
-    int co[3] = {i, j, k};
-#pragma unroll
-    for (int d = 0; d < DIM; d++) {
-        if (!((fb >> (1 + d)) & 1)) continue;
-        int I = i >> 1, J = j >> 1, K = k / kz;
-        C e;
-        if ((co[d] & 1) == 0) {
-            e = c.X(1 + d, I, J, K);
-        } else {
-            e = c.X(1 + d, I, J, K) + c.X(1 + d, I + (d == 0), J + (d == 1), K + (d == 2));
-            e *= C(0.5);
-        }
-        long o = (long)(1 + d) * gf.S + n;
-        xf[o] = Cvt<TS>::st(Cvt<TS>::ld(xf[o]) + e);
-    }
-}
-
-template <typename TS, int DIM>
-__global__ void __launch_bounds__(256) k_prolong(Lvl gf, Lvl gc, const uint8_t *flf, const TS *ec, TS *xf)
-{
-    prolong_body<TS, DIM>(gf, gc, flf, ec, xf, (long)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // coarse flags (free if any coincident child is free) and coarse face alpha
@@ -546,263 +321,111 @@ __global__ void k_probe(Lvl g, const uint8_t *fl, const TS *al, const long *dofs
     }
 }
 
-// in-place Gauss-Jordan inverse with partial pivoting, one workgroup.  info: 0 ok,
-// k > 0 zero pivot at step k (singular), -1 a non-finite entry (nothing is inverted)
-__global__ void __launch_bounds__(1024) k_gauss_jordan(int n, double *A, int *perm, int *info)
+// in-place Gauss-Jordan inverse with partial pivoting of the coarsest matrix (n <= 64),
+// one workgroup, the matrix in LDS.  A step is one read and one write of the matrix:
+// every wave finds the pivot itself by shuffles, and every lane forms the new values of
+// its entries (row swap, scaling and elimination in one) before any is written.  The
+// 44 steps of 3D take 46 us, the 16 of 2D 15 us (194 and 58 us with the matrix in
+// memory, a tree of barriers per pivot and four passes per step).  info: 0 ok, k > 0 zero pivot at step k (singular), -1 a non-finite
+// entry (nothing is inverted)
+constexpr int GJ_MAX = 64, GJ_NT = 1024;
+// maximum over the wave, in every lane, by DPP row shifts and broadcasts
+__device__ __forceinline__ unsigned wave_max_u32(unsigned v)
 {
-    __shared__ double sv[1024];
-    __shared__ int si[1024];
-    __shared__ int piv_s, bad;
-    const int tid = threadIdx.x, nt = blockDim.x;
+    auto mx = [](unsigned a, unsigned b) { return a > b ? a : b; };
+    v = mx(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));  // row_shr 1
+    v = mx(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));  // row_shr 2
+    v = mx(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));  // row_shr 4
+    v = mx(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));  // row_shr 8
+    v = mx(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xf, 0xf, false));  // row_bcast 15
+    v = mx(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xf, 0xf, false));  // row_bcast 31
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+__global__ void __launch_bounds__(GJ_NT) k_gauss_jordan(int n, double *A, int *info)
+{
+    __shared__ double M[GJ_MAX][GJ_MAX + 1];
+    __shared__ int perm[GJ_MAX], bad, zero_at;
+    constexpr int PER = GJ_MAX * GJ_MAX / GJ_NT;  // entries per lane
+    const int tid = threadIdx.x, lane = tid & 63, c = lane, r0 = tid >> 6;
     if (tid == 0) {
-        *info = 0;
         bad = 0;
+        zero_at = 0;
     }
     __syncthreads();
-    for (long q = tid; q < (long)n * n; q += nt)
-        if (!isfinite(A[q])) bad = 1;
+    // lane: column c of the rows r0, r0 + 16, ..
+    for (int e = 0; e < PER; e++) {
+        const int r = r0 + e * (GJ_NT / 64);
+        if (r < n && c < n) {
+            const double v = A[(long)r * n + c];
+            if (!isfinite(v)) bad = 1;
+            M[r][c] = v;
+        }
+    }
     __syncthreads();
     if (bad) {  // the same value for every thread: the whole workgroup returns here
         if (tid == 0) *info = -1;
         return;
     }
     for (int k = 0; k < n; k++) {
-        double best = -1.0;
-        int bi = k;
-        for (int r = k + tid; r < n; r += nt) {
-            double a = fabs(A[(long)r * n + k]);
-            if (a > best) { best = a; bi = r; }
-        }
-        sv[tid] = best;
-        si[tid] = bi;
-        __syncthreads();
-        for (int o = nt >> 1; o > 0; o >>= 1) {
-            if (tid < o && (sv[tid + o] > sv[tid] || (sv[tid + o] == sv[tid] && si[tid + o] < si[tid]))) {
-                sv[tid] = sv[tid + o];
-                si[tid] = si[tid + o];
+        // pivot row: largest |M[r][k]|, r >= k, to 17 bits (any row that near the largest
+        // serves), the first of equals; magnitudes that vanish in FP32 are compared in full
+        const double mag = (lane >= k && lane < n) ? fabs(M[lane][k]) : -1.0;
+        const unsigned fbits = mag > 0.0 ? __float_as_uint((float)mag) : 0u;
+        const unsigned key = wave_max_u32((fbits & ~63u) | (63u - (unsigned)lane));
+        int p = 63 - (int)(key & 63u);
+        if ((key & ~63u) == 0u) {
+            double best = mag;
+            p = lane;
+            for (int o = 32; o > 0; o >>= 1) {
+                const double ov = __shfl_xor(best, o, 64);
+                const int oi = __shfl_xor(p, o, 64);
+                if (ov > best || (ov == best && oi < p)) {
+                    best = ov;
+                    p = oi;
+                }
             }
-            __syncthreads();
+            if (!(best >= 0.0)) p = k;
+        }
+        const double pv = M[p][k];
+        const double pinv = (pv != 0.0) ? 1.0 / pv : 0.0;
+        double nv[PER];
+        if (c < n) {
+            const double pc = M[p][c] * pinv;  // new row k
+#pragma unroll
+            for (int e = 0; e < PER; e++) {
+                const int r = r0 + e * (GJ_NT / 64);
+                if (r >= n) continue;
+                const int src = (r == p) ? k : r;  // rows k and p are swapped
+                const double f = M[src][k];
+                if (r == k) nv[e] = (c == k) ? pinv : pc;
+                else nv[e] = (c == k) ? -f * pinv : M[src][c] - f * pc;
+            }
+        }
+        __syncthreads();
+        if (c < n) {
+#pragma unroll
+            for (int e = 0; e < PER; e++) {
+                const int r = r0 + e * (GJ_NT / 64);
+                if (r < n) M[r][c] = nv[e];
+            }
         }
         if (tid == 0) {
-            piv_s = si[0];
-            perm[k] = si[0];
-            if (sv[0] == 0.0) *info = k + 1;
-        }
-        __syncthreads();
-        const int p = piv_s;
-        if (p != k)
-            for (int c = tid; c < n; c += nt) {
-                double t = A[(long)k * n + c];
-                A[(long)k * n + c] = A[(long)p * n + c];
-                A[(long)p * n + c] = t;
-            }
-        __syncthreads();
-        const double pv = A[(long)k * n + k];
-        const double pinv = (pv != 0.0) ? 1.0 / pv : 0.0;
-        __syncthreads();
-        for (int c = tid; c < n; c += nt) {
-            double v = (c == k) ? 1.0 : A[(long)k * n + c];
-            A[(long)k * n + c] = v * pinv;
-        }
-        __syncthreads();
-        for (int r = tid >> 6; r < n; r += (nt >> 6)) {
-            if (r == k) continue;
-            const double f = A[(long)r * n + k];
-            for (int c = tid & 63; c < n; c += 64) {
-                if (c == k) continue;
-                A[(long)r * n + c] -= f * A[(long)k * n + c];
-            }
-        }
-        __syncthreads();
-        for (int r = tid; r < n; r += nt) {
-            if (r == k) continue;
-            double f = A[(long)r * n + k];
-            A[(long)r * n + k] = -f * pinv;
+            perm[k] = p;
+            if (pv == 0.0) zero_at = k + 1;
         }
         __syncthreads();
     }
+    // undo the row swaps on the columns, last first: where column c ends up
+    int cc = c;
     for (int k = n - 1; k >= 0; k--) {
-        int p = perm[k];
-        if (p != k)
-            for (int r = tid; r < n; r += nt) {
-                double t = A[(long)r * n + k];
-                A[(long)r * n + k] = A[(long)r * n + p];
-                A[(long)r * n + p] = t;
-            }
-        __syncthreads();
+        const int p = perm[k];
+        cc = (cc == k) ? p : (cc == p ? k : cc);
     }
-}
-
-// x = Minv b over the compact list (FP64 arithmetic whatever the storage type)
-template <typename TS>
-__global__ void k_coarse_solve(int nd, const long *dofs, const double *Minv, const TS *b, TS *x)
-{
-    extern __shared__ double bs[];
-    for (int c = threadIdx.x; c < nd; c += blockDim.x) bs[c] = (double)Cvt<TS>::ld(b[dofs[c]]);
-    __syncthreads();
-    for (int r = threadIdx.x; r < nd; r += blockDim.x) {
-        double s = 0.0;
-        const double *row = Minv + (long)r * nd;
-        for (int c = 0; c < nd; c++) s += row[c] * bs[c];
-        x[dofs[r]] = Cvt<TS>::st((typename Cvt<TS>::C)s);
+    for (int e = 0; e < PER; e++) {
+        const int r = r0 + e * (GJ_NT / 64);
+        if (r < n && c < n) A[(long)r * n + cc] = M[r][c];
     }
-}
-
-// ------------------------------------------------ fused coarse V-cycle
-
-// One workgroup runs every pass of the coarse levels: each pass is a
-// workgroup-strided loop over the level's cells or nodes, passes are separated by
-// barriers (the level data, a few hundred KB, stays in L2).  The same bodies as the
-// per-level kernels, so the result is identical; it replaces about eleven
-// latency-bound launches per level.  b[l0] is the caller's right-hand side; bw[l]
-// (l > l0) receive the restricted residuals.
-template <typename TS, int DIM>
-__global__ void __launch_bounds__(512) k_vcycle_tail(const TailArgs<TS> *__restrict__ a, const TS *b0, TS *x0)
-{
-    extern __shared__ double bs[];
-    const long T = blockDim.x;
-    const int l0 = a->l0, L = a->L;
-    const float om = a->omega;
-    auto bof = [&](int l) -> const TS * { return l == 0 ? b0 : a->b[l]; };
-    auto xof = [&](int l) -> TS * { return l == 0 ? x0 : a->x[l]; };
-    auto smooth = [&](int l, int nu, int first, bool zero) {
-        const Lvl g = a->g[l];
-        const uint8_t *fl = a->fl[l];
-        const TS *al = a->al[l], *b = bof(l);
-        TS *x = xof(l), *t = a->t[l];
-        const long nc = (long)g.nx * g.ny * g.nz;
-        for (int sw = 0; sw < nu; sw++) {
-            if (zero && sw == 0)
-                for (long q = threadIdx.x; q < nc; q += T) smooth_body<TS, DIM, true>(g, fl, al, b, x, t, first, om, q);
-            else
-                for (long q = threadIdx.x; q < nc; q += T) smooth_body<TS, DIM, false>(g, fl, al, b, x, t, first, om, q);
-            __syncthreads();
-            for (long q = threadIdx.x; q < nc; q += T) smooth_body<TS, DIM, false>(g, fl, al, b, t, x, first ^ 1, om, q);
-            __syncthreads();
-        }
-    };
-    for (int l = l0; l + 1 < L; l++) {
-        const Lvl g = a->g[l];
-        if (a->nu_pre > 0) {
-            smooth(l, a->nu_pre, 0, true);
-        } else {
-            TS *x = xof(l);
-            for (long q = threadIdx.x; q < (long)g.nfield * g.S; q += T) x[q] = Cvt<TS>::st((typename Cvt<TS>::C)0);
-            __syncthreads();
-        }
-        for (long n = threadIdx.x; n < g.S; n += T) residual_body<TS, DIM>(g, a->fl[l], a->al[l], bof(l), xof(l), a->r[l], n);
-        __syncthreads();
-        const Lvl gc = a->g[l + 1];
-        for (long n = threadIdx.x; n < gc.S; n += T) restrict_body<TS, DIM>(g, gc, a->fl[l + 1], a->r[l], a->b[l + 1], n);
-        __syncthreads();
-    }
-    const int Lc = L - 1, nd = a->nd;
-    const TS *bc = bof(Lc);
-    TS *xc = xof(Lc);
-    const long *dofs = a->dofs;
-    for (int c = threadIdx.x; c < nd; c += T) bs[c] = (double)Cvt<TS>::ld(bc[dofs[c]]);
-    __syncthreads();
-    for (int r = threadIdx.x; r < nd; r += T) {
-        double sacc = 0.0;
-        const double *row = a->minv + (long)r * nd;
-        for (int c = 0; c < nd; c++) sacc += row[c] * bs[c];
-        xc[dofs[r]] = Cvt<TS>::st((typename Cvt<TS>::C)sacc);
-    }
-    __syncthreads();
-    for (int l = L - 2; l >= l0; l--) {
-        const Lvl g = a->g[l];
-        for (long n = threadIdx.x; n < g.S; n += T) prolong_body<TS, DIM>(g, a->g[l + 1], a->fl[l], a->x[l + 1], xof(l), n);
-        __syncthreads();
-        if (a->nu_post > 0) smooth(l, a->nu_post, 1, false);
-    }
-}
-
-// The same cycle with every level buffer staged in LDS (the levels of the tail
-// fit: ~136 KB in FP64 from 8^3 down): flags, alpha and the right-hand side are
-// loaded once, all passes read and write LDS, x of level l0 is written back.
-template <typename TS, int DIM>
-__global__ void __launch_bounds__(512) k_vcycle_tail_lds(const TailArgs<TS> *__restrict__ a, const TS *b0g, TS *x0g)
-{
-    __shared__ __align__(16) unsigned char pool[ST_TAIL_LDS_BYTES];
-    const long T = blockDim.x;
-    const int l0 = a->l0, L = a->L;
-    const float om = a->omega;
-    // level buffers in the pool, formed where they are used (so the compiler sees LDS
-    // pointers and emits LDS instructions, not flat ones)
-    auto Pfl = [&](int l) { return (uint8_t *)(pool + a->lds.fl[l]); };
-    auto Pal = [&](int l) { return (TS *)(pool + a->lds.al[l]); };
-    auto Pb = [&](int l) { return (TS *)(pool + a->lds.b[l]); };
-    auto Px = [&](int l) { return (TS *)(pool + a->lds.x[l]); };
-    auto Pt = [&](int l) { return (TS *)(pool + a->lds.t[l]); };
-    auto Pr = [&](int l) { return (TS *)(pool + a->lds.r[l]); };
-    for (long q = threadIdx.x; q < a->lds.bytes / 4; q += T) ((unsigned *)pool)[q] = 0u;  // padding = 0
-    __syncthreads();
-    for (int l = l0; l < L; l++) {
-        const Lvl g = a->g[l];
-        uint8_t *fl = (uint8_t *)Pfl(l);
-        TS *al = (TS *)Pal(l);
-        for (long q = threadIdx.x; q < g.S; q += T) fl[q] = a->fl[l][q];
-        for (long q = threadIdx.x; q < (long)g.dim * g.S; q += T) al[q] = a->al[l][q];
-    }
-    {
-        const Lvl g = a->g[l0];
-        const TS *bsrc = (l0 == 0) ? b0g : a->b[l0];
-        for (long q = threadIdx.x; q < (long)g.nfield * g.S; q += T) Pb(l0)[q] = bsrc[q];
-    }
-    __syncthreads();
-    auto smooth = [&](int l, int nu, int first, bool zero) {
-        const Lvl g = a->g[l];
-        const uint8_t *fl = Pfl(l);
-        const TS *al = Pal(l), *b = Pb(l);
-        TS *x = Px(l), *t = Pt(l);
-        const long nc = (long)g.nx * g.ny * g.nz;
-        for (int sw = 0; sw < nu; sw++) {
-            if (zero && sw == 0)
-                for (long q = threadIdx.x; q < nc; q += T) smooth_body<TS, DIM, true>(g, fl, al, b, x, t, first, om, q);
-            else
-                for (long q = threadIdx.x; q < nc; q += T) smooth_body<TS, DIM, false>(g, fl, al, b, x, t, first, om, q);
-            __syncthreads();
-            for (long q = threadIdx.x; q < nc; q += T) smooth_body<TS, DIM, false>(g, fl, al, b, t, x, first ^ 1, om, q);
-            __syncthreads();
-        }
-    };
-    for (int l = l0; l + 1 < L; l++) {
-        const Lvl g = a->g[l];
-        if (a->nu_pre > 0) {
-            smooth(l, a->nu_pre, 0, true);
-        } else {
-            for (long q = threadIdx.x; q < (long)g.nfield * g.S; q += T) Px(l)[q] = Cvt<TS>::st((typename Cvt<TS>::C)0);
-            __syncthreads();
-        }
-        for (long n = threadIdx.x; n < g.S; n += T) residual_body<TS, DIM>(g, Pfl(l), Pal(l), Pb(l), Px(l), Pr(l), n);
-        __syncthreads();
-        const Lvl gc = a->g[l + 1];
-        for (long n = threadIdx.x; n < gc.S; n += T) restrict_body<TS, DIM>(g, gc, Pfl(l + 1), Pr(l), Pb(l + 1), n);
-        __syncthreads();
-    }
-    const int Lc = L - 1, nd = a->nd;
-    double *bs = (double *)(pool + a->lds.bs);
-    const long *dofs = a->dofs;
-    for (int c = threadIdx.x; c < nd; c += T) bs[c] = (double)Cvt<TS>::ld(Pb(Lc)[dofs[c]]);
-    __syncthreads();
-    for (int r = threadIdx.x; r < nd; r += T) {
-        double sacc = 0.0;
-        const double *row = a->minv + (long)r * nd;
-        for (int c = 0; c < nd; c++) sacc += row[c] * bs[c];
-        Px(Lc)[dofs[r]] = Cvt<TS>::st((typename Cvt<TS>::C)sacc);
-    }
-    __syncthreads();
-    for (int l = L - 2; l >= l0; l--) {
-        const Lvl g = a->g[l];
-        for (long n = threadIdx.x; n < g.S; n += T) prolong_body<TS, DIM>(g, a->g[l + 1], Pfl(l), Px(l + 1), Px(l), n);
-        __syncthreads();
-        if (a->nu_post > 0) smooth(l, a->nu_post, 1, false);
-    }
-    {
-        const Lvl g = a->g[l0];
-        TS *xdst = (l0 == 0) ? x0g : a->x[l0];
-        for (long q = threadIdx.x; q < (long)g.nfield * g.S; q += T) xdst[q] = Px(l0)[q];
-    }
+    if (tid == 0) *info = zero_at;
 }
 
 // --------------------------------------------------- ABI <-> padded layout
@@ -1465,49 +1088,30 @@ static inline unsigned nb_grid(long n)
 template <typename TS>
 void launch_apply(const Lvl &g, const uint8_t *fl, const TS *al, const TS *x, TS *y, hipStream_t s)
 {
-    if (march_ok(g)) { march_apply<TS>(g, fl, al, x, y, s); return; }
-    if (g.dim == 3) hipLaunchKernelGGL((k_apply<TS, 3>), dim3(nb(g.S)), dim3(256), 0, s, g, fl, al, x, y);
-    else hipLaunchKernelGGL((k_apply<TS, 2>), dim3(nb(g.S)), dim3(256), 0, s, g, fl, al, x, y);
+    if (march_ok(g)) march_apply<TS>(g, fl, al, x, y, s);
+    else launch_node_apply<TS>(g, fl, al, x, y, s);
 }
 template <typename TS>
 void launch_residual(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b, const TS *x, TS *r, double *part,
                      hipStream_t s)
 {
-    if (march_ok(g)) { march_residual<TS>(g, fl, al, b, x, r, part, s); return; }
-    if (g.dim == 3) hipLaunchKernelGGL((k_residual<TS, 3>), dim3(nb(g.S)), dim3(256), 0, s, g, fl, al, b, x, r, part);
-    else hipLaunchKernelGGL((k_residual<TS, 2>), dim3(nb(g.S)), dim3(256), 0, s, g, fl, al, b, x, r, part);
+    if (march_ok(g)) march_residual<TS>(g, fl, al, b, x, r, part, s);
+    else launch_node_residual<TS>(g, fl, al, b, x, r, part, s);
 }
 unsigned residual_blocks(const Lvl &g) { return march_ok(g) ? march_blocks(g) : nb(g.S); }
 
 template <typename TS>
 void launch_smooth(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b, const TS *xin, TS *xout, int color,
-                   float omega, bool zero, hipStream_t s)
+                   float omega, bool zero, bool inner, hipStream_t s)
 {
-    long nc = (long)g.nx * g.ny * g.nz;
-    if (!zero && march_ok(g)) { march_smooth<TS>(g, fl, al, b, xin, xout, color, omega, s); return; }
-    if (zero && g.dim == 3 && g.nz % 2 == 0) {
-        hipLaunchKernelGGL((k_smooth0_pairs<TS>), dim3(nb(nc / 2)), dim3(256), 0, s, g, fl, al, b, xout, color, omega);
-        return;
-    }
-    if (g.dim == 3) {
-        if (zero) hipLaunchKernelGGL((k_smooth<TS, 3, true>), dim3(nb(nc)), dim3(256), 0, s, g, fl, al, b, xin, xout, color, omega);
-        else hipLaunchKernelGGL((k_smooth<TS, 3, false>), dim3(nb(nc)), dim3(256), 0, s, g, fl, al, b, xin, xout, color, omega);
-    } else {
-        if (zero) hipLaunchKernelGGL((k_smooth<TS, 2, true>), dim3(nb(nc)), dim3(256), 0, s, g, fl, al, b, xin, xout, color, omega);
-        else hipLaunchKernelGGL((k_smooth<TS, 2, false>), dim3(nb(nc)), dim3(256), 0, s, g, fl, al, b, xin, xout, color, omega);
-    }
+    if (!zero && march_ok(g)) march_smooth<TS>(g, fl, al, b, xin, xout, color, omega, s);
+    else launch_box<TS>(g, fl, al, b, xin, xout, color, omega, zero, inner, s);
 }
 template <typename TS>
 void launch_restrict(const Lvl &gf, const Lvl &gc, const uint8_t *flc, const TS *rf, TS *bc, hipStream_t s)
 {
     if (gf.dim == 3) hipLaunchKernelGGL((k_restrict<TS, 3>), dim3(nb(gc.S)), dim3(256), 0, s, gf, gc, flc, rf, bc);
     else hipLaunchKernelGGL((k_restrict<TS, 2>), dim3(nb(gc.S)), dim3(256), 0, s, gf, gc, flc, rf, bc);
-}
-template <typename TS>
-void launch_prolong(const Lvl &gf, const Lvl &gc, const uint8_t *flf, const TS *ec, TS *xf, hipStream_t s)
-{
-    if (gf.dim == 3) hipLaunchKernelGGL((k_prolong<TS, 3>), dim3(nb(gf.S)), dim3(256), 0, s, gf, gc, flf, ec, xf);
-    else hipLaunchKernelGGL((k_prolong<TS, 2>), dim3(nb(gf.S)), dim3(256), 0, s, gf, gc, flf, ec, xf);
 }
 template <typename TF, typename TC>
 void launch_coarsen(const Lvl &gf, const Lvl &gc, const uint8_t *flf, const TF *alf, uint8_t *flc, TC *alc,
@@ -1523,14 +1127,9 @@ void launch_probe(const Lvl &g, const uint8_t *fl, const TS *al, const long *dof
     if (g.dim == 3) hipLaunchKernelGGL((k_probe<TS, 3>), dim3(nd), dim3(256), 0, s, g, fl, al, dofs, nd, closed, A);
     else hipLaunchKernelGGL((k_probe<TS, 2>), dim3(nd), dim3(256), 0, s, g, fl, al, dofs, nd, closed, A);
 }
-void launch_gauss_jordan(int n, double *A, int *perm, int *info, hipStream_t s)
+void launch_gauss_jordan(int n, double *A, int *info, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_gauss_jordan, dim3(1), dim3(1024), 0, s, n, A, perm, info);
-}
-template <typename TS>
-void launch_coarse_solve(int nd, const long *dofs, const double *Minv, const TS *b, TS *x, hipStream_t s)
-{
-    hipLaunchKernelGGL((k_coarse_solve<TS>), dim3(1), dim3(512), nd * sizeof(double), s, nd, dofs, Minv, b, x);
+    hipLaunchKernelGGL(k_gauss_jordan, dim3(1), dim3(GJ_NT), 0, s, n, A, info);
 }
 template <typename TS>
 void launch_pack(const Lvl &g, const double *abi, TS *pad, int fixed_only, const uint8_t *fl, double scale,
@@ -1706,36 +1305,20 @@ void launch_fill(long n, TS *y, double v, hipStream_t s)
     hipLaunchKernelGGL((k_fill<TS>), dim3(nb_grid(n)), dim3(256), 0, s, n, y, v);
 }
 
-template <typename TS>
-void launch_vcycle_tail(const TailArgs<TS> *a, int dim, const TS *b0, TS *x0, int nd, bool lds, hipStream_t s)
-{
-    if (lds) {
-        if (dim == 3) hipLaunchKernelGGL((k_vcycle_tail_lds<TS, 3>), dim3(1), dim3(512), 0, s, a, b0, x0);
-        else hipLaunchKernelGGL((k_vcycle_tail_lds<TS, 2>), dim3(1), dim3(512), 0, s, a, b0, x0);
-        return;
-    }
-    const size_t sh = sizeof(double) * (size_t)(nd > 0 ? nd : 1);
-    if (dim == 3) hipLaunchKernelGGL((k_vcycle_tail<TS, 3>), dim3(1), dim3(512), sh, s, a, b0, x0);
-    else hipLaunchKernelGGL((k_vcycle_tail<TS, 2>), dim3(1), dim3(512), sh, s, a, b0, x0);
-}
-
 // explicit instantiations
 #define INST_TS(T)                                                                                          \
     template void launch_apply<T>(const Lvl &, const uint8_t *, const T *, const T *, T *, hipStream_t);     \
     template void launch_residual<T>(const Lvl &, const uint8_t *, const T *, const T *, const T *, T *,     \
                                      double *, hipStream_t);                                               \
     template void launch_smooth<T>(const Lvl &, const uint8_t *, const T *, const T *, const T *, T *, int,  \
-                                   float, bool, hipStream_t);                                              \
+                                   float, bool, bool, hipStream_t);                                              \
     template void launch_restrict<T>(const Lvl &, const Lvl &, const uint8_t *, const T *, T *, hipStream_t); \
-    template void launch_prolong<T>(const Lvl &, const Lvl &, const uint8_t *, const T *, T *, hipStream_t);  \
     template void launch_probe<T>(const Lvl &, const uint8_t *, const T *, const long *, int, int, double *,   \
                                   hipStream_t);                                                            \
-    template void launch_coarse_solve<T>(int, const long *, const double *, const T *, T *, hipStream_t);    \
     template void launch_pack<T>(const Lvl &, const double *, T *, int, const uint8_t *, double, hipStream_t); \
     template void launch_unpack<T>(const Lvl &, const T *, double *, hipStream_t);                          \
     template void launch_alpha_from_pen<T>(const Lvl &, const double *, const uint8_t *, T *, hipStream_t);  \
-    template void launch_fill<T>(long, T *, double, hipStream_t);                                           \
-    template void launch_vcycle_tail<T>(const TailArgs<T> *, int, const T *, T *, int, bool, hipStream_t);
+    template void launch_fill<T>(long, T *, double, hipStream_t);
 
 INST_TS(double)
 INST_TS(float)

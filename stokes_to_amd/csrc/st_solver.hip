@@ -32,8 +32,6 @@ namespace {
 
 template <typename TS> struct Hier {
     std::vector<TS *> al, b, x, t, r;
-    TailArgs<TS> *tail = nullptr;  // device copy of the fused coarse V-cycle's arguments
-    bool tail_lds = false;         // its levels fit the LDS pool
 };
 
 struct Net;  // learned predictor (st_net.hip)
@@ -52,7 +50,7 @@ struct st_ctx {
     long *d_dofs = nullptr;
     int nd = 0;
     double *d_minv = nullptr;
-    int *d_perm = nullptr, *d_info = nullptr;
+    int *d_info = nullptr;
     // finest FP64 state (padded)
     long ndof = 0, ncell = 0, nvec = 0;  // ABI sizes and padded vector length
     double *X = nullptr, *B = nullptr, *XD = nullptr, *BODY = nullptr, *LAM = nullptr, *BA = nullptr, *ZERO = nullptr;
@@ -248,7 +246,7 @@ static int setup_hierarchy(st_ctx *c)
     if (c->prm.precision == ST_BF16) convert_alpha<bf16>(c);
     const int Lc = c->L - 1;
     launch_probe<double>(c->lv[Lc], c->fl[Lc], c->h64.al[Lc], c->d_dofs, c->nd, c->prm.closed, c->d_minv, c->s);
-    launch_gauss_jordan(c->nd, c->d_minv, c->d_perm, c->d_info, c->s);
+    launch_gauss_jordan(c->nd, c->d_minv, c->d_info, c->s);
     int info = 0;
     CK(hipMemcpyAsync(&info, c->d_info, sizeof(int), hipMemcpyDeviceToHost, c->s));
     hipEvent_t e3;
@@ -287,9 +285,9 @@ template <typename TS> static void smooth(st_ctx *c, int l, const TS *b, TS *x, 
             int sw = 0;
             if (zero) {
                 if (pr) prof_mark(c, ST_PROF_SMOOTH0);
-                launch_smooth<TS>(g, c->fl[l], h.al[l], b, x, x, first, om, true, c->s);
+                launch_smooth<TS>(g, c->fl[l], h.al[l], b, x, x, first, om, true, l > 0, c->s);
                 if (pr) { prof_mark(c, ST_PROF_SMOOTH0); prof_mark(c, ST_PROF_SMOOTH); }
-                launch_smooth<TS>(g, c->fl[l], h.al[l], b, x, t, first ^ 1, om, false, c->s);
+                launch_smooth<TS>(g, c->fl[l], h.al[l], b, x, t, first ^ 1, om, false, l > 0, c->s);
                 if (pr) prof_mark(c, ST_PROF_SMOOTH);
                 src = t;
                 dst = x;
@@ -309,117 +307,64 @@ template <typename TS> static void smooth(st_ctx *c, int l, const TS *b, TS *x, 
         // the pass from x = 0 is another kernel (k_smooth0_pairs) with other bytes
         const int k0 = (zero && sw == 0) ? ST_PROF_SMOOTH0 : ST_PROF_SMOOTH;
         if (pr) prof_mark(c, k0);
-        launch_smooth<TS>(g, c->fl[l], h.al[l], b, x, t, first, om, zero && sw == 0, c->s);
+        launch_smooth<TS>(g, c->fl[l], h.al[l], b, x, t, first, om, zero && sw == 0, l > 0, c->s);
         if (pr) { prof_mark(c, k0); prof_mark(c, ST_PROF_SMOOTH); }
-        launch_smooth<TS>(g, c->fl[l], h.al[l], b, t, x, first ^ 1, om, false, c->s);
+        launch_smooth<TS>(g, c->fl[l], h.al[l], b, t, x, first ^ 1, om, false, l > 0, c->s);
         if (pr) prof_mark(c, ST_PROF_SMOOTH);
     }
 }
 
-// first level handled by the fused coarse V-cycle: the largest level with at most
-// ST_TAIL_MAX_CELLS cells (one workgroup), or L when there is none
+// first level handled by the fused coarse V-cycle (st_coarse.hip): 8 cells a side in
+// 3D; in 2D 32, or the grid itself when it is smaller.  The line lies where one CU stops keeping up: a pass over 8^3 or 32^2
+// takes it ~1 us against 4-5 us for a launch, over 16^3 or 64^2 6 us (8-16 times the
+// cells, and in FP64 more than the LDS holds).
 static int tail_level(const st_ctx *c)
 {
-    for (int l = 0; l < c->L; l++) {
-        const Lvl &g = c->lv[l];
-        if ((long)g.nx * g.ny * g.nz <= ST_TAIL_MAX_CELLS) return l;
+    const int side = (c->dim == 3) ? 8 : 32;
+    int l = 0;
+    while (c->lv[l].nx > side) l++;
+    return l;
+}
+
+template <typename TS> static TailArgs<TS> tail_args(st_ctx *c, int l0)
+{
+    Hier<TS> &h = hier<TS>(c);
+    TailArgs<TS> a;
+    std::memset(&a, 0, sizeof(a));
+    a.nu_pre = c->prm.nu_pre;
+    a.nu_post = c->prm.nu_post;
+    a.nd = c->nd;
+    a.omega = (float)c->prm.omega;
+    for (int l = l0; l < c->L; l++) {
+        a.fl[l - l0] = c->fl[l];
+        a.al[l - l0] = h.al[l];
     }
-    return c->L;
+    a.minv = c->d_minv;
+    return a;
 }
 
 template <typename TS> static void vcycle(st_ctx *c, const TS *b0, TS *x0)
 {
     Hier<TS> &h = hier<TS>(c);
-    const int L = c->L;
     const int lt = tail_level(c);
-    for (int l = 0; l + 1 < L && l < lt; l++) {
+    for (int l = 0; l < lt; l++) {
         const Lvl &g = c->lv[l];
         const TS *b = (l == 0) ? b0 : h.b[l];
         TS *x = (l == 0) ? x0 : h.x[l];
         if (c->prm.nu_pre > 0) smooth<TS>(c, l, b, x, c->prm.nu_pre, 0, true);
         else launch_fill<TS>((long)g.nfield * g.S, x, 0.0, c->s);
         if (l == 0) prof_mark(c, ST_PROF_RESIDUAL);
-        launch_residual<TS>(g, c->fl[l], h.al[l], b, x, h.r[l], nullptr, c->s);
-        if (l == 0) prof_mark(c, ST_PROF_RESIDUAL);
-        launch_restrict<TS>(g, c->lv[l + 1], c->fl[l + 1], h.r[l], h.b[l + 1], c->s);
-    }
-    if (lt < L) {
-        if (!h.tail) {  // built once: the level buffers do not move
-            TailArgs<TS> a;
-            std::memset(&a, 0, sizeof(a));
-            a.l0 = lt;
-            a.L = L;
-            a.nu_pre = c->prm.nu_pre;
-            a.nu_post = c->prm.nu_post;
-            a.nd = c->nd;
-            a.dim = c->dim;
-            a.omega = (float)c->prm.omega;
-            for (int l = lt; l < L; l++) {
-                a.g[l] = c->lv[l];
-                a.fl[l] = c->fl[l];
-                a.al[l] = h.al[l];
-                a.b[l] = h.b[l];
-                a.x[l] = h.x[l];
-                a.t[l] = h.t[l];
-                a.r[l] = h.r[l];
-            }
-            a.dofs = c->d_dofs;
-            a.minv = c->d_minv;
-            // LDS layout of the staged variant (16-byte aligned buffers)
-            {
-                long off = 0;
-                auto take = [&](long bytes) {
-                    const long o = off;
-                    off += (bytes + 15) / 16 * 16;
-                    return (int)o;
-                };
-                for (int l = lt; l < L; l++) {
-                    const Lvl &g = c->lv[l];
-                    const long nv = (long)g.nfield * g.S;
-                    a.lds.fl[l] = take(g.S);
-                    a.lds.al[l] = take((long)g.dim * g.S * sizeof(TS));
-                    a.lds.b[l] = take(nv * sizeof(TS));
-                    a.lds.x[l] = take(nv * sizeof(TS));
-                    a.lds.t[l] = take(nv * sizeof(TS));
-                    a.lds.r[l] = take(nv * sizeof(TS));
-                }
-                a.lds.bs = take((long)c->nd * sizeof(double));
-                a.lds.bytes = (int)off;
-                a.lds.ok = off <= ST_TAIL_LDS_BYTES;
-            }
-            h.tail_lds = a.lds.ok != 0;
-            void *p = nullptr;
-            if (hipMalloc(&p, sizeof(a)) == hipSuccess && hipMemcpy(p, &a, sizeof(a), hipMemcpyHostToDevice) == hipSuccess) {
-                c->allocs.push_back(p);
-                h.tail = (TailArgs<TS> *)p;
-            }
+        if (march_ok(g)) {
+            launch_residual<TS>(g, c->fl[l], h.al[l], b, x, h.r[l], nullptr, c->s);
+            if (l == 0) prof_mark(c, ST_PROF_RESIDUAL);
+            launch_restrict<TS>(g, c->lv[l + 1], c->fl[l + 1], h.r[l], h.b[l + 1], c->s);
+        } else {
+            launch_resid_restrict<TS>(g, c->lv[l + 1], c->fl[l], h.al[l], b, x, c->fl[l + 1], h.b[l + 1], l > 0, c->s);
+            if (l == 0) prof_mark(c, ST_PROF_RESIDUAL);
         }
-        if (h.tail) {
-            launch_vcycle_tail<TS>(h.tail, c->dim, lt == 0 ? b0 : h.b[lt], lt == 0 ? x0 : h.x[lt], c->nd, h.tail_lds,
-                                   c->s);
-        } else {  // allocation failed: per-level kernels (same arithmetic)
-            for (int l = lt; l + 1 < L; l++) {
-                const Lvl &g = c->lv[l];
-                const TS *b = (l == 0) ? b0 : h.b[l];
-                TS *x = (l == 0) ? x0 : h.x[l];
-                if (c->prm.nu_pre > 0) smooth<TS>(c, l, b, x, c->prm.nu_pre, 0, true);
-                else launch_fill<TS>((long)g.nfield * g.S, x, 0.0, c->s);
-                launch_residual<TS>(g, c->fl[l], h.al[l], b, x, h.r[l], nullptr, c->s);
-                launch_restrict<TS>(g, c->lv[l + 1], c->fl[l + 1], h.r[l], h.b[l + 1], c->s);
-            }
-            launch_coarse_solve<TS>(c->nd, c->d_dofs, c->d_minv, (L - 1 == 0) ? b0 : h.b[L - 1],
-                                    (L - 1 == 0) ? x0 : h.x[L - 1], c->s);
-            for (int l = L - 2; l >= lt; l--) {
-                const TS *b = (l == 0) ? b0 : h.b[l];
-                TS *x = (l == 0) ? x0 : h.x[l];
-                launch_prolong<TS>(c->lv[l], c->lv[l + 1], c->fl[l], h.x[l + 1], x, c->s);
-                if (c->prm.nu_post > 0) smooth<TS>(c, l, b, x, c->prm.nu_post, 1, false);
-            }
-        }
-    } else {
-        launch_coarse_solve<TS>(c->nd, c->d_dofs, c->d_minv, h.b[L - 1], h.x[L - 1], c->s);
     }
-    for (int l = std::min(lt, L - 1) - 1; l >= 0; l--) {
+    launch_vcycle_tail<TS>(tail_args<TS>(c, lt), c->dim, c->lv[lt].nx, lt == 0 ? b0 : h.b[lt], lt == 0 ? x0 : h.x[lt], lt > 0, c->s);
+    for (int l = lt - 1; l >= 0; l--) {
         const TS *b = (l == 0) ? b0 : h.b[l];
         TS *x = (l == 0) ? x0 : h.x[l];
         launch_prolong<TS>(c->lv[l], c->lv[l + 1], c->fl[l], h.x[l + 1], x, c->s);
@@ -649,7 +594,7 @@ template <typename TS> static int mg_smooth_lowp(st_ctx *c, int l, int color, co
     CKR(stage_in(c, xin, nd));
     launch_pack<TS>(g, c->abi_a, xi, 0, c->fl[l], 1.0, c->s);
     launch_fill<TS>((long)g.nfield * g.S, xo, 0.0, c->s);
-    launch_smooth<TS>(g, c->fl[l], hier<TS>(c).al[l], bb, xi, xo, color, (float)c->prm.omega, false, c->s);
+    launch_smooth<TS>(g, c->fl[l], hier<TS>(c).al[l], bb, xi, xo, color, (float)c->prm.omega, false, false, c->s);
     launch_unpack<TS>(g, xo, c->abi_b, c->s);
     return stage_out(c, xout, nd);
 }
@@ -785,7 +730,6 @@ int st_create(st_ctx **out, const st_params *p)
         c->nd = (int)dofs.size();
         rc = dalloc(c, &c->d_dofs, c->nd);
         if (rc == ST_OK) rc = dalloc(c, &c->d_minv, (long)c->nd * c->nd);
-        if (rc == ST_OK) rc = dalloc(c, &c->d_perm, c->nd);
         if (rc == ST_OK) rc = dalloc(c, &c->d_info, 4);
         if (rc == ST_OK && hipMemcpy(c->d_dofs, dofs.data(), sizeof(long) * c->nd, hipMemcpyHostToDevice) != hipSuccess)
             rc = ST_EHIP;
@@ -1905,7 +1849,7 @@ int st_mg_smooth(st_ctx *c, int l, int color, const double *b, const double *xin
     CKR(stage_in(c, xin, nd));
     launch_pack<double>(g, c->abi_a, c->Wv, 0, c->fl[l], 1.0, c->s);
     launch_fill<double>((long)g.nfield * g.S, c->V, 0.0, c->s);
-    launch_smooth<double>(g, c->fl[l], c->h64.al[l], c->BA, c->Wv, c->V, color, (float)c->prm.omega, false, c->s);
+    launch_smooth<double>(g, c->fl[l], c->h64.al[l], c->BA, c->Wv, c->V, color, (float)c->prm.omega, false, false, c->s);
     launch_unpack<double>(g, c->V, c->abi_b, c->s);
     return stage_out(c, xout, nd);
 }

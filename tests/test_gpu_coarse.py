@@ -1,0 +1,48 @@
+"""The kernels of the levels that are not marched (st_coarse.hip) against the oracle's
+V-cycle, smoother and transfers: every side at which the fused coarsest cycle, the
+one-launch residual and restriction, and their level-0 forms (values on fixed DOFs)
+start or end.  FP64 bars are those of the parity tests (1e-10 relative)."""
+import numpy as np
+import pytest
+
+from conftest import rel
+from helpers import oracle_desc, setup, solver_for
+from stokes_to_amd.problems import reference_test0
+
+pytestmark = pytest.mark.gpu
+
+
+def scattered(P, seed):
+    """P's flags with 2% more fixed cells and interior faces."""
+    rng = np.random.default_rng(seed)
+    f = P.fixed.copy()
+    f[rng.integers(0, f.size, f.size // 50)] = 1
+    return f
+
+
+@pytest.mark.parametrize("dim,n", [(2, 8), (2, 16), (2, 32), (2, 64), (2, 128), (3, 8), (3, 16), (3, 32)])
+@pytest.mark.parametrize("nu", [(1, 2), (0, 1), (2, 1), (1, 0), (2, 3)])
+def test_vcycle_matches_oracle_with_fixed_dofs(make_solver, orc, dim, n, nu):
+    P, rho = setup(dim, n, sigma=max(1.5, n / 12))
+    P.fixed[:] = scattered(P, n)
+    fixed, vol, pen = oracle_desc(orc, P, rho)
+    s = solver_for(make_solver, P, rho, nu_pre=nu[0], nu_post=nu[1])
+    mg = orc.MG(dim, P.shape, fixed, pen, nu_pre=nu[0], nu_post=nu[1], omega=1.0, tang=0)
+    b = np.random.default_rng(7).standard_normal(fixed.size)
+    assert rel(s.mg_vcycle(b), mg.vcycle(b)) < 1e-10
+
+
+@pytest.mark.parametrize("dim,n", [(2, 32), (3, 64)])
+def test_closed_box_solves_reach_rtol(make_solver, dim, n):
+    """The gauge of a closed box passes through the LDS inverse of the coarsest matrix."""
+    P = reference_test0(dim, n)
+    a = P.alpha
+    s = make_solver(dim, n, rtol=1e-10, alpha_max=a.alpha_max, alpha_min=a.alpha_min, q=a.q, power=a.power,
+                    alpha_scale=a.scale)
+    s.init_boundary(P.fixed, closed=True)
+    s.set_design(np.full(n ** dim, 0.3))
+    s.update_b(body=P.body)
+    x, st = s.solve()
+    assert st["converged"]
+    b = np.where(P.fixed.astype(bool), 0.0, P.body)
+    assert rel(s.applyMapping(x), b) < 1e-9
