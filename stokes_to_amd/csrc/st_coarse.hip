@@ -329,18 +329,218 @@ __global__ void __launch_bounds__(256) k_prolong(Lvl gf, Lvl gc, const uint8_t *
     }
 }
 
+// ------------------------------------------------------------ LDS tiles
+
+// A box of NI x NJ x NK nodes (NK = 1 in 2D) of x and the flags in LDS, entries outside
+// the level zero, so that the stencil needs no range test and its offsets are constants
+// of the LDS instructions.
+template <typename TS, int DIM, int NI, int NJ, int NK> struct Tile {
+    typedef typename Cvt<TS>::C C;
+    static constexpr int SI = DIM == 3 ? NJ * NK : NJ, SJ = DIM == 3 ? NK : 1, SK = DIM == 3 ? 1 : 0, N = NI * NJ * NK;
+    TS x[DIM + 1][N];
+    uint8_t f[N];
+
+    // nodes from (i0, j0, k0); PROL: x + P ec instead of x; ZERO: x = 0 and not read
+    template <int NT, bool ZERO, bool PROL>
+    __device__ __forceinline__ void load(const Lvl &g, const uint8_t *fl, const TS *xg, const Lvl &gc, const TS *ec, int i0,
+                                         int j0, int k0)
+    {
+        static_assert(!PROL || DIM == 2, "the prolongation is fused in 2D");
+#pragma unroll 2
+        for (int t = threadIdx.x; t < N; t += NT) {
+            int i, j, k;
+            if (DIM == 3) {
+                k = k0 + t % NK;
+                j = j0 + (t / NK) % NJ;
+                i = i0 + t / (NK * NJ);
+            } else {
+                k = 0;
+                j = j0 + t % NJ;
+                i = i0 + t / NJ;
+            }
+            const bool in = i >= 0 && i <= g.nx && j >= 0 && j <= g.ny && (DIM == 2 || (k >= 0 && k <= g.nz));
+            const unsigned q = in ? ((unsigned)i * (unsigned)g.Py + (unsigned)j) * (unsigned)g.Pz + (unsigned)k : 0u;
+            const int fb = in ? (int)at(fl, q) : 0;
+            f[t] = (uint8_t)fb;
+            if (ZERO) {
+#pragma unroll
+                for (int c = 0; c <= DIM; c++) x[c][t] = Cvt<TS>::st(C(0));
+                continue;
+            }
+            TS v[DIM + 1];
+#pragma unroll
+            for (int c = 0; c <= DIM; c++) v[c] = at(xg + c * g.S, q);
+            if constexpr (PROL) {  // as k_prolong
+                const unsigned qc = in ? (unsigned)(i >> 1) * (unsigned)gc.Py + (unsigned)(j >> 1) : 0u;
+#pragma unroll
+                for (int c = 0; c <= 2; c++) {
+                    C e = Cvt<TS>::ld(at(ec + c * gc.S, qc));
+                    if (c == 0) {
+                        e = C(0.5) * e;
+                    } else {
+                        const bool odd = (c == 1 ? i : j) & 1;
+                        const C h = Cvt<TS>::ld(at(ec + c * gc.S, odd && in ? qc + (c == 1 ? (unsigned)gc.Py : 1u) : qc));
+                        if (odd) {
+                            e = e + h;
+                            e *= C(0.5);
+                        }
+                    }
+                    if ((fb >> c) & 1) v[c] = Cvt<TS>::st(Cvt<TS>::ld(v[c]) + e);
+                }
+            }
+#pragma unroll
+            for (int c = 0; c <= DIM; c++) x[c][t] = in ? v[c] : Cvt<TS>::st(C(0));
+        }
+    }
+};
+
+// --------------------------------------------------------- sweeps in 2D
+
+// NPASS colour passes (first colour col0) of a 2D level in one launch: a workgroup holds
+// a tile of 16 x 16 cells and a ring of 2 (NPASS - 1) cells around it in LDS and updates
+// it in place, the ring losing two cells a side per pass, so no workgroup waits for
+// another; the passes on the ring are done by every tile that needs them.  A lane keeps
+// its pair of cells (one of each colour) and their right-hand sides and penalties in
+// registers for all passes.  ZERO: x starts at zero; PROL: at xin + P ec (the
+// prolongated correction).
+//
+// The four passes and the prolongation after the coarse correction take 9-12 us (64^2 to
+// 256^2, FP32 / FP64) against five launches of 3.5-5.7 us; a whole FP64 solve 128^2 1.84 ->
+// 1.54 ms, 512^2 3.08 -> 2.63, 1024^2 7.23 -> 6.60, so every 2D level takes this way.  In
+// 3D the ring of one sweep is six times a tile of the same memory: measured as two
+// passes per launch, 32^3 FP64 solves 2.03 -> 2.02 ms, 64^3 and 128^3 slower.
+template <int NPASS> struct SwTile {
+    static constexpr int H = 2 * (NPASS - 1), TI = 16, TJ = 16;
+    static constexpr int RI = TI + 2 * H, RJ = TJ + 2 * H;                     // cells of the first pass
+    static constexpr int NP = RI * RJ / 2, NT = (NP + 63) / 64 * 64;           // a lane per pair of them
+    static constexpr int NI = RI + 3, NJ = RJ + 3;                             // nodes: one below, two above
+};
+
+// the pair's right-hand sides and penalties: x faces [high][cell], y faces low to high
+template <typename C> struct PairOps {
+    C p[2], bx[2][2], ax[2][2], by[3], ay[3];
+};
+template <typename TS, typename T, bool M> struct PairAcc {
+    typedef typename Cvt<TS>::C C;
+    static constexpr bool MASK = M;
+    const T &t;
+    const PairOps<C> &o;
+    int q;
+    bool par;  // the odd cell of the pair
+    __device__ __forceinline__ int F(int di, int dj, int) const { return t.f[q + di * T::SI + dj * T::SJ]; }
+    __device__ __forceinline__ C X(int f, int di, int dj, int) const { return Cvt<TS>::ld(t.x[f][q + di * T::SI + dj * T::SJ]); }
+    // by value: a conditional between two members would be an address, and keep the
+    // operands out of registers
+    __device__ __forceinline__ C sel(C even, C odd) const { return par ? odd : even; }
+    __device__ __forceinline__ C B(int f, int di, int dj, int) const
+    { return f == 0 ? sel(o.p[0], o.p[1]) : (f == 1 ? sel(o.bx[di][0], o.bx[di][1]) : sel(o.by[dj], o.by[1 + dj])); }
+    __device__ __forceinline__ C AL(int d, int di, int dj, int) const
+    { return d == 0 ? sel(o.ax[di][0], o.ax[di][1]) : sel(o.ay[dj], o.ay[1 + dj]); }
+};
+
+template <typename TS, int NPASS, bool ZERO, bool PROL, bool MASK>
+__global__ void __launch_bounds__(SwTile<NPASS>::NT) k_sweeps(Lvl g, Lvl gc, const uint8_t *__restrict__ fl,
+                                                              const TS *__restrict__ al, const TS *__restrict__ b,
+                                                              const TS *__restrict__ xin, const TS *__restrict__ ec,
+                                                              TS *__restrict__ xout, int col0, float omega)
+{
+    typedef typename Cvt<TS>::C C;
+    typedef SwTile<NPASS> W;
+    typedef Tile<TS, 2, W::NI, W::NJ, 1> T;
+    __shared__ T s;
+    const int I0 = blockIdx.y * W::TI, J0 = blockIdx.x * W::TJ;
+    // the lane's pair (i, j), (i, j + 1) in the region of the first pass
+    const int t = threadIdx.x, rj = 2 * (t % (W::RJ / 2)), ri = t / (W::RJ / 2);
+    const int i = I0 - W::H + ri, j = J0 - W::H + rj;
+    const bool in = t < W::NP && i >= 0 && i < g.nx && j >= 0 && j < g.ny;
+    const unsigned q = in ? (unsigned)i * (unsigned)g.Py + (unsigned)j : 0u;
+    PairOps<C> o;
+    if (in) {
+        auto ldb = [&](int f, long off) -> C { return Cvt<TS>::ld(at(b + f * g.S + off, q)); };
+        auto lda = [&](int d, long off) -> C { return Cvt<TS>::ld(at(al + d * g.S + off, q)); };
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            o.p[c] = ldb(0, c);
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                o.bx[h][c] = ldb(1, h * g.Py + c);
+                o.ax[h][c] = lda(0, h * g.Py + c);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < 3; h++) {
+            o.by[h] = ldb(2, h);
+            o.ay[h] = lda(1, h);
+        }
+    }
+    s.template load<W::NT, ZERO, PROL>(g, fl, xin, gc, ec, I0 - W::H - 1, J0 - W::H - 1, 0);
+    __syncthreads();
+    const int n0 = (ri + 1) * T::SI + rj + 1;  // LDS node of the even cell
+#pragma unroll 1
+    for (int p = 0; p < NPASS; p++) {
+        const int ring = 2 * p;  // cells of the first region that this pass leaves out, a side
+        const bool on = in && ri >= ring && ri < W::RI - ring && rj >= ring && rj < W::RJ - ring;
+        const bool par = (i + j + col0 + p) & 1;  // which cell has this pass's colour
+        const int n1 = n0 + (par ? 1 : 0);
+        C pn, u0[3], u1[3];
+        if (on) {
+            const PairAcc<TS, T, MASK> a{s, o, n1, par};
+            if (ZERO && p == 0) box_cell<C, 2, true>(a, omega, pn, u0, u1);
+            else box_cell<C, 2, false>(a, omega, pn, u0, u1);
+        }
+        if (p + 1 < NPASS) {
+            __syncthreads();
+            if (on) {
+                s.x[0][n1] = Cvt<TS>::st(pn);
+                s.x[1][n1] = Cvt<TS>::st(u0[0]);
+                s.x[1][n1 + T::SI] = Cvt<TS>::st(u1[0]);
+                s.x[2][n1] = Cvt<TS>::st(u0[1]);
+                s.x[2][n1 + 1] = Cvt<TS>::st(u1[1]);
+            }
+            __syncthreads();
+        } else if (on) {  // the tile's own cells: their block, and what the colour does not own
+            const unsigned qc = q + (par ? 1u : 0u), qo = q + (par ? 0u : 1u);
+            const int no = n0 + (par ? 0 : 1), oj = j + (par ? 0 : 1);
+            put(xout, qo, s.x[0][no]);
+            if (i == 0) put(xout + g.S, qo, s.x[1][no]);
+            if (i == g.nx - 1) put(xout + g.S + g.Py, qo, s.x[1][no + T::SI]);
+            if (oj == 0) put(xout + 2 * g.S, qo, s.x[2][no]);
+            if (oj == g.ny - 1) put(xout + 2 * g.S + 1, qo, s.x[2][no + 1]);
+            put(xout, qc, Cvt<TS>::st(pn));
+            put(xout + g.S, qc, Cvt<TS>::st(u0[0]));
+            put(xout + g.S + g.Py, qc, Cvt<TS>::st(u1[0]));
+            put(xout + 2 * g.S, qc, Cvt<TS>::st(u0[1]));
+            put(xout + 2 * g.S + 1, qc, Cvt<TS>::st(u1[1]));
+        }
+    }
+}
+
 // ------------------------------------------------- residual + restriction
 
-// Coarse right-hand side R (b - A x) in one launch: a workgroup evaluates the fine
-// residual on the (2 CI + 1) x (2 CJ + 1) x (2 CK + 1) nodes under its CI x CJ x CK
-// coarse nodes into LDS (rounded to the storage type, as a stored residual is) and
-// restricts from there with restrict_body's sums.  The residual never reaches memory
+// Coarse right-hand side R (b - A x) in one launch: a workgroup stages x around its CI x
+// CJ x CK coarse nodes in LDS, evaluates the fine residual on the (2 CI + 1) x (2 CJ + 1) x
+// (2 CK + 1) nodes under them (rounded to the storage type, as a stored residual is) and
+// restricts from LDS with restrict_body's sums.  The residual never reaches memory
 // and one launch of each level's cycle is saved; 1.3-1.5 of the residual rows are
 // evaluated twice, which on these levels is cheaper than a launch.
 template <int DIM> struct RrTile {  // NT: one lane per residual node
     static constexpr int CI = DIM == 3 ? 2 : 4, CJ = DIM == 3 ? 4 : 16, CK = DIM == 3 ? 8 : 1;
     static constexpr int FI = 2 * CI + 1, FJ = 2 * CJ + 1, FK = DIM == 3 ? 2 * CK + 1 : 1, N = FI * FJ * FK;
     static constexpr int NT = (N + 63) / 64 * 64;
+};
+// a residual node in the tile: b and alpha of the own node from memory
+template <typename TS, int DIM, typename T, bool M> struct RrAcc {
+    typedef typename Cvt<TS>::C C;
+    static constexpr bool MASK = M;
+    const T &t;
+    const TS *al;
+    long S;
+    int n0;
+    unsigned q;
+    __device__ __forceinline__ int n(int di, int dj, int dk) const { return n0 + di * T::SI + dj * T::SJ + dk * T::SK; }
+    __device__ __forceinline__ int F(int di, int dj, int dk) const { return t.f[n(di, dj, dk)]; }
+    __device__ __forceinline__ C X(int f, int di, int dj, int dk) const { return Cvt<TS>::ld(t.x[f][n(di, dj, dk)]); }
+    __device__ __forceinline__ C AL(int d, int, int, int) const { return Cvt<TS>::ld(at(al + d * S, q)); }
 };
 
 // row f of the restriction at a free coarse DOF (else 0) from the residual r of field f
@@ -375,22 +575,30 @@ __global__ void __launch_bounds__(RrTile<DIM>::NT) k_resid_restrict(Lvl gf, Lvl 
 {
     typedef typename Cvt<TS>::C C;
     typedef RrTile<DIM> T;
+    typedef Tile<TS, DIM, T::FI + 2, T::FJ + 2, DIM == 3 ? T::FK + 2 : 1> X;
+    __shared__ X xt;
     __shared__ TS sr[DIM + 1][T::N];
     const int K0 = blockIdx.x * T::CK, J0 = blockIdx.y * T::CJ, I0 = blockIdx.z * T::CI;
-    if (const int t = threadIdx.x; t < T::N) {
-        const int c = t % T::FK, r = t / T::FK;
-        const int i = 2 * I0 - 1 + r / T::FJ, j = 2 * J0 - 1 + r % T::FJ, k = DIM == 3 ? 2 * K0 - 1 + c : 0;
-        C v[4] = {C(0), C(0), C(0), C(0)};
-        if (i >= 0 && j >= 0 && k >= 0 && i <= gf.nx && j <= gf.ny && (DIM == 2 || k <= gf.nz)) {
-            const NodeAcc<TS, DIM, MASK> a(gf, flf, al, x, i, j, k);
-            const BoxSten<C, DIM, NodeAcc<TS, DIM, MASK>> s{a};
-            v[0] = Cvt<TS>::ld(at(b, a.q)) - s.cell();
-            v[1] = Cvt<TS>::ld(at(b + gf.S, a.q)) - s.template face<0>(0, 0, 0);
-            v[2] = Cvt<TS>::ld(at(b + 2 * gf.S, a.q)) - s.template face<1>(0, 0, 0);
-            if (DIM == 3) v[3] = Cvt<TS>::ld(at(b + 3 * gf.S, a.q)) - s.template face<2>(0, 0, 0);
-        }
+    const int t0 = threadIdx.x;
+    const int fk = t0 % T::FK, fj = (t0 / T::FK) % T::FJ, fi = t0 / (T::FK * T::FJ);
+    const int i = 2 * I0 - 1 + fi, j = 2 * J0 - 1 + fj, k = DIM == 3 ? 2 * K0 - 1 + fk : 0;
+    const bool in = t0 < T::N && i >= 0 && j >= 0 && k >= 0 && i <= gf.nx && j <= gf.ny && (DIM == 2 || k <= gf.nz);
+    const unsigned q = in ? ((unsigned)i * (unsigned)gf.Py + (unsigned)j) * (unsigned)gf.Pz + (unsigned)k : 0u;
+    C v[4];
 #pragma unroll
-        for (int f = 0; f <= DIM; f++) sr[f][t] = Cvt<TS>::st(v[f]);
+    for (int f = 0; f <= DIM; f++) v[f] = Cvt<TS>::ld(at(b + f * gf.S, q));
+    xt.template load<T::NT, false, false>(gf, flf, x, gc, (const TS *)nullptr, 2 * I0 - 2, 2 * J0 - 2,
+                                          DIM == 3 ? 2 * K0 - 2 : 0);
+    __syncthreads();
+    if (t0 < T::N) {
+        const RrAcc<TS, DIM, X, MASK> a{xt, al, gf.S, (fi + 1) * X::SI + (fj + 1) * X::SJ + (DIM == 3 ? fk + 1 : 0), q};
+        const BoxSten<C, DIM, RrAcc<TS, DIM, X, MASK>> s{a};
+        v[0] -= s.cell();
+        v[1] -= s.template face<0>(0, 0, 0);
+        v[2] -= s.template face<1>(0, 0, 0);
+        if (DIM == 3) v[3] -= s.template face<2>(0, 0, 0);
+#pragma unroll
+        for (int f = 0; f <= DIM; f++) sr[f][t0] = Cvt<TS>::st(in ? v[f] : C(0));
     }
     __syncthreads();
     constexpr int NC = T::CI * T::CJ * T::CK;
@@ -723,12 +931,41 @@ void launch_box(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b, cons
         if (zero) ST_BOX(3, true, false);  // reads no x
         else if (inner) ST_BOX(3, false, false);
         else ST_BOX(3, false, true);
-    } else {
-        if (zero) ST_BOX(2, true, false);
-        else if (inner) ST_BOX(2, false, false);
-        else ST_BOX(2, false, true);
+    } else {  // a single pass in 2D: st_mg_smooth (a cycle's passes run in k_sweeps)
+        ST_BOX(2, false, true);
     }
 #undef ST_BOX
+}
+
+template <typename TS, int NPASS, bool ZERO, bool PROL>
+static void sweeps_go(const Lvl &g, const Lvl &gc, const uint8_t *fl, const TS *al, const TS *b, const TS *xin,
+                      const TS *ec, TS *xout, int col0, float omega, bool inner, hipStream_t s)
+{
+    typedef SwTile<NPASS> W;
+    const dim3 gr((unsigned)((g.ny + W::TJ - 1) / W::TJ), (unsigned)((g.nx + W::TI - 1) / W::TI)), bl(W::NT);
+    if (inner)
+        hipLaunchKernelGGL((k_sweeps<TS, NPASS, ZERO, PROL, false>), gr, bl, 0, s, g, gc, fl, al, b, xin, ec, xout, col0,
+                           omega);
+    else
+        hipLaunchKernelGGL((k_sweeps<TS, NPASS, ZERO, PROL, true>), gr, bl, 0, s, g, gc, fl, al, b, xin, ec, xout, col0,
+                           omega);
+}
+
+template <typename TS>
+void launch_sweeps(const Lvl &g, const Lvl &gc, const uint8_t *fl, const TS *al, const TS *b, const TS *xin, const TS *ec,
+                   TS *xout, int nsweep, int col0, float omega, bool zero, bool inner, hipStream_t s)
+{
+#define ST_SW(NP, Z, P) sweeps_go<TS, NP, Z, P>(g, gc, fl, al, b, xin, ec, xout, col0, omega, inner, s)
+    if (nsweep == 1) {
+        if (zero) ST_SW(2, true, false);
+        else if (ec) ST_SW(2, false, true);
+        else ST_SW(2, false, false);
+    } else {
+        if (zero) ST_SW(4, true, false);
+        else if (ec) ST_SW(4, false, true);
+        else ST_SW(4, false, false);
+    }
+#undef ST_SW
 }
 
 template <typename TS>
@@ -799,6 +1036,8 @@ void launch_vcycle_tail(const TailArgs<TS> &a, int dim, int n, const TS *b0, TS 
                                 bool, hipStream_t);                                                                     \
     template void launch_resid_restrict<T>(const Lvl &, const Lvl &, const uint8_t *, const T *, const T *,       \
                                            const T *, const uint8_t *, T *, bool, hipStream_t);                   \
+    template void launch_sweeps<T>(const Lvl &, const Lvl &, const uint8_t *, const T *, const T *, const T *, const T *, \
+                                   T *, int, int, float, bool, bool, hipStream_t);                                \
     template void launch_node_apply<T>(const Lvl &, const uint8_t *, const T *, const T *, T *, hipStream_t);      \
     template void launch_node_residual<T>(const Lvl &, const uint8_t *, const T *, const T *, const T *, T *,     \
                                           double *, hipStream_t);                                                 \

@@ -31,6 +31,12 @@ void launch_vcycle_tail(const TailArgs<TS> &a, int dim, int n, const TS *b0, TS 
 template <typename TS>
 void launch_box(const Lvl &, const uint8_t *, const TS *al, const TS *b, const TS *xin, TS *xout, int color,
                 float omega, bool zero, bool inner, hipStream_t);
+// nsweep (1 to ST_SWEEPS) whole sweeps (first colour col0, then the other) of a 2D level in
+// one launch, xin -> xout; zero: from x = 0; ec: from xin + P ec
+constexpr int ST_SWEEPS = 2;
+template <typename TS>
+void launch_sweeps(const Lvl &, const Lvl &gc, const uint8_t *, const TS *al, const TS *b, const TS *xin, const TS *ec,
+                   TS *xout, int nsweep, int col0, float omega, bool zero, bool inner, hipStream_t);
 // y = A x and r = b - A x (partials of |r|^2 per 256 nodes) of such a level
 template <typename TS>
 void launch_node_apply(const Lvl &, const uint8_t *, const TS *al, const TS *x, TS *y, hipStream_t);

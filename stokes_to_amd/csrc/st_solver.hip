@@ -343,32 +343,72 @@ template <typename TS> static TailArgs<TS> tail_args(st_ctx *c, int l0)
     return a;
 }
 
+// The sweeps of a 2D level run up to ST_SWEEPS to a launch, each launch from one buffer to
+// the other (x and t).  Whether the cycle's first launch writes x, so that its last does:
+static bool first_writes_x(const st_ctx *c)
+{
+    auto launches = [](int nu) { return (nu + ST_SWEEPS - 1) / ST_SWEEPS; };
+    return (launches(c->prm.nu_pre) + launches(c->prm.nu_post)) % 2 == 1;
+}
+// nu sweeps of the 2D level l from cur (zero: from 0; ec: from cur + P ec); cur ends at the result
+template <typename TS>
+static void fused_sweeps(st_ctx *c, int l, const TS *b, TS *x, TS *&cur, int nu, int first, bool zero, const TS *ec)
+{
+    Hier<TS> &h = hier<TS>(c);
+    const Lvl &g = c->lv[l];
+    for (int done = 0; done < nu;) {
+        const int ns = std::min(nu - done, ST_SWEEPS);
+        TS *to = (cur == x) ? h.t[l] : x;
+        if (l == 0) prof_mark(c, ST_PROF_SWEEP);
+        launch_sweeps<TS>(g, c->lv[l + 1], c->fl[l], h.al[l], b, cur, done ? (const TS *)nullptr : ec, to, ns, first,
+                          (float)c->prm.omega, zero && done == 0, l > 0, c->s);
+        if (l == 0) prof_mark(c, ST_PROF_SWEEP);
+        cur = to;
+        done += ns;
+    }
+}
+
 template <typename TS> static void vcycle(st_ctx *c, const TS *b0, TS *x0)
 {
     Hier<TS> &h = hier<TS>(c);
     const int lt = tail_level(c);
+    const int nu_pre = c->prm.nu_pre, nu_post = c->prm.nu_post;
+    TS *cur[ST_MAX_LEVELS];  // where a level's x is after its way down
     for (int l = 0; l < lt; l++) {
         const Lvl &g = c->lv[l];
         const TS *b = (l == 0) ? b0 : h.b[l];
         TS *x = (l == 0) ? x0 : h.x[l];
-        if (c->prm.nu_pre > 0) smooth<TS>(c, l, b, x, c->prm.nu_pre, 0, true);
-        else launch_fill<TS>((long)g.nfield * g.S, x, 0.0, c->s);
+        cur[l] = x;
+        if (c->dim == 2) {
+            cur[l] = first_writes_x(c) ? h.t[l] : x;  // the first launch writes the other
+            if (nu_pre > 0) fused_sweeps<TS>(c, l, b, x, cur[l], nu_pre, 0, true, nullptr);
+            else launch_fill<TS>((long)g.nfield * g.S, cur[l], 0.0, c->s);
+        } else if (nu_pre > 0) {
+            smooth<TS>(c, l, b, x, nu_pre, 0, true);
+        } else {
+            launch_fill<TS>((long)g.nfield * g.S, x, 0.0, c->s);
+        }
         if (l == 0) prof_mark(c, ST_PROF_RESIDUAL);
         if (march_ok(g)) {
             launch_residual<TS>(g, c->fl[l], h.al[l], b, x, h.r[l], nullptr, c->s);
             if (l == 0) prof_mark(c, ST_PROF_RESIDUAL);
             launch_restrict<TS>(g, c->lv[l + 1], c->fl[l + 1], h.r[l], h.b[l + 1], c->s);
         } else {
-            launch_resid_restrict<TS>(g, c->lv[l + 1], c->fl[l], h.al[l], b, x, c->fl[l + 1], h.b[l + 1], l > 0, c->s);
+            launch_resid_restrict<TS>(g, c->lv[l + 1], c->fl[l], h.al[l], b, cur[l], c->fl[l + 1], h.b[l + 1], l > 0, c->s);
             if (l == 0) prof_mark(c, ST_PROF_RESIDUAL);
         }
     }
-    launch_vcycle_tail<TS>(tail_args<TS>(c, lt), c->dim, c->lv[lt].nx, lt == 0 ? b0 : h.b[lt], lt == 0 ? x0 : h.x[lt], lt > 0, c->s);
+    launch_vcycle_tail<TS>(tail_args<TS>(c, lt), c->dim, c->lv[lt].nx, lt == 0 ? b0 : h.b[lt], lt == 0 ? x0 : h.x[lt],
+                           lt > 0, c->s);
     for (int l = lt - 1; l >= 0; l--) {
         const TS *b = (l == 0) ? b0 : h.b[l];
         TS *x = (l == 0) ? x0 : h.x[l];
-        launch_prolong<TS>(c->lv[l], c->lv[l + 1], c->fl[l], h.x[l + 1], x, c->s);
-        if (c->prm.nu_post > 0) smooth<TS>(c, l, b, x, c->prm.nu_post, 1, false);
+        if (c->dim == 2 && nu_post > 0) {
+            fused_sweeps<TS>(c, l, b, x, cur[l], nu_post, 1, false, h.x[l + 1]);
+        } else {  // without sweeps after it, a 2D level's x is in place too (first_writes_x)
+            launch_prolong<TS>(c->lv[l], c->lv[l + 1], c->fl[l], h.x[l + 1], x, c->s);
+            if (nu_post > 0) smooth<TS>(c, l, b, x, nu_post, 1, false);
+        }
     }
 }
 
