@@ -20,126 +20,13 @@
 
 namespace st {
 
-namespace {
-
-// value at a 32-bit element offset from a uniform base
-template <typename T> __device__ __forceinline__ T at(const T *p, unsigned i)
-{
-    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + i * (unsigned)sizeof(T));
-}
-template <typename T> __device__ __forceinline__ void put(T *p, unsigned i, T v)
-{
-    *reinterpret_cast<T *>(reinterpret_cast<char *>(p) + i * (unsigned)sizeof(T)) = v;
-}
-
-// accessor of a cell (i, j, k all below the level's side) in the node layout: at most
-// one offset is negative; below the grid it reads the own node and F, p are 0; the
-// only node past the box that a cell's rows name is i + 2 (in the last cell plane)
-template <typename TS, int DIM, bool M> struct CellAcc {
-    typedef typename Cvt<TS>::C C;
-    static constexpr bool MASK = M;
-    const uint8_t *fl;
-    const TS *x, *b, *al;
-    long S, sI, sJ;
-    unsigned q, qi, qj, qk;  // own node; the node below along each axis (own at the edge)
-    bool li, lj, lk, hi;     // first cell along an axis, last along i
-
-    __device__ __forceinline__ CellAcc(const Lvl &g, const uint8_t *f, const TS *a, const TS *bb, const TS *xx, int i,
-                                       int j, int k)
-        : fl(f), x(xx), b(bb), al(a), S(g.S), sI((long)g.Py * g.Pz), sJ(g.Pz)
-    {
-        q = ((unsigned)i * (unsigned)g.Py + (unsigned)j) * (unsigned)g.Pz + (unsigned)k;
-        li = i == 0;
-        lj = j == 0;
-        lk = k == 0;
-        hi = i == g.nx - 1;
-        qi = li ? q : q - (unsigned)sI;
-        qj = lj ? q : q - (unsigned)sJ;
-        qk = lk ? q : q - 1u;
-    }
-    // lane part and uniform part of the offset of a neighbour
-    __device__ __forceinline__ unsigned lane(int di, int dj, int dk) const
-    { return di < 0 ? qi : (dj < 0 ? qj : (dk < 0 ? qk : q)); }
-    __device__ __forceinline__ long uni(int di, int dj, int dk) const
-    { return (di > 0 ? di * sI : 0) + (dj > 0 ? dj * sJ : 0) + (dk > 0 ? dk : 0); }
-    __device__ __forceinline__ bool out(int di, int dj, int dk) const
-    { return (di < 0 && li) || (dj < 0 && lj) || (dk < 0 && lk) || (di > 1 && hi); }
-
-    __device__ __forceinline__ int F(int di, int dj, int dk) const
-    {
-        if (di > 1) {  // one plane short of i + 2 in the last cell plane, and discarded
-            const int f = at(fl + sI, hi ? q : q + (unsigned)sI);
-            return hi ? 0 : f;
-        }
-        const int f = at(fl + uni(di, dj, dk), lane(di, dj, dk));
-        return out(di, dj, dk) ? 0 : f;
-    }
-    __device__ __forceinline__ C X(int f, int di, int dj, int dk) const
-    {
-        // i + 2 of u_x in the last cell plane lies in u_y's first plane: in bounds, and it
-        // enters only the divergence of the cell i + 1, whose flag is 0 there
-        const C v = Cvt<TS>::ld(at(x + f * S + uni(di, dj, dk), lane(di, dj, dk)));
-        return ((f == 0 || !MASK) && out(di, dj, dk)) ? C(0) : v;
-    }
-    __device__ __forceinline__ C B(int f, int di, int dj, int dk) const
-    { return Cvt<TS>::ld(at(b + f * S + uni(di, dj, dk), q)); }
-    __device__ __forceinline__ C AL(int d, int di, int dj, int dk) const
-    { return Cvt<TS>::ld(at(al + d * S + uni(di, dj, dk), q)); }
-};
-
-// accessor of any node of the box: offsets in -1..1 per axis, 0 outside the box
-template <typename TS, int DIM, bool M> struct NodeAcc {
-    typedef typename Cvt<TS>::C C;
-    static constexpr bool MASK = M;
-    const uint8_t *fl;
-    const TS *x, *al;
-    long S;
-    unsigned q, im, ip, jm, jp, km, kp;  // steps to the neighbours (0 at the edge)
-    bool li, lj, lk, hi, hj, hk;
-
-    __device__ __forceinline__ NodeAcc(const Lvl &g, const uint8_t *f, const TS *a, const TS *xx, int i, int j, int k)
-        : fl(f), x(xx), al(a), S(g.S)
-    {
-        const unsigned sI = (unsigned)g.Py * (unsigned)g.Pz, sJ = (unsigned)g.Pz;
-        q = (unsigned)i * sI + (unsigned)j * sJ + (unsigned)k;
-        li = i == 0; lj = j == 0; lk = k == 0;
-        hi = i == g.nx; hj = j == g.ny; hk = (DIM == 2) || k >= g.nz;
-        im = li ? 0u : sI; ip = hi ? 0u : sI;
-        jm = lj ? 0u : sJ; jp = hj ? 0u : sJ;
-        km = lk ? 0u : 1u; kp = hk ? 0u : 1u;
-    }
-    __device__ __forceinline__ unsigned node(int di, int dj, int dk) const
-    {
-        return q + (di > 0 ? ip : 0u) + (dj > 0 ? jp : 0u) + (dk > 0 ? kp : 0u) - (di < 0 ? im : 0u) -
-               (dj < 0 ? jm : 0u) - (dk < 0 ? km : 0u);
-    }
-    __device__ __forceinline__ bool out(int di, int dj, int dk) const
-    {
-        return (di < 0 && li) || (dj < 0 && lj) || (dk < 0 && lk) || (di > 0 && hi) || (dj > 0 && hj) || (dk > 0 && hk);
-    }
-    __device__ __forceinline__ int F(int di, int dj, int dk) const
-    {
-        const int f = at(fl, node(di, dj, dk));
-        return out(di, dj, dk) ? 0 : f;
-    }
-    __device__ __forceinline__ C X(int f, int di, int dj, int dk) const
-    {
-        const C v = Cvt<TS>::ld(at(x + f * S, node(di, dj, dk)));
-        return ((f == 0 || !MASK) && out(di, dj, dk)) ? C(0) : v;
-    }
-    __device__ __forceinline__ C AL(int d, int di, int dj, int dk) const
-    { return Cvt<TS>::ld(at(al + d * S, node(di, dj, dk))); }
-};
-
-}  // namespace
-
 // ------------------------------------------------------------ colour pass
 
 // One colour of the smoother, xin -> xout, one lane per pair of cells along the fastest
 // axis: the lane solves the block of the pair's colour cell and copies what the colour
 // does not own (the other cell's p, and its faces on the domain boundary).  lg: log2 of
 // the level side.  ZERO: xin is zero and not read.
-template <typename TS, int DIM, bool ZERO, bool MASK>
+template <typename TS, int DIM, bool ZERO, bool MASK, bool FINE>
 __global__ void __launch_bounds__(256) k_box(Lvl g, int lg, const uint8_t *__restrict__ fl, const TS *__restrict__ al,
                                              const TS *__restrict__ b, const TS *__restrict__ xin,
                                              TS *__restrict__ xout, int color, float omega)
@@ -163,7 +50,7 @@ __global__ void __launch_bounds__(256) k_box(Lvl g, int lg, const uint8_t *__res
     }
     const CellAcc<TS, DIM, MASK> a(g, fl, al, b, xin, i, j, k);
     C pn, u0[3], u1[3];
-    box_cell<C, DIM, ZERO>(a, omega, pn, u0, u1);
+    box_cell<C, DIM, ZERO, FINE>(a, omega, pn, u0, u1);
     const long st[3] = {a.sI, a.sJ, 1};
     // copy-through first (its loads are independent of the solve)
     const unsigned qo = a.q + (DIM == 3 ? (unsigned)(ok - k) : (unsigned)(oj - j));
@@ -919,20 +806,22 @@ static int lg2(int n) { return __builtin_ctz((unsigned)n); }
 
 template <typename TS>
 void launch_box(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b, const TS *xin, TS *xout, int color,
-                float omega, bool zero, bool inner, hipStream_t s)
+                float omega, bool zero, bool inner, bool fine, hipStream_t s)
 {
     const int lg = lg2(g.nx);
     const unsigned np = 1u << (g.dim * lg - 1);
     // one wave per workgroup on the smallest levels, so that every wave has a CU
     const unsigned bs = np <= (1u << 16) ? 64 : 256;
     const dim3 gr((np + bs - 1) / bs), bl(bs);
-#define ST_BOX(D, Z, M) hipLaunchKernelGGL((k_box<TS, D, Z, M>), gr, bl, 0, s, g, lg, fl, al, b, xin, xout, color, omega)
+#define ST_BOX(D, Z, M, F) \
+    hipLaunchKernelGGL((k_box<TS, D, Z, M, F>), gr, bl, 0, s, g, lg, fl, al, b, xin, xout, color, omega)
     if (g.dim == 3) {
-        if (zero) ST_BOX(3, true, false);  // reads no x
-        else if (inner) ST_BOX(3, false, false);
-        else ST_BOX(3, false, true);
+        if (zero) ST_BOX(3, true, false, false);  // reads no x
+        else if (fine) ST_BOX(3, false, true, true);
+        else if (inner) ST_BOX(3, false, false, false);
+        else ST_BOX(3, false, true, false);
     } else {  // a single pass in 2D: st_mg_smooth (a cycle's passes run in k_sweeps)
-        ST_BOX(2, false, true);
+        ST_BOX(2, false, true, false);
     }
 #undef ST_BOX
 }
@@ -1033,7 +922,7 @@ void launch_vcycle_tail(const TailArgs<TS> &a, int dim, int n, const TS *b0, TS 
 
 #define INST_C(T)                                                                                                  \
     template void launch_box<T>(const Lvl &, const uint8_t *, const T *, const T *, const T *, T *, int, float, bool, \
-                                bool, hipStream_t);                                                                     \
+                                bool, bool, hipStream_t);                                                                     \
     template void launch_resid_restrict<T>(const Lvl &, const Lvl &, const uint8_t *, const T *, const T *,       \
                                            const T *, const uint8_t *, T *, bool, hipStream_t);                   \
     template void launch_sweeps<T>(const Lvl &, const Lvl &, const uint8_t *, const T *, const T *, const T *, const T *, \

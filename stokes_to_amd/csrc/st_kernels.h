@@ -27,10 +27,11 @@ template <typename TS> struct TailArgs {
 // and solution
 template <typename TS>
 void launch_vcycle_tail(const TailArgs<TS> &a, int dim, int n, const TS *b0, TS *x0, bool inner, hipStream_t);
-// smoother colour pass of a level that is not marched, one lane per pair of cells
+// smoother colour pass, one lane per pair of cells; fine: with the arithmetic of
+// march_smooth, else with that of the levels that are not marched
 template <typename TS>
 void launch_box(const Lvl &, const uint8_t *, const TS *al, const TS *b, const TS *xin, TS *xout, int color,
-                float omega, bool zero, bool inner, hipStream_t);
+                float omega, bool zero, bool inner, bool fine, hipStream_t);
 // nsweep (1 to ST_SWEEPS) whole sweeps (first colour col0, then the other) of a 2D level in
 // one launch, xin -> xout; zero: from x = 0; ec: from xin + P ec
 constexpr int ST_SWEEPS = 2;
@@ -53,6 +54,10 @@ template <typename TS>
 void launch_residual(const Lvl &, const uint8_t *, const TS *, const TS *b, const TS *x, TS *r, double *part,
                      hipStream_t);
 unsigned residual_blocks(const Lvl &);
+// the FP64 residual and norm of the plain FP64 solve (plain_residual_blocks partials)
+void launch_plain_residual(const Lvl &, const uint8_t *, const double *, const double *b, const double *x, double *r,
+                           double *part, hipStream_t);
+unsigned plain_residual_blocks(const Lvl &);
 template <typename TS>
 void launch_smooth(const Lvl &, const uint8_t *, const TS *, const TS *b, const TS *xin, TS *xout, int color,
                    float omega, bool zero, bool inner, hipStream_t);
@@ -122,18 +127,21 @@ template <typename TS> void launch_fill(long n, TS *y, double v, hipStream_t);
 // 2.5D marching kernels (st_march.hip) for 3D levels with ny % 4 == 0, nz % 64 == 0
 bool march_ok(const Lvl &);
 unsigned march_blocks(const Lvl &);
-template <typename TS> void march_apply(const Lvl &, const uint8_t *, const TS *, const TS *, TS *, hipStream_t);
-template <typename TS>
-void march_residual(const Lvl &, const uint8_t *, const TS *, const TS *b, const TS *x, TS *r, double *part,
-                    hipStream_t);
+void march_residual(const Lvl &, const uint8_t *, const double *, const double *b, const double *x, double *r,
+                    double *part, hipStream_t);
 template <typename TS>
 void march_smooth(const Lvl &, const uint8_t *, const TS *, const TS *b, const TS *xin, TS *xout, int color,
                   float omega, hipStream_t);
 // FP64 residual r = b - A x stored in FP32 (+ FP64 partial sums of |r|^2)
 void march_residual_f32(const Lvl &, const uint8_t *, const double *al, const double *b, const double *x, float *r,
                         double *part, hipStream_t);
+// operator and residual of the same levels without LDS (st_fine.hip)
+template <typename TS> void fine_apply(const Lvl &, const uint8_t *, const TS *, const TS *, TS *, hipStream_t);
+template <typename TS>
+void fine_residual(const Lvl &, const uint8_t *, const TS *, const TS *b, const TS *x, TS *r, double *part, hipStream_t);
 // FP64 operator applied to an FP32-stored vector (x float, alpha and y double)
-void march_apply_mixed(const Lvl &, const uint8_t *, const double *al, const float *x, double *y, hipStream_t);
+void fine_apply_mixed(const Lvl &, const uint8_t *, const double *al, const float *x, double *y, hipStream_t);
+unsigned fine_blocks(const Lvl &);
 // one red-black sweep (colour col0, then the other) in one pass (st_sweep.hip);
 // FP32 arithmetic, TS = float or bf16 storage, levels with march_ok
 template <typename TS>

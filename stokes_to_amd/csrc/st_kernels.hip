@@ -6,6 +6,8 @@
 // CX/grid3D.cu:431-455, and are not).  Reductions are two-stage, fixed order.
 #include "st_kernels.h"
 
+#include <type_traits>
+
 namespace st {
 
 // ----------------------------------------------------------------- stencil
@@ -1088,24 +1090,49 @@ static inline unsigned nb_grid(long n)
 template <typename TS>
 void launch_apply(const Lvl &g, const uint8_t *fl, const TS *al, const TS *x, TS *y, hipStream_t s)
 {
-    if (march_ok(g)) march_apply<TS>(g, fl, al, x, y, s);
+    if (march_ok(g)) fine_apply<TS>(g, fl, al, x, y, s);
     else launch_node_apply<TS>(g, fl, al, x, y, s);
 }
 template <typename TS>
 void launch_residual(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b, const TS *x, TS *r, double *part,
                      hipStream_t s)
 {
-    if (march_ok(g)) march_residual<TS>(g, fl, al, b, x, r, part, s);
-    else launch_node_residual<TS>(g, fl, al, b, x, r, part, s);
+    if (march_ok(g)) {
+        // With its norm: the marching kernel, in FP64.  The mixed-precision paths start
+        // and stop their cycles on this norm, and a sequence of warm-started solves
+        // carries its rounding on: summed in another order, the objectives of a 64^3 FP32
+        // run differ by up to 6e-10 after three design steps.  It runs two or three times
+        // a solve.
+        if constexpr (std::is_same<TS, double>::value) {
+            if (part) {
+                march_residual(g, fl, al, b, x, r, part, s);
+                return;
+            }
+        }
+        fine_residual<TS>(g, fl, al, b, x, r, part, s);
+    } else {
+        launch_node_residual<TS>(g, fl, al, b, x, r, part, s);
+    }
 }
 unsigned residual_blocks(const Lvl &g) { return march_ok(g) ? march_blocks(g) : nb(g.S); }
+void launch_plain_residual(const Lvl &g, const uint8_t *fl, const double *al, const double *b, const double *x, double *r,
+                           double *part, hipStream_t s)
+{
+    if (march_ok(g)) fine_residual<double>(g, fl, al, b, x, r, part, s);
+    else launch_node_residual<double>(g, fl, al, b, x, r, part, s);
+}
+unsigned plain_residual_blocks(const Lvl &g) { return march_ok(g) ? fine_blocks(g) : nb(g.S); }
 
 template <typename TS>
 void launch_smooth(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b, const TS *xin, TS *xout, int color,
                    float omega, bool zero, bool inner, hipStream_t s)
 {
-    if (!zero && march_ok(g)) march_smooth<TS>(g, fl, al, b, xin, xout, color, omega, s);
-    else launch_box<TS>(g, fl, al, b, xin, xout, color, omega, zero, inner, s);
+    // The marching pass needs planes to march: with a lane per pair of cells instead a pass
+    // takes 10.7 / 9.6 us at 64^3 (FP64 / FP32; marched 29.7 / 24.8), 79 / 44 us at 128^3 (84 /
+    // 38.6) and 645 / 358 us at 256^3 (590 / 317)
+    const int box_max = std::is_same<TS, double>::value ? 128 : 64;
+    if (!zero && march_ok(g) && g.nx > box_max) march_smooth<TS>(g, fl, al, b, xin, xout, color, omega, s);
+    else launch_box<TS>(g, fl, al, b, xin, xout, color, omega, zero, inner, march_ok(g), s);
 }
 template <typename TS>
 void launch_restrict(const Lvl &gf, const Lvl &gc, const uint8_t *flc, const TS *rf, TS *bc, hipStream_t s)

@@ -11,7 +11,8 @@
 // The k direction (contiguous in memory) maps to the 64 lanes of a wave, so all
 // global loads and stores are coalesced.
 //
-// Modes: APPLY y = A x;  RESID r = b - A x (+ FP64 partial sums of r^2);
+// Modes: RESID r = b - A x with FP64 partial sums of r^2 (FP64; a residual without its
+//        norm and the operator itself are in st_fine.hip);
 //        SMOOTH one colour of the box-Vanka smoother (xin -> xout), with the
 //        7 local residuals of each colour cell read from the staged planes.
 #include "st_kernels.h"
@@ -20,7 +21,7 @@ namespace st {
 
 namespace {
 constexpr int BK = 64, LK = BK + 3;
-enum { M_APPLY = 0, M_RESID = 1, M_SMOOTH = 2 };
+enum { M_RESID = 1, M_SMOOTH = 2 };
 
 __device__ __forceinline__ int slot3(int s) { return (s + 3) % 3; }
 __device__ __forceinline__ int slot2(int s) { return s & 1; }
@@ -62,18 +63,16 @@ __device__ __forceinline__ void gst(T *p, typename Ix<O32>::T i, T v)
         p[i] = v;
 }
 
-// TS: storage of alpha and b (and the compute type through Cvt<TS>::C); TX: storage
-// of x (a lower-precision x is widened on load: the FP64 operator on an FP32 vector);
-// BJ: tile rows; TY: storage of y (an FP64 residual stored in FP32); O32: 32-bit
-// offsets.
+// TS: storage of alpha, b and x (and the compute type through Cvt<TS>::C); BJ: tile
+// rows; TY: storage of y (an FP64 residual stored in FP32); O32: 32-bit offsets.
 //
 // SMOOTH: half of the workgroup's waves (BJ x 32 lanes) take the BJ x 32 cells of the
 // colour in the tile's plane, one per lane, the other half the other cells
 // (copy-through of p and of the domain-boundary faces).  A lane per colour cell, not
 // per node, so no wave runs the block solve with half of its lanes idle.
-template <typename TS, int MODE, typename TX = TS, int BJ = 4, typename TY = TS, bool O32 = false>
+template <typename TS, int MODE, int BJ = 4, typename TY = TS, bool O32 = false>
 __global__ void __launch_bounds__(BJ * 64) k_march(Lvl g, const uint8_t *__restrict__ fl, const TS *__restrict__ al,
-                                                   const TS *__restrict__ b, const TX *__restrict__ x,
+                                                   const TS *__restrict__ b, const TS *__restrict__ x,
                                                    TY *__restrict__ y, double *part, int chunk, int color,
                                                    float omega)
 {
@@ -109,21 +108,16 @@ __global__ void __launch_bounds__(BJ * 64) k_march(Lvl g, const uint8_t *__restr
     const int cown = (tj + 1) * LK + (tk + 1);
     // field base pointers (uniform)
     const long S = g.S;
-    const TX *xf[4] = {x, x + S, x + 2 * S, x + 3 * S};
+    const TS *xf[4] = {x, x + S, x + 2 * S, x + 3 * S};
     const TS *af[3] = {al, al + S, al + 2 * S};
-    const TS *bf[4] = {b, b, b, b};
-    if (MODE != M_APPLY) {
-        bf[1] = b + S;
-        bf[2] = b + 2 * S;
-        bf[3] = b + 3 * S;
-    }
+    const TS *bf[4] = {b, b + S, b + 2 * S, b + 3 * S};
     TY *yf[4] = {y, y, y, y};  // y is null for a residual norm without the residual
     if (y) {
         yf[1] = y + S;
         yf[2] = y + 2 * S;
         yf[3] = y + 3 * S;
     }
-    auto ldx = [&](int f, I q) -> C { return (C)Cvt<TX>::ld(gld<O32>(xf[f], q)); };
+    auto ldx = [&](int f, I q) -> C { return (C)Cvt<TS>::ld(gld<O32>(xf[f], q)); };
     auto lda = [&](int f, I q) -> C { return (C)Cvt<TS>::ld(gld<O32>(af[f], q)); };
     auto ldb = [&](int f, I q) -> C { return (C)Cvt<TS>::ld(gld<O32>(bf[f], q)); };
     auto sty = [&](int f, I q, C v) { gst<O32>(yf[f], q, Cvt<TY>::st((CY)v)); };
@@ -207,7 +201,7 @@ __global__ void __launch_bounds__(BJ * 64) k_march(Lvl g, const uint8_t *__restr
     gdiv(ic0);
     // g, p and flags of the plane below (i - 1) at a column: the low x face's row
     // needs them, and their slots are reused before the plane is processed.  Kept for
-    // the own column (APPLY, RESID) or for both columns of the lane's pair (SMOOTH).
+    // the own column (RESID) or for both columns of the lane's pair (SMOOTH).
     auto below = [&](int c, C &gv, C &pv, int &fv) {
         const int a = slot3(ic0 - 1), bq = slot3(ic0);
         const C dv = sW[bq][0][c] - sW[a][0][c] + sW[a][1][c + LK] - sW[a][1][c] + sW[a][2][c + 1] - sW[a][2][c];
@@ -236,10 +230,8 @@ __global__ void __launch_bounds__(BJ * 64) k_march(Lvl g, const uint8_t *__restr
         const int so = slot3(i), sn = slot3(i + 1);
         const int fo = sF[so][c];
         auto raw = [&](int fixed, int f, I qq) -> C { return fixed ? ldx(f, qq) : C(0); };
-        if (MODE != M_APPLY) {
 #pragma unroll
-            for (int f = 0; f < 4; f++) pb[f] = ldb(f, q);
-        }
+        for (int f = 0; f < 4; f++) pb[f] = ldb(f, q);
 #pragma unroll
         for (int f = 0; f < 3; f++) pa[f] = lda(f, q);
         if (SM) {  // a cell: i < nx, j < ny, k < nz, so the high faces exist
@@ -306,14 +298,12 @@ __global__ void __launch_bounds__(BJ * 64) k_march(Lvl g, const uint8_t *__restr
         if (!SM) {
             auto emit = [&](int c, I qq, C gim1, C pim1, const C *bb, const C *xr, const C *av) {
                 C v0 = yp(c), v1 = yx(c, gim1, pim1, xr[0], av[0]), v2 = yy(c, xr[1], av[1]), v3 = yz(c, xr[2], av[2]);
-                if (MODE == M_RESID) {
-                    v0 = bb[0] - v0;
-                    v1 = bb[1] - v1;
-                    v2 = bb[2] - v2;
-                    v3 = bb[3] - v3;
-                    acc += (double)v0 * v0 + (double)v1 * v1 + (double)v2 * v2 + (double)v3 * v3;
-                }
-                if (MODE != M_RESID || y) {  // a residual without y: its norm only
+                v0 = bb[0] - v0;
+                v1 = bb[1] - v1;
+                v2 = bb[2] - v2;
+                v3 = bb[3] - v3;
+                acc += (double)v0 * v0 + (double)v1 * v1 + (double)v2 * v2 + (double)v3 * v3;
+                if (y) {  // without y: the norm only
                     sty(0, qq, v0);
                     sty(1, qq, v1);
                     sty(2, qq, v2);
@@ -326,7 +316,7 @@ __global__ void __launch_bounds__(BJ * 64) k_march(Lvl g, const uint8_t *__restr
             auto emit_edge = [&](int c, I qq) {
                 C bb[4], xr[3], av[3];
 #pragma unroll
-                for (int f = 0; f < 4; f++) bb[f] = (MODE == M_RESID) ? ldb(f, qq) : C(0);
+                for (int f = 0; f < 4; f++) bb[f] = ldb(f, qq);
 #pragma unroll
                 for (int f = 0; f < 3; f++) {
                     xr[f] = ldx(f + 1, qq);
@@ -480,36 +470,31 @@ unsigned march_blocks(const Lvl &g)
 // used is a high face one plane up: S + sI nodes, at most 8 bytes each)
 static bool off32(const Lvl &g) { return (unsigned long)(g.S + (long)g.Py * g.Pz) * 8UL < (1UL << 32); }
 
-template <typename TS, int MODE, typename TX, typename TY>
-static void launch_march(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b, const TX *x, TY *y, double *part,
+template <typename TS, int MODE, typename TY>
+static void launch_march(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b, const TS *x, TY *y, double *part,
                          int color, float omega, hipStream_t s)
 {
     int ch;
     dim3 grid = march_grid(g, 4, 2048, ch);
     if (off32(g))
-        hipLaunchKernelGGL((k_march<TS, MODE, TX, 4, TY, true>), grid, dim3(256), 0, s, g, fl, al, b, x, y, part, ch,
-                           color, omega);
+        hipLaunchKernelGGL((k_march<TS, MODE, 4, TY, true>), grid, dim3(256), 0, s, g, fl, al, b, x, y, part, ch, color,
+                           omega);
     else
-        hipLaunchKernelGGL((k_march<TS, MODE, TX, 4, TY, false>), grid, dim3(256), 0, s, g, fl, al, b, x, y, part, ch,
-                           color, omega);
+        hipLaunchKernelGGL((k_march<TS, MODE, 4, TY, false>), grid, dim3(256), 0, s, g, fl, al, b, x, y, part, ch, color,
+                           omega);
 }
 
-template <typename TS>
-void march_apply(const Lvl &g, const uint8_t *fl, const TS *al, const TS *x, TS *y, hipStream_t s)
-{
-    launch_march<TS, M_APPLY>(g, fl, al, (const TS *)nullptr, x, y, (double *)nullptr, 0, 0.f, s);
-}
-template <typename TS>
-void march_residual(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b, const TS *x, TS *r, double *part,
-                    hipStream_t s)
-{
-    launch_march<TS, M_RESID>(g, fl, al, b, x, r, part, 0, 0.f, s);
-}
 template <typename TS>
 void march_smooth(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b, const TS *xin, TS *xout, int color,
                   float omega, hipStream_t s)
 {
     launch_march<TS, M_SMOOTH>(g, fl, al, b, xin, xout, (double *)nullptr, color, omega, s);
+}
+
+void march_residual(const Lvl &g, const uint8_t *fl, const double *al, const double *b, const double *x, double *r,
+                    double *part, hipStream_t s)
+{
+    launch_march<double, M_RESID>(g, fl, al, b, x, r, part, 0, 0.f, s);
 }
 
 void march_residual_f32(const Lvl &g, const uint8_t *fl, const double *al, const double *b, const double *x, float *r,
@@ -518,15 +503,7 @@ void march_residual_f32(const Lvl &g, const uint8_t *fl, const double *al, const
     launch_march<double, M_RESID>(g, fl, al, b, x, r, part, 0, 0.f, s);
 }
 
-void march_apply_mixed(const Lvl &g, const uint8_t *fl, const double *al, const float *x, double *y, hipStream_t s)
-{
-    launch_march<double, M_APPLY>(g, fl, al, (const double *)nullptr, x, y, (double *)nullptr, 0, 0.f, s);
-}
-
 #define INST_M(T)                                                                                              \
-    template void march_apply<T>(const Lvl &, const uint8_t *, const T *, const T *, T *, hipStream_t);       \
-    template void march_residual<T>(const Lvl &, const uint8_t *, const T *, const T *, const T *, T *,       \
-                                    double *, hipStream_t);                                                   \
     template void march_smooth<T>(const Lvl &, const uint8_t *, const T *, const T *, const T *, T *, int,    \
                                   float, hipStream_t);
 INST_M(double)

@@ -173,6 +173,19 @@ template <typename T> static int dalloc(st_ctx *c, T **p, long n)
     return ST_OK;
 }
 
+// n values in the node layout of level g, with a zero plane before them and two planes of
+// room after them: the kernels of the finest levels read a plane around the level
+// without a test (st_fine.hip).  The plane is rounded up so that the values keep the
+// allocation's alignment.
+template <typename T> static int dvec(st_ctx *c, T **p, long n, const Lvl &g)
+{
+    const long lead = ((long)g.Py * g.Pz + 63) / 64 * 64;
+    T *q = nullptr;
+    CKR(dalloc(c, &q, n + 3 * lead));
+    *p = q + lead;
+    return ST_OK;
+}
+
 static long abi_dofs(int dim, int n)
 {
     if (dim == 3) return (long)n * n * n + 3L * (n + 1) * n * n;
@@ -216,11 +229,11 @@ template <typename TS> static int alloc_hier(st_ctx *c, bool level0_vectors)
         long nv = (long)g.nfield * g.S;
         if (l > 0 || !std::is_same<TS, double>::value) CKR(dalloc(c, &h.al[l], (long)g.dim * g.S));
         if (l > 0 || level0_vectors) {
-            CKR(dalloc(c, &h.b[l], nv));
-            CKR(dalloc(c, &h.x[l], nv));
+            CKR(dvec(c, &h.b[l], nv, g));
+            CKR(dvec(c, &h.x[l], nv, g));
         }
-        CKR(dalloc(c, &h.t[l], nv));
-        CKR(dalloc(c, &h.r[l], nv));
+        CKR(dvec(c, &h.t[l], nv, g));
+        CKR(dvec(c, &h.r[l], nv, g));
     }
     return ST_OK;
 }
@@ -443,7 +456,7 @@ static void apply64(st_ctx *c, const float *z, double *w)
 {
     const Lvl &g = c->lv[0];
     if (march_ok(g)) {
-        march_apply_mixed(g, c->fl[0], c->h64.al[0], z, w, c->s);
+        fine_apply_mixed(g, c->fl[0], c->h64.al[0], z, w, c->s);
     } else {
         launch_axpby<float, double>(c->nvec, 1.0, z, 0.0, c->h64.t[0], c->s);
         launch_apply<double>(g, c->fl[0], c->h64.al[0], c->h64.t[0], w, c->s);
@@ -499,7 +512,8 @@ template <typename TV, typename TW> static int fgmres(st_ctx *c, const double *b
     std::vector<double> sig(m + 1, 1.0), sig2(m + 1, 1.0);
     int it = 0;
     double rr = 0.0, rr0 = -1.0;
-    const int rb = (int)residual_blocks(g);
+    const bool plain = std::is_same<TV, double>::value;
+    const int rb = (int)(plain ? plain_residual_blocks(g) : residual_blocks(g));
     for (;;) {
         double *r0 = std::is_same<TV, double>::value ? c->V : c->Wv;  // FP64 residual
         // FP32 path on a tiled level: the FP64 residual goes straight into u_0 in FP32
@@ -509,6 +523,7 @@ template <typename TV, typename TW> static int fgmres(st_ctx *c, const double *b
             beta = c->r0_beta;
         } else {
             if (r_f32) march_residual_f32(g, c->fl[0], c->h64.al[0], b, x, reinterpret_cast<float *>(Vb), c->part, c->s);
+            else if (plain) launch_plain_residual(g, c->fl[0], c->h64.al[0], b, x, r0, c->part, c->s);
             else launch_residual<double>(g, c->fl[0], c->h64.al[0], b, x, r0, c->part, c->s);
             launch_sum(rb, 1, c->part, c->red, c->s);
             double r2 = 0.0;
@@ -710,7 +725,7 @@ int st_create(st_ctx **out, const st_params *p)
     }
     int rc = ST_OK;
     c->fl.assign(c->L, nullptr);
-    for (int l = 0; l < c->L && rc == ST_OK; l++) rc = dalloc(c, &c->fl[l], c->lv[l].S);
+    for (int l = 0; l < c->L && rc == ST_OK; l++) rc = dvec(c, &c->fl[l], c->lv[l].S, c->lv[l]);
     const Lvl &g0 = c->lv[0];
     c->nvec = (long)g0.nfield * g0.S;
     c->ndof = abi_dofs(c->dim, n);
@@ -725,28 +740,28 @@ int st_create(st_ctx **out, const st_params *p)
     }
     if (rc == ST_OK && p->precision == ST_FP32) rc = alloc_hier<float>(c, false);
     if (rc == ST_OK && p->precision == ST_BF16) rc = alloc_hier<bf16>(c, true);
-    if (rc == ST_OK) rc = dalloc(c, &c->X, c->nvec);
-    if (rc == ST_OK) rc = dalloc(c, &c->B, c->nvec);
-    if (rc == ST_OK) rc = dalloc(c, &c->XD, c->nvec);
-    if (rc == ST_OK) rc = dalloc(c, &c->BODY, c->nvec);
-    if (rc == ST_OK) rc = dalloc(c, &c->LAM, c->nvec);
-    if (rc == ST_OK) rc = dalloc(c, &c->BA, c->nvec);
-    if (rc == ST_OK) rc = dalloc(c, &c->ZERO, c->nvec);
-    if (rc == ST_OK) rc = dalloc(c, &c->Wv, c->nvec);
-    if (rc == ST_OK) rc = dalloc(c, &c->V, c->nvec * (mr + 1));
-    if (rc == ST_OK) rc = dalloc(c, &c->Zb, c->nvec * mr);
+    if (rc == ST_OK) rc = dvec(c, &c->X, c->nvec, g0);
+    if (rc == ST_OK) rc = dvec(c, &c->B, c->nvec, g0);
+    if (rc == ST_OK) rc = dvec(c, &c->XD, c->nvec, g0);
+    if (rc == ST_OK) rc = dvec(c, &c->BODY, c->nvec, g0);
+    if (rc == ST_OK) rc = dvec(c, &c->LAM, c->nvec, g0);
+    if (rc == ST_OK) rc = dvec(c, &c->BA, c->nvec, g0);
+    if (rc == ST_OK) rc = dvec(c, &c->ZERO, c->nvec, g0);
+    if (rc == ST_OK) rc = dvec(c, &c->Wv, c->nvec, g0);
+    if (rc == ST_OK) rc = dvec(c, &c->V, c->nvec * (mr + 1), g0);
+    if (rc == ST_OK) rc = dvec(c, &c->Zb, c->nvec * mr, g0);
     // the held solutions of the warm starts (and the FP32 differences of the
     // minimal-residual start) with the context's other vectors, not during a run
     if (p->warm_order > 0)
         for (double **pp : {&c->XH[0], &c->XH[1], &c->LH[0], &c->LH[1]})
-            if (rc == ST_OK) rc = dalloc(c, pp, c->nvec);
+            if (rc == ST_OK) rc = dvec(c, pp, c->nvec, g0);
     if (p->warm_order == 3 && p->precision == ST_FP32 && march_ok(c->lv[0]))
         for (float **pp : {&c->DX[0], &c->DX[1], &c->DX[2], &c->DL[0], &c->DL[1], &c->DL[2]}) {
-            double *t = nullptr;
-            if (rc == ST_OK) rc = dalloc(c, &t, (c->nvec + 1) / 2);
-            *pp = reinterpret_cast<float *>(t);
+            if (rc == ST_OK) rc = dvec(c, pp, c->nvec, g0);
         }
-    c->npart = 8192 * 33;
+    // partial sums: 33 vectors of the Krylov kernels' blocks, or one per block of a residual
+    // or of the objective (more than that from 512^3 and 2D 16384^2)
+    c->npart = std::max(8192 * 33, (int)std::max(std::max(residual_blocks(g0), plain_residual_blocks(g0)), energy_blocks(g0)));
     if (rc == ST_OK) rc = dalloc(c, &c->part, c->npart);
     if (rc == ST_OK) rc = dalloc(c, &c->red, 64);
     if (rc == ST_OK) rc = dalloc(c, &c->h_dev, 64);
@@ -1030,15 +1045,11 @@ static int warm_mr(st_ctx *c, const double *b, double **xp, double **h, int &nh,
     const long nv = c->nvec;
     const Lvl &g = c->lv[0];
     if (!h[0]) {
-        CKR(dalloc(c, &h[0], nv));
-        CKR(dalloc(c, &h[1], nv));
+        CKR(dvec(c, &h[0], nv, g));
+        CKR(dvec(c, &h[1], nv, g));
     }
     if (!dh[0])
-        for (int i = 0; i < 3; i++) {
-            double *t = nullptr;
-            CKR(dalloc(c, &t, (nv + 1) / 2));
-            dh[i] = reinterpret_cast<float *>(t);
-        }
+        for (int i = 0; i < 3; i++) CKR(dvec(c, &dh[i], nv, g));
     hipEvent_t a, e;
     CK(hipEventCreate(&a));
     CK(hipEventCreate(&e));
@@ -1070,7 +1081,7 @@ static int warm_mr(st_ctx *c, const double *b, double **xp, double **h, int &nh,
     bool take = false, updated = false;  // updated: u_0 holds r0, no longer r1
     if (nd >= 1 && std::isfinite(r1) && r1 > 0.0) {
         float *y = u0 + nv;  // basis slots 1..nd
-        for (int i = 0; i < nd; i++) march_apply<float>(g, c->fl[0], c->h32.al[0], dh[i], y + i * nv, c->s);
+        for (int i = 0; i < nd; i++) fine_apply<float>(g, c->fl[0], c->h32.al[0], dh[i], y + i * nv, c->s);
         const int nq = nd * (nd + 1) / 2 + nd;
         const int nbk = (int)mr_blocks(nv);
         launch_mr_gram(nd, nv, y, nv, u0, c->part, c->s);
@@ -1161,8 +1172,8 @@ static int warm_extrapolate(st_ctx *c, const double *b, double **xp, double **h,
     if (c->prm.warm_order == 3 && c->prm.precision == ST_FP32 && march_ok(c->lv[0]))
         return warm_mr(c, b, xp, h, nh, dh, ms);
     if (!h[0]) {
-        CKR(dalloc(c, &h[0], c->nvec));
-        CKR(dalloc(c, &h[1], c->nvec));
+        CKR(dvec(c, &h[0], c->nvec, c->lv[0]));
+        CKR(dvec(c, &h[1], c->nvec, c->lv[0]));
     }
     hipEvent_t a, e;
     CK(hipEventCreate(&a));

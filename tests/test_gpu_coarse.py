@@ -7,7 +7,7 @@ import pytest
 
 from conftest import rel
 from helpers import oracle_desc, setup, solver_for
-from stokes_to_amd.problems import reference_test0
+from stokes_to_amd.problems import _split, reference_test0
 
 pytestmark = pytest.mark.gpu
 
@@ -46,3 +46,25 @@ def test_closed_box_solves_reach_rtol(make_solver, dim, n):
     assert st["converged"]
     b = np.where(P.fixed.astype(bool), 0.0, P.body)
     assert rel(s.applyMapping(x), b) < 1e-9
+
+
+@pytest.mark.parametrize("n,prec", [(64, "fp64"), (64, "fp32"), (128, "fp64")])
+def test_fine_operator_and_residual_at_the_level_edges(make_solver, orc, n, prec):
+    """The operator of the tiled levels (st_fine.hip) on random values everywhere, fixed
+    DOFs scattered to the edges of the level included (what a lane reads outside the level
+    must not enter), against the oracle (1e-12); and one V-cycle, whose residual it also
+    computes, against the oracle's (1e-10 FP64, 1e-4 FP32 storage)."""
+    P, rho = setup(3, n)
+    P.fixed[:] = scattered(P, n)
+    fx, fy, fz = _split(3, n, P.fixed)[1:]
+    fx[n, n // 4:3 * n // 4, :] = 0   # free faces on the far sides, where the last plane, row
+    fy[:, n, n // 4:3 * n // 4] = 0   # and column of the box hold DOFs
+    fz[n // 4:3 * n // 4, :, n] = 0
+    fixed, vol, pen = oracle_desc(orc, P, rho)
+    s = solver_for(make_solver, P, rho, precision=prec)
+    x = np.random.default_rng(3).standard_normal(fixed.size)
+    assert rel(s.applyMapping(x), orc.apply(3, P.shape, fixed, vol, pen, x)) < 1e-12
+    if n == 64:
+        mg = orc.MG(3, P.shape, fixed, pen, nu_pre=1, nu_post=2, omega=1.0, tang=0)
+        x[fixed.astype(bool)] = 0.0
+        assert rel(s.mg_vcycle(x), mg.vcycle(x)) < (1e-10 if prec == "fp64" else 1e-4)
