@@ -10,8 +10,8 @@
 //
 // Per launch, us, against the marching kernel (LDS planes, two barriers per plane):
 //                     256^3 FP64  FP32   128^3 FP64  FP32   64^3 FP64  FP32
-//   y = A x           540 -> 444  262 -> 228   88 -> 68  35 -> 27   31 -> 10  24 -> 10
-//   r = b - A x       627 -> 515  316 -> 249  101 -> 74  44 -> 33   36 -> 13  28 -> 11
+//   y = A x           540 -> 443  262 -> 225   88 -> 66  35 -> 24   31 -> 10  24 -> 9
+//   r = b - A x       627 -> 528  316 -> 245  101 -> 73  44 -> 32   36 -> 13  28 -> 10
 // At 256^3 that is 3.7 to 4.6 TB/s of HBM traffic (FP32 0.83 / 1.14 GB, near the least).
 // Without the masks it gains 10% in FP64 and nothing in FP32, and with fewer registers
 // or other block orders nothing: the mix of 9 to 15 streams and short waves bounds it.
@@ -46,7 +46,9 @@ template <int N, typename T> __device__ __forceinline__ Vec<T, N> vat(const T *p
 }
 template <int N, typename T> __device__ __forceinline__ void vput(T *p, unsigned i, const Vec<T, N> &x)
 {
-    *reinterpret_cast<typename Vec<T, N>::R *>(reinterpret_cast<char *>(p) + i * (unsigned)sizeof(T)) = x.v;
+    // (nontemporal: x, read three times, keeps the caches: 3% at 128^3 and 256^3, 5 to 10% at 64^3)
+    typedef typename Vec<T, N>::R R;
+    __builtin_nontemporal_store(x.v, reinterpret_cast<R *>(reinterpret_cast<char *>(p) + i * (unsigned)sizeof(T)));
 }
 template <int V> struct FlagWord;
 template <> struct FlagWord<2> { typedef uint16_t T; };
@@ -182,6 +184,123 @@ void fine_residual(const Lvl &g, const uint8_t *fl, const TS *al, const TS *b, c
 void fine_apply_mixed(const Lvl &g, const uint8_t *fl, const double *al, const float *x, double *y, hipStream_t s)
 {
     launch_fine<double, float, double, false>(g, fl, al, (const double *)nullptr, x, y, nullptr, s);
+}
+
+// ------------------------------------------- operator on the caller's arrays
+//
+// y = A x on vectors in the caller's layout (fields concatenated without padding, rows of
+// nz, nz, nz and nz + 1 values), FP64, flags and alpha in the node layout: one launch
+// where packing x, the operator and unpacking y were three, two of them transposing
+// copies of the vector.  Kernel time at 256^3 808 -> 494 us (3.0 TB/s; 444 us in the node
+// layout, whose rows are whole lines), 128^3 119 -> 56, 32^3 14 -> 4.7.  A lane takes one
+// node: two of them in 16-byte accesses of 8-byte alignment took the same time, other
+// block orders 1 to 2% more, fewer registers (6 or 8 waves) two to three times as long.
+namespace {
+// The node at padded offset q; qa[f]: its index in field f of the caller's vector, whose
+// rows and planes are sj[f] and si[f] apart.  A velocity outside its field has a clear
+// flag bit, so its read only has to stay inside the vector: before the first entry of
+// field f lies field f - 1, behind the last one field f + 1, and with END (the last three
+// planes; clamping all of them costs 7%) the last field is clamped.  A pressure outside
+// is 0 by position.
+template <int DIM, bool END> struct UserAcc {
+    typedef double C;
+    static constexpr bool MASK = true;
+    const uint8_t *fl;
+    const double *al, *x[DIM + 1];
+    long S, sI, sJ;
+    long si[DIM + 1], sj[DIM + 1];
+    unsigned q, qa[DIM + 1], end;  // end: last entry of the last field
+    bool li, lj, lk, in;           // first node along an axis; a cell of the level
+
+    __device__ __forceinline__ int F(int di, int dj, int dk) const { return at(fl + (di * sI + dj * sJ + dk), q); }
+    __device__ __forceinline__ double X(int f, int di, int dj, int dk) const
+    {
+        if (f == 0) {  // own cell, or the one below along one axis
+            const bool off = di < 0 ? li : (dj < 0 ? lj : (dk < 0 ? lk : !in));
+            const unsigned d = (unsigned)(-di * (int)si[0] - dj * (int)sj[0] - dk);
+            const double v = at(x[0], off ? qa[0] : qa[0] - d);
+            return off ? 0.0 : v;
+        }
+        const long o = di * si[f] + dj * sj[f] + dk;
+        if (f < DIM || !END) return at(x[f] + o, qa[f]);
+        const int e = (int)qa[f] + (int)o;
+        return x[f][e < (int)end ? e : (int)end];
+    }
+    __device__ __forceinline__ double AL(int d, int di, int dj, int dk) const
+    {
+        return at(al + d * S + (di * sI + dj * sJ + dk), q);
+    }
+};
+
+// the rows of node (i, j, k), written to y
+template <int DIM, bool END>
+__device__ __forceinline__ void user_rows(const Lvl &g, const uint8_t *fl, const double *al, const double *x, double *y,
+                                          int i, int j, int k)
+{
+    UserAcc<DIM, END> a;
+    a.fl = fl;
+    a.al = al;
+    a.S = g.S;
+    a.sI = (long)g.Py * g.Pz;
+    a.sJ = g.Pz;
+    a.q = ((unsigned)i * (unsigned)g.Py + (unsigned)j) * (unsigned)g.Pz + (unsigned)k;
+    a.li = i == 0;
+    a.lj = j == 0;
+    a.lk = k == 0;
+    a.in = i < g.nx && j < g.ny && k < g.nz;
+    bool own[DIM + 1];
+    long off = 0;
+#pragma unroll
+    for (int f = 0; f <= DIM; f++) {
+        const int A = g.nx + (f == 1), B = g.ny + (f == 2), Cc = g.nz + (f == 3);
+        a.x[f] = x + off;
+        a.si[f] = (long)B * Cc;
+        a.sj[f] = Cc;
+        a.qa[f] = ((unsigned)i * (unsigned)B + (unsigned)j) * (unsigned)Cc + (unsigned)k;
+        own[f] = i < A && j < B && k < Cc;
+        if (f == DIM) a.end = (unsigned)((long)A * B * Cc - 1);
+        off += (long)A * B * Cc;
+    }
+    const BoxSten<double, DIM, UserAcc<DIM, END>, DIM == 3> s{a};
+    double v[DIM + 1];
+    v[0] = s.cell();
+    v[1] = s.template face<0>(0, 0, 0);
+    v[2] = s.template face<1>(0, 0, 0);
+    if constexpr (DIM == 3) v[3] = s.template face<2>(0, 0, 0);
+#pragma unroll
+    for (int f = 0; f <= DIM; f++)
+        if (own[f]) put(y + (a.x[f] - x), a.qa[f], v[f]);
+}
+}  // namespace
+
+__global__ void __launch_bounds__(256) k_user_apply3(Lvl g, const uint8_t *__restrict__ fl, const double *__restrict__ al,
+                                                     const double *__restrict__ x, double *__restrict__ y, int nb, int sb)
+{
+    int i, blk;
+    if (!strip_of(g.Px, nb, sb, i, blk)) return;
+    const unsigned t = (unsigned)blk * 256u + threadIdx.x;
+    if (t >= (unsigned)g.Py * (unsigned)g.Pz) return;
+    const int j = (int)(t / (unsigned)g.Pz), k = (int)(t - (unsigned)j * (unsigned)g.Pz);
+    if (k > g.nz) return;
+    if (i < g.nx - 2) user_rows<3, false>(g, fl, al, x, y, i, j, k);
+    else user_rows<3, true>(g, fl, al, x, y, i, j, k);
+}
+__global__ void __launch_bounds__(256) k_user_apply2(Lvl g, const uint8_t *__restrict__ fl, const double *__restrict__ al,
+                                                     const double *__restrict__ x, double *__restrict__ y)
+{
+    const unsigned n = blockIdx.x * 256u + threadIdx.x;
+    if (n >= (unsigned)g.S) return;
+    const int i = (int)(n / (unsigned)g.Py);
+    user_rows<2, true>(g, fl, al, x, y, i, (int)(n - (unsigned)i * (unsigned)g.Py), 0);
+}
+void user_apply(const Lvl &g, const uint8_t *fl, const double *al, const double *x, double *y, hipStream_t s)
+{
+    if (g.dim == 2) {
+        hipLaunchKernelGGL(k_user_apply2, dim3((unsigned)((g.S + 255) / 256)), dim3(256), 0, s, g, fl, al, x, y);
+        return;
+    }
+    const int nb = (int)(((long)g.Py * g.Pz + 255) / 256), sb = nb < STRIP ? nb : STRIP;
+    hipLaunchKernelGGL(k_user_apply3, dim3(strip_grid(g.Px, nb, sb)), dim3(256), 0, s, g, fl, al, x, y, nb, sb);
 }
 
 #define INST_F(T)                                                                                          \

@@ -1455,9 +1455,7 @@ int st_apply(st_ctx *c, const double *x, double *y)
     if (!c || !x || !y) return ST_EINVAL;
     if (!c->geom || !c->alpha) return fail(c, ST_ESTATE, "geometry and penalty/design must be set");
     CKR(stage_in(c, x, c->ndof));
-    launch_pack<double>(c->lv[0], c->abi_a, c->Wv, 0, c->fl[0], 1.0, c->s);
-    launch_apply<double>(c->lv[0], c->fl[0], c->h64.al[0], c->Wv, c->BA, c->s);
-    launch_unpack<double>(c->lv[0], c->BA, c->abi_b, c->s);
+    user_apply(c->lv[0], c->fl[0], c->h64.al[0], c->abi_a, c->abi_b, c->s);
     return stage_out(c, y, c->ndof);
 }
 
@@ -1465,9 +1463,10 @@ int st_apply_device(st_ctx *c, const double *d_x, double *d_y)
 {
     if (!c || !d_x || !d_y) return ST_EINVAL;
     if (!c->geom || !c->alpha) return fail(c, ST_ESTATE, "geometry and penalty/design must be set");
-    launch_pack<double>(c->lv[0], d_x, c->Wv, 0, c->fl[0], 1.0, c->s);
-    launch_apply<double>(c->lv[0], c->fl[0], c->h64.al[0], c->Wv, c->BA, c->s);
-    launch_unpack<double>(c->lv[0], c->BA, d_y, c->s);
+    // y on top of x (in place, or shifted): the neighbours' values are read from a copy
+    const bool over = d_x < d_y + c->ndof && d_y < d_x + c->ndof;
+    if (over) CK(hipMemcpyAsync(c->abi_a, d_x, sizeof(double) * c->ndof, hipMemcpyDeviceToDevice, c->s));
+    user_apply(c->lv[0], c->fl[0], c->h64.al[0], over ? c->abi_a : d_x, d_y, c->s);
     CK(hipStreamSynchronize(c->s));
     return ST_OK;
 }

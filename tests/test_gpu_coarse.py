@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from conftest import rel
-from helpers import oracle_desc, setup, solver_for
+from helpers import DeviceArray, oracle_desc, setup, solver_for
 from stokes_to_amd.problems import _split, reference_test0
 
 pytestmark = pytest.mark.gpu
@@ -68,3 +68,29 @@ def test_fine_operator_and_residual_at_the_level_edges(make_solver, orc, n, prec
         mg = orc.MG(3, P.shape, fixed, pen, nu_pre=1, nu_post=2, omega=1.0, tang=0)
         x[fixed.astype(bool)] = 0.0
         assert rel(s.mg_vcycle(x), mg.vcycle(x)) < (1e-10 if prec == "fp64" else 1e-4)
+
+
+@pytest.mark.parametrize("dim,n", [(2, 8), (2, 64), (3, 8), (3, 16), (3, 64)])
+def test_operator_on_device_vectors_stays_inside_and_may_overlap(make_solver, orc, dim, n):
+    """st_apply_device on a vector between NaNs (what lies outside x must not enter, what
+    lies outside y stays), then with y over x, shifted and in place: 1e-12 of the oracle."""
+    P, rho = setup(dim, n)
+    P.fixed[:] = scattered(P, n)
+    fixed, vol, pen = oracle_desc(orc, P, rho)
+    s = solver_for(make_solver, P, rho)
+    nd, pad = fixed.size, 2 * n * n
+    x = np.random.default_rng(5).standard_normal(nd)
+    ref = orc.apply(dim, P.shape, fixed, vol, pen, x)
+    band = np.full(nd + 2 * pad, np.nan)
+    band[pad:-pad] = x
+    dx, dy = DeviceArray(band), DeviceArray(np.full(nd + 2 * pad, 7.0))
+    assert s.lib.st_apply_device(s.h, dx.ptr.value + 8 * pad, dy.ptr.value + 8 * pad) == 0
+    y = dy.get()
+    assert rel(y[pad:-pad], ref) < 1e-12
+    assert (y[:pad] == 7.0).all() and (y[-pad:] == 7.0).all()
+    assert s.lib.st_apply_device(s.h, dx.ptr.value + 8 * pad, dx.ptr.value + 8 * (pad - 3)) == 0
+    assert rel(dx.get()[pad - 3:pad - 3 + nd], ref) < 1e-12
+    assert s.lib.st_apply_device(s.h, dy.ptr.value + 8 * pad, dy.ptr.value + 8 * pad) == 0
+    assert rel(dy.get()[pad:-pad], orc.apply(dim, P.shape, fixed, vol, pen, y[pad:-pad])) < 1e-12
+    dx.free()
+    dy.free()
