@@ -50,35 +50,72 @@ __device__ __forceinline__ void tap_off(int t, int ntap, int &a, int &b, int &c)
 
 // ------------------------------------------------------------- convolution
 
-// out[v][co] (+)= bias[co] + sum_t sum_ci in[v + o_t][ci] W[t][ci][co]
+// out[v][co] = bias[co] + sum_t sum_ci in[v + o_t][ci] W[t][ci][co]
 // D = A B with A = W^T (16 out channels x 16 in channels per tap/block, packed in
 // the MFMA A-operand lane order) and B = 16 input channels x 16 voxels; each wave
-// produces 16 out channels x 16 voxels.  OUTM: 0 bf16 store, 1 f32 store,
-// 2 f32 accumulate.
-template <int NTAP, int OUTM, bool RELU>
+// produces 16 out channels x 16 voxels.  OUTM: 0 bf16 store, 1 f32 store.
+// NCIB: input channel blocks (0: ncib, at run time).  The products of a wave form one
+// chain in a fixed order, so what bounds it is how early the operands are there: with
+// NCIB known the operands of a row of three taps are loaded while the row before is
+// multiplied: 18 -> 6.0 us (32^3 voxels, 16 channels), 26 -> 7.3 (16^3, 32), 28 -> 17
+// (8^3, 64: 27 KB of weights a wave, read once).
+template <int NTAP, int NCIB, int OUTM, bool RELU>
 __global__ void __launch_bounds__(256) k_conv(int R, const bf16 *__restrict__ in, int csi, int cio, int ncib,
                                               const bf4 *__restrict__ Wp, const float *__restrict__ bias, void *out,
                                               int cso, int coo, int ncob)
 {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const long nv = (long)R * R * R;
-    const long v0 = ((long)blockIdx.x * 4 + w) * 16;
+    const int nv = R * R * R;
     const int ob = blockIdx.y;
-    const long v = v0 + (lane & 15);
+    const int v = (blockIdx.x * 4 + w) * 16 + (lane & 15);
     const int kq = lane >> 4;
-    const int vi = (int)(v / ((long)R * R)), vj = (int)((v / R) % R), vk = (int)(v % R);
+    const int vi = v / (R * R), vj = (v / R) % R, vk = v % R;
     f4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int t = 0; t < NTAP; t++) {
-        int a, b, c;
-        tap_off(t, NTAP, a, b, c);
+    auto tap_in = [&](int a, int b, int c) {
         const int ii = vi + a, jj = vj + b, kk = vk + c;
-        const bool ok = v < nv && ii >= 0 && jj >= 0 && kk >= 0 && ii < R && jj < R && kk < R;
-        const long nb = (((long)ii * R + jj) * R + kk);
-        for (int cb = 0; cb < ncib; cb++) {
-            bf4 xb = {{0, 0, 0, 0}};
-            if (ok) xb = *(const bf4 *)(in + nb * csi + cio + cb * 16 + kq * 4);
-            const bf4 wa = Wp[(((long)t * ncib + cb) * ncob + ob) * 64 + lane];
-            acc = mfma16(as_s4(wa), as_s4(xb), acc);
+        return v < nv && ii >= 0 && jj >= 0 && kk >= 0 && ii < R && jj < R && kk < R;
+    };
+    if constexpr (NTAP == 27 && NCIB > 0) {
+        constexpr int N = 3 * NCIB;
+        bf4 X[2][N], A[2][N];
+        bool ok[2][3];
+        const unsigned own = (v < nv ? (unsigned)v : 0u) * (unsigned)csi + (unsigned)(cio + kq * 4);
+        auto load = [&](int r, int h) {  // the taps (r / 3 - 1, r % 3 - 1, *)
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                const int a = r / 3 - 1, b = r % 3 - 1;
+                ok[h][c] = tap_in(a, b, c - 1);
+                const unsigned o = own + (ok[h][c] ? (unsigned)((((a * R + b) * R) + c - 1) * csi) : 0u);
+#pragma unroll
+                for (int cb = 0; cb < NCIB; cb++) {
+                    X[h][c * NCIB + cb] = *(const bf4 *)(in + o + cb * 16);
+                    A[h][c * NCIB + cb] = Wp[(unsigned)(((r * 3 + c) * NCIB + cb) * ncob + ob) * 64u + lane];
+                }
+            }
+        };
+        load(0, 0);
+#pragma unroll
+        for (int r = 0; r < 9; r++) {
+            if (r < 8) load(r + 1, (r + 1) & 1);
+#pragma unroll
+            for (int q = 0; q < N; q++) {
+                const s4 z = {0, 0, 0, 0};
+                const s4 xb = as_s4(X[r & 1][q]);
+                acc = mfma16(as_s4(A[r & 1][q]), ok[r & 1][q / NCIB] ? xb : z, acc);
+            }
+        }
+    } else {
+        for (int t = 0; t < NTAP; t++) {
+            int a, b, c;
+            tap_off(t, NTAP, a, b, c);
+            const bool ok = tap_in(a, b, c);
+            const long nb = ((long)(vi + a) * R + vj + b) * R + vk + c;
+            for (int cb = 0; cb < ncib; cb++) {
+                bf4 xb = {{0, 0, 0, 0}};
+                if (ok) xb = *(const bf4 *)(in + nb * csi + cio + cb * 16 + kq * 4);
+                const bf4 wa = Wp[(((long)t * ncib + cb) * ncob + ob) * 64 + lane];
+                acc = mfma16(as_s4(wa), as_s4(xb), acc);
+            }
         }
     }
     if (v >= nv) return;
@@ -90,14 +127,13 @@ __global__ void __launch_bounds__(256) k_conv(int R, const bf16 *__restrict__ in
             if (RELU && s < 0.f) s = 0.f;
             o.v[q] = to_bf16(s).v;
         }
-        *(bf4 *)((bf16 *)out + v * cso + coo + co) = o;
+        *(bf4 *)((bf16 *)out + (long)v * cso + coo + co) = o;
     } else {
-        float *op = (float *)out + v * cso + coo + co;
+        float *op = (float *)out + (long)v * cso + coo + co;
         for (int q = 0; q < 4; q++) {
             float s = acc[q] + (bias ? bias[co + q] : 0.f);
             if (RELU && s < 0.f) s = 0.f;
-            if (OUTM == 2) op[q] += s;
-            else op[q] = s;
+            op[q] = s;
         }
     }
 }
@@ -158,18 +194,35 @@ __global__ void __launch_bounds__(64) k_conv_wgrad(int R, const bf16 *__restrict
 //     k shifts)
 //   gs[ob][v/4][co%16][v%4] = gz(v, ob*16 + co%16)
 // so the operand of lane l = 16 qd + m for the 16 voxels from v0 (one k row) is the
-// 8 bytes at 64 (v0/4 + qd) + 4 m: a wave's load is 512 contiguous bytes.  One wave
-// accumulates all taps of one (ci block, co block) over its voxel groups and writes
-// its partial.
-// one (i+1, j+1) row of xs for one ci block per workgroup (grid: P*P rows x ncib): the
+// 8 bytes at 64 (v0/4 + qd) + 4 m: a wave's load is 512 contiguous bytes.
+//
+// One launch stages both and applies the activation's derivative on the way: gz =
+// bf16(gy (y > 0)) (relu) or bf16(gy), also written channel-last for the data gradient.
+// Its first P*P*ncib workgroups stage x, one (i+1, j+1) row for one ci block each: the
 // row's R voxels x 16 channels are read channel-contiguous into LDS with a zero at
-// each end, then written as the three k-shifted interleaved rows; pad rows are zero
-__global__ void __launch_bounds__(256) k_wg_stage_x(int R, const bf16 *__restrict__ x, int csx, int cix, int ncib,
-                                                    bf16 *__restrict__ xs)
+// each end, then written as the three k-shifted interleaved rows; pad rows are zero.
+__global__ void __launch_bounds__(256) k_wg_stage(int R, const bf16 *__restrict__ x, int csx, int cix, int ncib,
+                                                  bf16 *__restrict__ xs, int C, const bf16 *__restrict__ y, int csy,
+                                                  int cy, const float *__restrict__ gy, int csg, int cg, int relu,
+                                                  bf16 *__restrict__ gz, bf16 *__restrict__ gs)
 {
     __shared__ uint16_t sm[16][130];  // R <= 128
-    const int P = R + 2;
-    const int row = blockIdx.x, cb = blockIdx.y;
+    const int P = R + 2, nbx = P * P * ncib;
+    if ((int)blockIdx.x >= nbx) {
+        const int nv = R * R * R, tot = nv * C, step = (int)(gridDim.x - nbx) * 256;
+        for (int q = ((int)blockIdx.x - nbx) * 256 + (int)threadIdx.x; q < tot; q += step) {
+            // q = ((ob (nv/4) + v/4) 16 + co%16) 4 + v%4
+            const int v = ((q >> 6) % (nv >> 2)) * 4 + (q & 3);
+            const int co = (q / (16 * nv)) * 16 + ((q >> 2) & 15);
+            float g = gy[(long)v * csg + cg + co];
+            if (relu && !(to_f(y[(long)v * csy + cy + co]) > 0.f)) g = 0.f;
+            const bf16 z = to_bf16(g);
+            gz[(long)v * C + co] = z;
+            gs[q] = z;
+        }
+        return;
+    }
+    const int row = (int)blockIdx.x % (P * P), cb = (int)blockIdx.x / (P * P);
     const int i = row / P - 1, j = row % P - 1;
     const bool pad = i < 0 || i >= R || j < 0 || j >= R;
     if (!pad) {
@@ -200,75 +253,62 @@ __device__ __forceinline__ long gs_at(long nv, long v, int co)
     return (((long)(co >> 4) * (nv >> 2) + (v >> 2)) * 16 + (co & 15)) * 4 + (v & 3);
 }
 
-__global__ void __launch_bounds__(256) k_wg_stage_g(long nv, int C, const bf16 *__restrict__ gz, bf16 *__restrict__ gs)
+// The sum over the voxels is split into nsplit runs of gpw groups of 16 voxels (one
+// chain of products each) and these are added, in order, in WG_G segments: a workgroup
+// does one segment of one tap of one (ci block, co block), its waves the runs of it in
+// turn, and adds their results in order from LDS.  part2[segment][t][ci][co]; segment =
+// blockIdx.x, so the workgroups that read the same voxels run on one XCD (WG_G % 8 == 0).
+// (With all taps in one wave, and each run's sum written out and summed by a second
+// launch, 56 MB of partials went through memory at 32^3, 16 channels: 14 + 20 us, now 13.5.)
+constexpr int WG_G = 32, WG_RUNS = 64;  // segments (weights and bias), most runs of one
+template <int W>
+__global__ void __launch_bounds__(64 * W) k_wg(int R, int ntap, const bf16 *__restrict__ xs,
+                                               const bf16 *__restrict__ gs, int ncib, int ncob, int nsplit, int gpw,
+                                               float *__restrict__ part2)
 {
-    const long tot = nv * C;
-    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < tot; q += (long)gridDim.x * blockDim.x) {
-        // q = ((ob (nv/4) + v/4) 16 + co%16) 4 + v%4
-        const long v = ((q >> 6) % (nv >> 2)) * 4 + (q & 3);
-        const int co = (int)(q / (16 * nv)) * 16 + (int)((q >> 2) & 15);
-        gs[q] = gz[v * C + co];
-    }
-}
-
-// 1D grid of nch chunks x (ci blocks x co blocks) pairs, a multiple of 8 workgroups,
-// 4 waves per block, gpw voxel groups of 16 per wave; part[split][t][ci][co], split =
-// chunk * 4 + wave (every entry of every split is written, zeros for a wave past the
-// last group).  Workgroup L runs on XCD L % 8; it takes logical block
-// (L % 8) * (nblocks / 8) + L / 8, so each XCD sweeps a contiguous run of chunks and
-// the rows that neighbouring chunks share (taps one row or plane away) meet in its L2.
-template <int NTAP>
-__global__ void __launch_bounds__(256) k_wg_staged(int R, const bf16 *__restrict__ xs, const bf16 *__restrict__ gs,
-                                                   int ncib, int ncob, int nch, long gpw, float *__restrict__ part)
-{
+    constexpr int RUNS = W == 16 ? WG_RUNS : (W == 4 ? 16 : 1);
+    __shared__ float sh[W > 1 ? RUNS * 256 : 1];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int L = blockIdx.x, per = gridDim.x >> 3;
-    const int lb = (L & 7) * per + (L >> 3);
-    const int chunk = lb % nch, pair = lb / nch;
-    const int cb = pair / ncob, ob = pair % ncob;
-    const long nv = (long)R * R * R, ngroups = nv / 16;
-    const int P = R + 2;
+    const int seg = blockIdx.x, cb = (int)blockIdx.y / ncob, ob = (int)blockIdx.y % ncob, t = blockIdx.z;
+    const int p0 = (int)((long)nsplit * seg / WG_G), p1 = (int)((long)nsplit * (seg + 1) / WG_G);
+    const int ngroups = R * R * R / 16, P = R + 2;
     const int m = lane & 15, qd = lane >> 4;
     const long rowl = 16L * R, plane = (long)P * P * rowl;
-    const bf16 *xb = xs + (long)cb * 3 * plane + 4 * m;
-    const bf16 *gb = gs + (long)ob * 16 * nv + 4 * m;
-    f4 acc[NTAP];
+    int a, b, c;
+    tap_off(t, ntap, a, b, c);
+    const bf16 *xb = xs + (long)cb * 3 * plane + (c + 1) * plane + ((long)(a + 1) * P + b + 1) * rowl + 4 * m;
+    const bf16 *gb = gs + (long)ob * ngroups * 256 + 4 * m;
+    f4 s = {0.f, 0.f, 0.f, 0.f};
+    for (int p = p0 + w; p < p1; p += W) {
+        f4 acc = {0.f, 0.f, 0.f, 0.f};
+        const int g0 = p * gpw, g1 = g0 + gpw < ngroups ? g0 + gpw : ngroups;
+#pragma unroll 4
+        for (int g = g0; g < g1; g++) {
+            const int v = g * 16 + 4 * qd;  // this lane's quad of voxels (one k row: R % 4 == 0)
+            const int k = v % R, j = (v / R) % R, i = v / (R * R);
+            const bf4 bq = *(const bf4 *)(gb + 16 * (long)v);  // B[k = voxel][n = co]
+            const bf4 aq = *(const bf4 *)(xb + ((long)i * P + j) * rowl + 16 * k);
+            acc = mfma16(as_s4(aq), as_s4(bq), acc);  // A[m = ci][k = voxel]
+        }
 #pragma unroll
-    for (int t = 0; t < NTAP; t++) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-    const long split = (long)chunk * 4 + w;
-    const long g0 = split * gpw;
-    const long g1 = (g0 + gpw < ngroups) ? g0 + gpw : ngroups;
-    for (long g = g0; g < g1; g++) {
-        const long v = g * 16 + 4 * qd;  // this lane's quad of voxels (one k row: R % 4 == 0)
-        const int k = (int)(v % R), j = (int)((v / R) % R), i = (int)(v / ((long)R * R));
-        const bf4 bq = *(const bf4 *)(gb + 16 * v);  // B[k = voxel][n = co]
-#pragma unroll
-        for (int t = 0; t < NTAP; t++) {
-            int a, b, c;
-            tap_off(t, NTAP, a, b, c);
-            const long row = (long)(i + a + 1) * P + (j + b + 1);
-            const bf4 aq = *(const bf4 *)(xb + (c + 1) * plane + row * rowl + 16 * k);
-            acc[t] = mfma16(as_s4(aq), as_s4(bq), acc[t]);  // A[m = ci][k = voxel]
+        for (int q = 0; q < 4; q++) {
+            if (W > 1) sh[(p - p0) * 256 + q * 64 + lane] = acc[q];
+            else s[q] += acc[q];
         }
     }
     const int Cin = ncib * 16, Cout = ncob * 16;
+    float *o = part2 + (((long)seg * ntap + t) * Cin + cb * 16 + 4 * qd) * Cout + ob * 16 + m;
+    if (W == 1) {
 #pragma unroll
-    for (int t = 0; t < NTAP; t++)
-        for (int q = 0; q < 4; q++)
-            part[((split * NTAP + t) * Cin + cb * 16 + 4 * qd + q) * Cout + ob * 16 + m] = acc[t][q];
-}
-
-// first stage of the reduction of many partials: group g of the nsplit partials of
-// every entry summed into part2[g][q] (grid: entry blocks x groups)
-__global__ void __launch_bounds__(256) k_reduce_parts_grouped(long n, int nsplit, const float *part, float *part2)
-{
-    const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n) return;
-    const int G = gridDim.y, g = blockIdx.y;
-    const int p0 = (int)((long)nsplit * g / G), p1 = (int)((long)nsplit * (g + 1) / G);
-    float s = 0.f;
-    for (int p = p0; p < p1; p++) s += part[(long)p * n + q];
-    part2[(long)g * n + q] = s;
+        for (int q = 0; q < 4; q++) o[(long)q * Cout] = s[q];
+        return;
+    }
+    __syncthreads();
+    if (w < 4) {
+        float r = 0.f;
+        for (int p = 0; p < p1 - p0; p++) r += sh[p * 256 + w * 64 + lane];
+        o[(long)w * Cout] = r;
+    }
 }
 
 // bias gradient partials from the staged gradient: block (g, co) sums its segment of
@@ -412,46 +452,74 @@ __global__ void __launch_bounds__(256) k_loss(long nv, const float *y, const flo
     if (threadIdx.x == 0) part[blockIdx.x] = sh[0] / (double)(nv * NET_NOUT);
 }
 
-__global__ void k_adam(long n, float *p, const float *g, float *m, float *v, float lr, float b1, float b2, float eps,
-                       float c1, float c2)
+// Layers of the flat parameter array: [W | b] per layer (off), the segment sums of its
+// weight and bias gradients (p2: [WG_G][nw] then [WG_G][cout]; < 0: the gradient is in g
+// already), its packed weights (pk).
+struct NetTab {
+    int ntap[NET_NLAYER], ncib[NET_NLAYER], ncob[NET_NLAYER];
+    long off[NET_NLAYER], p2[NET_NLAYER], pk[NET_NLAYER];
+};
+
+// gradient of every parameter from the segment sums, and with train the Adam step;
+// blockIdx.y: the layer (one launch where each layer took two for either)
+__global__ void __launch_bounds__(256) k_update(NetTab tb, const float *__restrict__ part2, float *__restrict__ gr,
+                                                int train, float *__restrict__ pa, float *__restrict__ ma,
+                                                float *__restrict__ va, float lr, float b1, float b2, float eps,
+                                                float c1, float c2)
 {
-    long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n) return;
-    float gg = g[q];
-    float mm = b1 * m[q] + (1.f - b1) * gg;
-    float vv = b2 * v[q] + (1.f - b2) * gg * gg;
-    m[q] = mm;
-    v[q] = vv;
-    p[q] -= lr * (mm / c1) / (sqrtf(vv / c2) + eps);
+    const int l = blockIdx.y;
+    const int cout = tb.ncob[l] * 16, nw = tb.ntap[l] * tb.ncib[l] * 16 * cout;
+    const int q = (int)(blockIdx.x * 256 + threadIdx.x);
+    if (q >= nw + cout) return;
+    const long e = tb.off[l] + q;
+    if (tb.p2[l] >= 0) {
+        const float *part = part2 + tb.p2[l] + (q < nw ? q : (long)WG_G * nw + (q - nw));
+        const int n = q < nw ? nw : cout;
+        float s = 0.f;
+#pragma unroll 8
+        for (int p = 0; p < WG_G; p++) s += part[(long)p * n];
+        gr[e] = s;
+    }
+    if (!train) return;
+    float gg = gr[e];
+    float mm = b1 * ma[e] + (1.f - b1) * gg;
+    float vv = b2 * va[e] + (1.f - b2) * gg * gg;
+    ma[e] = mm;
+    va[e] = vv;
+    pa[e] -= lr * (mm / c1) / (sqrtf(vv / c2) + eps);
 }
 
-// pack W[t][ci][co] (f32) into the MFMA A-operand lane order:
+// pack W[t][ci][co] (f32) of every layer into the MFMA A-operand lane order:
 // forward  A[m = co][k = ci] per (t, ci block, co block)
 // backward A[m = ci][k = co] of the flipped kernel W'[t][co][ci] = W[T-1-t][ci][co]
-__global__ void k_pack_w(int ntap, int ncib, int ncob, const float *W, bf4 *Wp, int flip)
+// blockIdx.y: the layer, twice (forward, backward)
+__global__ void __launch_bounds__(256) k_pack_w(NetTab tb, const float *__restrict__ pa, bf4 *__restrict__ Wf,
+                                                bf4 *__restrict__ Wb)
 {
-    long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    long n = (long)ntap * ncib * ncob * 64;
-    if (q >= n) return;
-    int lane = (int)(q % 64);
-    long r = q / 64;
+    const int l = blockIdx.y >> 1, flip = blockIdx.y & 1;
+    const int ntap = tb.ntap[l], ncib = tb.ncib[l], ncob = tb.ncob[l];
+    const int q = (int)(blockIdx.x * 256 + threadIdx.x);
+    if (q >= ntap * ncib * ncob * 64) return;
+    const float *W = pa + tb.off[l];
+    int lane = q % 64;
+    int r = q / 64;
     int Cin = ncib * 16, Cout = ncob * 16;
     bf4 o;
     if (!flip) {
-        int ob = (int)(r % ncob), cb = (int)((r / ncob) % ncib), t = (int)(r / (ncob * ncib));
+        int ob = r % ncob, cb = (r / ncob) % ncib, t = r / (ncob * ncib);
         for (int j = 0; j < 4; j++) {
             int ci = cb * 16 + 4 * (lane >> 4) + j, co = ob * 16 + (lane & 15);
             o.v[j] = to_bf16(W[((long)t * Cin + ci) * Cout + co]).v;
         }
     } else {
         // conv over gz (in channels = co, blocks ncob) producing gx (out channels = ci)
-        int cb = (int)(r % ncib), ob = (int)((r / ncib) % ncob), t = (int)(r / (ncib * ncob));
+        int cb = r % ncib, ob = (r / ncib) % ncob, t = r / (ncib * ncob);
         for (int j = 0; j < 4; j++) {
             int ci = cb * 16 + (lane & 15), co = ob * 16 + 4 * (lane >> 4) + j;
             o.v[j] = to_bf16(W[((long)(ntap - 1 - t) * Cin + ci) * Cout + co]).v;
         }
     }
-    Wp[q] = o;
+    (flip ? Wb : Wf)[tb.pk[l] + q] = o;
 }
 
 template <typename TS>
@@ -619,35 +687,53 @@ long wg_xs_elems(int R, int cin)
     return (long)(cin / 16) * 3 * 16 * P * P * R;
 }
 bool wg_staged_ok(int R) { return R >= 4 && R % 4 == 0 && R <= 128; }
-constexpr int WG_G = 32;  // groups of the first reduction stage (weights and bias)
-// gW = sum over voxels of x(v + o_t) gz(v) for every tap, gb = sum over voxels of gz(v)
-// (xs, gs: staging buffers of wg_xs_elems(R, cin) and R^3 cout elements; part:
-// wg_plan(...).nsplit * ntap cin cout; part2: WG_G * max(ntap cin cout, cout))
-void wgrad_staged(int R, int ntap, int cin, int cout, const bf16 *x, int csx, int cix, const bf16 *gz, bf16 *xs,
-                  bf16 *gs, float *part, float *part2, float *gW, float *gb, hipStream_t s)
+// segment sums of gW = sum over voxels of x(v + o_t) gz(v) for every tap (part2) and of
+// gb = sum over voxels of gz(v) (part2 + WG_G ntap cin cout), and gz itself from gy and
+// the activation y (xs, gs: staging buffers of wg_xs_elems(R, cin) and R^3 cout elements).
+// Waves of a workgroup by the runs in a segment: up to 64 runs (16 channels) over 16
+// waves, the 1 to 3 of the layers with many channels over one (and no LDS).
+void wgrad_staged(int R, int ntap, int cin, int cout, const bf16 *x, int csx, int cix, const bf16 *y, int csy, int cy,
+                  const float *gy, int csg, int cg, int relu, bf16 *gz, bf16 *xs, bf16 *gs, float *part2, hipStream_t s)
 {
     const WgPlan pl = wg_plan(R, cin, cout);
     const long nv = (long)R * R * R, nw = (long)ntap * cin * cout;
-    hipLaunchKernelGGL(k_wg_stage_x, dim3((unsigned)((R + 2) * (R + 2)), (unsigned)(cin / 16)), dim3(256), 0, s, R, x, csx,
-                       cix, cin / 16, xs);
-    hipLaunchKernelGGL(k_wg_stage_g, dim3(nblk_cap(nv * cout)), dim3(256), 0, s, nv, cout, gz, gs);
-    const dim3 grid((unsigned)(pl.nchunks * (cin / 16) * (cout / 16)));
-    const int nch = (int)pl.nchunks;
-    if (ntap == 27)
-        hipLaunchKernelGGL((k_wg_staged<27>), grid, dim3(256), 0, s, R, xs, gs, cin / 16, cout / 16, nch, pl.gpw, part);
+    const unsigned nbx = (unsigned)((R + 2) * (R + 2) * (cin / 16));
+    hipLaunchKernelGGL(k_wg_stage, dim3(nbx + nblk_cap(nv * cout)), dim3(256), 0, s, R, x, csx, cix, cin / 16, xs, cout, y,
+                       csy, cy, gy, csg, cg, relu, gz, gs);
+    const dim3 grid(WG_G, (unsigned)((cin / 16) * (cout / 16)), (unsigned)ntap);
+    const int ns = (int)pl.nsplit, gpw = (int)pl.gpw, runs = (ns + WG_G - 1) / WG_G;
+    if (runs > 16)
+        hipLaunchKernelGGL((k_wg<16>), grid, dim3(1024), 0, s, R, ntap, xs, gs, cin / 16, cout / 16, ns, gpw, part2);
+    else if (runs > 3)
+        hipLaunchKernelGGL((k_wg<4>), grid, dim3(256), 0, s, R, ntap, xs, gs, cin / 16, cout / 16, ns, gpw, part2);
     else
-        hipLaunchKernelGGL((k_wg_staged<1>), grid, dim3(256), 0, s, R, xs, gs, cin / 16, cout / 16, nch, pl.gpw, part);
-    hipLaunchKernelGGL(k_reduce_parts_grouped, dim3(nblk(nw), WG_G), dim3(256), 0, s, nw, (int)pl.nsplit, part, part2);
-    hipLaunchKernelGGL(k_reduce_parts, dim3(nblk(nw)), dim3(256), 0, s, nw, WG_G, part2, gW);
-    hipLaunchKernelGGL(k_rowsum_parts, dim3(WG_G, cout), dim3(256), 0, s, nv, gs, part2);
-    hipLaunchKernelGGL(k_reduce_parts, dim3(nblk(cout)), dim3(256), 0, s, (long)cout, WG_G, part2, gb);
+        hipLaunchKernelGGL((k_wg<1>), grid, dim3(64), 0, s, R, ntap, xs, gs, cin / 16, cout / 16, ns, gpw, part2);
+    hipLaunchKernelGGL(k_rowsum_parts, dim3(WG_G, cout), dim3(256), 0, s, nv, gs, part2 + WG_G * nw);
+}
+
+// the convolution kernel for the layer's input channels
+template <int OUTM, bool RELU>
+void conv27(dim3 grid, int R, const bf16 *in, int csi, int cio, int ncib, const bf4 *Wp, const float *bias, void *out,
+            int cso, int coo, int ncob, hipStream_t s)
+{
+#define ST_CONV(N)                                                                                                    \
+    hipLaunchKernelGGL((k_conv<27, N, OUTM, RELU>), grid, dim3(256), 0, s, R, in, csi, cio, ncib, Wp, bias, out, cso, \
+                       coo, ncob)
+    switch (ncib) {
+    case 1: ST_CONV(1); break;
+    case 2: ST_CONV(2); break;
+    case 3: ST_CONV(3); break;
+    case 4: ST_CONV(4); break;
+    case 6: ST_CONV(6); break;
+    default: ST_CONV(0); break;
+    }
+#undef ST_CONV
 }
 
 struct Layer {
     NetLayerSpec sp;
     long nw = 0;
-    float *W = nullptr, *b = nullptr, *mW = nullptr, *vW = nullptr, *mb = nullptr, *vb = nullptr, *gW = nullptr,
-          *gb = nullptr;
+    float *W = nullptr, *b = nullptr, *gW = nullptr, *gb = nullptr, *part2 = nullptr;  // in the flat arrays
     bf4 *Wp = nullptr, *Wq = nullptr;
 };
 }  // namespace
@@ -662,7 +748,11 @@ struct NetImpl {
     float *OUT, *gOUT, *gD1b, *gD1a, *gD1in, *gD2b, *gD2a, *gD2in, *gE3b, *gE3a, *gP2, *gE2a, *gP1, *gE1a;
     float *part, *feat, *tgt_raw, *tgt, *scale;
     bf16 *wxs = nullptr, *wgs = nullptr;  // staging of the weight gradient
-    float *part2 = nullptr;               // its first reduction stage
+    float *part2 = nullptr;               // its segment sums, per layer
+    float *par = nullptr, *mom = nullptr, *var = nullptr, *grd = nullptr;  // flat [W | b] per layer
+    bf4 *wpk = nullptr, *wqk = nullptr;                                    // packed weights
+    NetTab tab;
+    long npar = 0, npk = 0;
     double *lpart;
     bool scaled = false;
     float hscale[NET_NOUT] = {1, 1, 1, 1};
@@ -687,12 +777,10 @@ struct NetImpl {
         dim3 grid(nblk(nv(p.lvl), 64), p.cout / 16);
         const int ncib = p.cin / 16, ncob = p.cout / 16;
         if (p.ntap == 27) {
-            if (outm == 0 && p.relu)
-                hipLaunchKernelGGL((k_conv<27, 0, true>), grid, dim3(256), 0, s, Rl, in, csi, cio, ncib, L[l].Wp, L[l].b, out, cso, coo, ncob);
-            else
-                hipLaunchKernelGGL((k_conv<27, 1, false>), grid, dim3(256), 0, s, Rl, in, csi, cio, ncib, L[l].Wp, L[l].b, out, cso, coo, ncob);
+            if (outm == 0 && p.relu) conv27<0, true>(grid, Rl, in, csi, cio, ncib, L[l].Wp, L[l].b, out, cso, coo, ncob, s);
+            else conv27<1, false>(grid, Rl, in, csi, cio, ncib, L[l].Wp, L[l].b, out, cso, coo, ncob, s);
         } else {
-            hipLaunchKernelGGL((k_conv<1, 1, false>), grid, dim3(256), 0, s, Rl, in, csi, cio, ncib, L[l].Wp, L[l].b, out, cso, coo, ncob);
+            hipLaunchKernelGGL((k_conv<1, 0, 1, false>), grid, dim3(256), 0, s, Rl, in, csi, cio, ncib, L[l].Wp, L[l].b, out, cso, coo, ncob);
         }
     }
     // gx = conv^T(gz) written (f32) into a channel slice
@@ -702,45 +790,47 @@ struct NetImpl {
         const int Rl = res(p.lvl);
         dim3 grid(nblk(nv(p.lvl), 64), p.cin / 16);
         if (p.ntap == 27)
-            hipLaunchKernelGGL((k_conv<27, 1, false>), grid, dim3(256), 0, s, Rl, gzin, p.cout, 0, p.cout / 16, L[l].Wq, (const float *)nullptr, (void *)gx, csg, cig, p.cin / 16);
+            conv27<1, false>(grid, Rl, gzin, p.cout, 0, p.cout / 16, L[l].Wq, nullptr, gx, csg, cig, p.cin / 16, s);
         else
-            hipLaunchKernelGGL((k_conv<1, 1, false>), grid, dim3(256), 0, s, Rl, gzin, p.cout, 0, p.cout / 16, L[l].Wq, (const float *)nullptr, (void *)gx, csg, cig, p.cin / 16);
+            hipLaunchKernelGGL((k_conv<1, 0, 1, false>), grid, dim3(256), 0, s, Rl, gzin, p.cout, 0, p.cout / 16, L[l].Wq, (const float *)nullptr, (void *)gx, csg, cig, p.cin / 16);
     }
-    void conv_wgrad(int l, const bf16 *x, int csx, int cix, const bf16 *gzin)
+    // gz = gradient through the activation y (csy, cy: its channel slice), and the weight and
+    // bias gradients of the layer for its input x (or their segment sums)
+    void layer_grad(int l, const bf16 *y, int csy, int cy, const float *gy, int csg, int cg, const bf16 *x, int csx, int cix)
     {
         const NetLayerSpec &p = L[l].sp;
         const int Rl = res(p.lvl);
         const long n = nv(p.lvl);
         if (wg_staged_ok(Rl)) {
-            wgrad_staged(Rl, p.ntap, p.cin, p.cout, x, csx, cix, gzin, wxs, wgs, part, part2, L[l].gW, L[l].gb, s);
+            wgrad_staged(Rl, p.ntap, p.cin, p.cout, x, csx, cix, y, csy, cy, gy, csg, cg, p.relu, gz, wxs, wgs, L[l].part2, s);
             return;
         }
+        hipLaunchKernelGGL(k_act_bwd, dim3(nblk(n * p.cout)), dim3(256), 0, s, n, p.cout, y, csy, cy, gy, csg, cg, gz, p.relu);
         int ns = nsplit;
         long chunk = (n + ns - 1) / ns;
         chunk = (chunk + 15) / 16 * 16;
         ns = (int)((n + chunk - 1) / chunk);
         dim3 grid(p.ntap * (p.cin / 16) * (p.cout / 16), ns);
         if (p.ntap == 27)
-            hipLaunchKernelGGL((k_conv_wgrad<27>), grid, dim3(64), 0, s, Rl, x, csx, cix, p.cin / 16, gzin, p.cout / 16, chunk, part);
+            hipLaunchKernelGGL((k_conv_wgrad<27>), grid, dim3(64), 0, s, Rl, x, csx, cix, p.cin / 16, gz, p.cout / 16, chunk, part);
         else
-            hipLaunchKernelGGL((k_conv_wgrad<1>), grid, dim3(64), 0, s, Rl, x, csx, cix, p.cin / 16, gzin, p.cout / 16, chunk, part);
+            hipLaunchKernelGGL((k_conv_wgrad<1>), grid, dim3(64), 0, s, Rl, x, csx, cix, p.cin / 16, gz, p.cout / 16, chunk, part);
         hipLaunchKernelGGL(k_reduce_parts, dim3(nblk(L[l].nw)), dim3(256), 0, s, L[l].nw, ns, part, L[l].gW);
-        hipLaunchKernelGGL(k_bias_grad, dim3(p.cout), dim3(256), 0, s, n, p.cout, gzin, L[l].gb);
-    }
-    void act_bwd(int l, const bf16 *y, int csy, int cy, const float *gy, int csg, int cg)
-    {
-        const NetLayerSpec &p = L[l].sp;
-        const long n = nv(p.lvl);
-        hipLaunchKernelGGL(k_act_bwd, dim3(nblk(n * p.cout)), dim3(256), 0, s, n, p.cout, y, csy, cy, gy, csg, cg, gz, p.relu);
+        hipLaunchKernelGGL(k_bias_grad, dim3(p.cout), dim3(256), 0, s, n, p.cout, gz, L[l].gb);
     }
     void pack()
     {
-        for (int l = 0; l < NET_NLAYER; l++) {
-            const NetLayerSpec &p = L[l].sp;
-            long n = (long)p.ntap * (p.cin / 16) * (p.cout / 16) * 64;
-            hipLaunchKernelGGL(k_pack_w, dim3(nblk(n)), dim3(256), 0, s, p.ntap, p.cin / 16, p.cout / 16, L[l].W, L[l].Wp, 0);
-            hipLaunchKernelGGL(k_pack_w, dim3(nblk(n)), dim3(256), 0, s, p.ntap, p.cin / 16, p.cout / 16, L[l].W, L[l].Wq, 1);
-        }
+        long m = 0;
+        for (int l = 0; l < NET_NLAYER; l++) m = std::max(m, L[l].nw / 4);
+        hipLaunchKernelGGL(k_pack_w, dim3(nblk(m), 2 * NET_NLAYER), dim3(256), 0, s, tab, par, wpk, wqk);
+    }
+    // the gradients of backward() from their segment sums, and the Adam step with train
+    void update(bool train, float lr, float b1, float b2, float eps, float c1, float c2)
+    {
+        long m = 0;
+        for (int l = 0; l < NET_NLAYER; l++) m = std::max(m, L[l].nw + L[l].sp.cout);
+        hipLaunchKernelGGL(k_update, dim3(nblk(m), NET_NLAYER), dim3(256), 0, s, tab, part2, grd, (int)train, par, mom, var,
+                           lr, b1, b2, eps, c1, c2);
     }
     void forward()
     {
@@ -760,45 +850,34 @@ struct NetImpl {
         conv_fwd(9, D1a, 16, 0, D1b, 16, 0, 0);
         conv_fwd(10, D1b, 16, 0, OUT, 16, 0, 1);
     }
-    // gradients of all parameters from gOUT (dL/dOUT)
+    // gradients of all parameters from gOUT (dL/dOUT), up to update()
     void backward()
     {
-        act_bwd(10, nullptr, 16, 0, gOUT, 16, 0);
-        conv_wgrad(10, D1b, 16, 0, gz);
+        layer_grad(10, nullptr, 16, 0, gOUT, 16, 0, D1b, 16, 0);
         conv_bwd_data(10, gz, gD1b, 16, 0);
-        act_bwd(9, D1b, 16, 0, gD1b, 16, 0);
-        conv_wgrad(9, D1a, 16, 0, gz);
+        layer_grad(9, D1b, 16, 0, gD1b, 16, 0, D1a, 16, 0);
         conv_bwd_data(9, gz, gD1a, 16, 0);
-        act_bwd(8, D1a, 16, 0, gD1a, 16, 0);
-        conv_wgrad(8, D1in, 48, 0, gz);
+        layer_grad(8, D1a, 16, 0, gD1a, 16, 0, D1in, 48, 0);
         conv_bwd_data(8, gz, gD1in, 48, 0);
         hipLaunchKernelGGL(k_up_bwd, dim3(nblk(nv1 * 32)), dim3(256), 0, s, R, 32, gD1in, 48, 0, gD2b);
-        act_bwd(7, D2b, 32, 0, gD2b, 32, 0);
-        conv_wgrad(7, D2a, 32, 0, gz);
+        layer_grad(7, D2b, 32, 0, gD2b, 32, 0, D2a, 32, 0);
         conv_bwd_data(7, gz, gD2a, 32, 0);
-        act_bwd(6, D2a, 32, 0, gD2a, 32, 0);
-        conv_wgrad(6, D2in, 96, 0, gz);
+        layer_grad(6, D2a, 32, 0, gD2a, 32, 0, D2in, 96, 0);
         conv_bwd_data(6, gz, gD2in, 96, 0);
         hipLaunchKernelGGL(k_up_bwd, dim3(nblk(nv2 * 64)), dim3(256), 0, s, R2, 64, gD2in, 96, 0, gE3b);
-        act_bwd(5, E3b, 64, 0, gE3b, 64, 0);
-        conv_wgrad(5, E3a, 64, 0, gz);
+        layer_grad(5, E3b, 64, 0, gE3b, 64, 0, E3a, 64, 0);
         conv_bwd_data(5, gz, gE3a, 64, 0);
-        act_bwd(4, E3a, 64, 0, gE3a, 64, 0);
-        conv_wgrad(4, P2, 32, 0, gz);
+        layer_grad(4, E3a, 64, 0, gE3a, 64, 0, P2, 32, 0);
         conv_bwd_data(4, gz, gP2, 32, 0);
         hipLaunchKernelGGL(k_pool_bwd, dim3(nblk(nv1 * 32)), dim3(256), 0, s, R4, 32, gP2, gD2in, 96, 64);
-        act_bwd(3, D2in, 96, 64, gD2in, 96, 64);
-        conv_wgrad(3, E2a, 32, 0, gz);
+        layer_grad(3, D2in, 96, 64, gD2in, 96, 64, E2a, 32, 0);
         conv_bwd_data(3, gz, gE2a, 32, 0);
-        act_bwd(2, E2a, 32, 0, gE2a, 32, 0);
-        conv_wgrad(2, P1, 16, 0, gz);
+        layer_grad(2, E2a, 32, 0, gE2a, 32, 0, P1, 16, 0);
         conv_bwd_data(2, gz, gP1, 16, 0);
         hipLaunchKernelGGL(k_pool_bwd, dim3(nblk(nv0 * 16)), dim3(256), 0, s, R2, 16, gP1, gD1in, 48, 32);
-        act_bwd(1, D1in, 48, 32, gD1in, 48, 32);
-        conv_wgrad(1, E1a, 16, 0, gz);
+        layer_grad(1, D1in, 48, 32, gD1in, 48, 32, E1a, 16, 0);
         conv_bwd_data(1, gz, gE1a, 16, 0);
-        act_bwd(0, E1a, 16, 0, gE1a, 16, 0);
-        conv_wgrad(0, X0, 16, 0, gz);
+        layer_grad(0, E1a, 16, 0, gE1a, 16, 0, X0, 16, 0);
     }
     double loss_of(const float *tg)
     {
@@ -844,22 +923,40 @@ NetImpl *net_create(int R, int max_samples, unsigned seed, hipStream_t s)
     n->maxs = max_samples;
     n->s = s;
     bool ok = true;
-    long maxparts = 0, wgparts = 0, wgx = 0, wgg = 0;
-    for (int l = 0; l < NET_NLAYER && ok; l++) {
+    long maxparts = 0, wgx = 0, wgg = 0;
+    NetTab &tb = n->tab;
+    long np2 = 0;
+    for (int l = 0; l < NET_NLAYER; l++) {
         Layer &L = n->L[l];
         L.sp = NET_SPEC[l];
         L.nw = (long)L.sp.ntap * L.sp.cin * L.sp.cout;
-        long np = (long)L.sp.ntap * (L.sp.cin / 16) * (L.sp.cout / 16) * 64;
-        ok = ok && n->alloc(&L.W, L.nw) && n->alloc(&L.b, L.sp.cout) && n->alloc(&L.mW, L.nw) && n->alloc(&L.vW, L.nw) &&
-             n->alloc(&L.mb, L.sp.cout) && n->alloc(&L.vb, L.sp.cout) && n->alloc(&L.gW, L.nw) &&
-             n->alloc(&L.gb, L.sp.cout) && n->alloc(&L.Wp, np) && n->alloc(&L.Wq, np);
-        if (L.nw > maxparts) maxparts = L.nw;
         const int Rl = R >> L.sp.lvl;
+        tb.ntap[l] = L.sp.ntap;
+        tb.ncib[l] = L.sp.cin / 16;
+        tb.ncob[l] = L.sp.cout / 16;
+        tb.off[l] = n->npar;
+        tb.pk[l] = n->npk;
+        tb.p2[l] = -1;
+        n->npar += L.nw + L.sp.cout;
+        n->npk += L.nw / 4;
         if (wg_staged_ok(Rl)) {
-            wgparts = std::max(wgparts, wg_plan(Rl, L.sp.cin, L.sp.cout).nsplit * L.nw);
+            tb.p2[l] = np2;
+            np2 += WG_G * (L.nw + L.sp.cout);
             wgx = std::max(wgx, wg_xs_elems(Rl, L.sp.cin));
             wgg = std::max(wgg, (long)Rl * Rl * Rl * L.sp.cout);
-        }
+        } else maxparts = std::max(maxparts, L.nw);
+    }
+    ok = n->alloc(&n->par, n->npar) && n->alloc(&n->mom, n->npar) && n->alloc(&n->var, n->npar) &&
+         n->alloc(&n->grd, n->npar) && n->alloc(&n->wpk, n->npk) && n->alloc(&n->wqk, n->npk) && n->alloc(&n->part2, np2);
+    for (int l = 0; l < NET_NLAYER && ok; l++) {
+        Layer &L = n->L[l];
+        L.W = n->par + tb.off[l];
+        L.b = L.W + L.nw;
+        L.gW = n->grd + tb.off[l];
+        L.gb = L.gW + L.nw;
+        if (tb.p2[l] >= 0) L.part2 = n->part2 + tb.p2[l];
+        L.Wp = n->wpk + tb.pk[l];
+        L.Wq = n->wqk + tb.pk[l];
     }
     const long v0 = n->nv0, v1 = n->nv1, v2 = n->nv2;
     ok = ok && n->alloc(&n->X0, v0 * 16) && n->alloc(&n->E1a, v0 * 16) && n->alloc(&n->D1in, v0 * 48) &&
@@ -872,8 +969,8 @@ NetImpl *net_create(int R, int max_samples, unsigned seed, hipStream_t s)
          n->alloc(&n->gD2in, v1 * 96) && n->alloc(&n->gE3b, v2 * 64) && n->alloc(&n->gE3a, v2 * 64) &&
          n->alloc(&n->gP2, v2 * 32) && n->alloc(&n->gE2a, v1 * 32) && n->alloc(&n->gP1, v1 * 16) &&
          n->alloc(&n->gE1a, v0 * 16);
-    ok = ok && n->alloc(&n->part, std::max(maxparts * n->nsplit, wgparts)) && n->alloc(&n->lpart, nblk(v0) + 1) &&
-         n->alloc(&n->wxs, wgx) && n->alloc(&n->wgs, wgg) && n->alloc(&n->part2, (long)WG_G * maxparts) &&
+    ok = ok && n->alloc(&n->part, maxparts * n->nsplit) && n->alloc(&n->lpart, (long)nblk(v0) * std::max(1, max_samples)) &&
+         n->alloc(&n->wxs, wgx) && n->alloc(&n->wgs, wgg) &&
          n->alloc(&n->feat, (long)(max_samples + 1) * v0 * 4) && n->alloc(&n->tgt_raw, (long)(max_samples + 1) * v0 * 4) &&
          n->alloc(&n->tgt, v0 * 4) && n->alloc(&n->scale, NET_NOUT);
     if (!ok) {
@@ -917,25 +1014,13 @@ long net_num_params(const NetImpl *n)
 
 int net_get_params(NetImpl *n, float *h)
 {
-    long o = 0;
-    for (int l = 0; l < NET_NLAYER; l++) {
-        hipMemcpyAsync(h + o, n->L[l].W, sizeof(float) * n->L[l].nw, hipMemcpyDeviceToHost, n->s);
-        o += n->L[l].nw;
-        hipMemcpyAsync(h + o, n->L[l].b, sizeof(float) * n->L[l].sp.cout, hipMemcpyDeviceToHost, n->s);
-        o += n->L[l].sp.cout;
-    }
+    hipMemcpyAsync(h, n->par, sizeof(float) * n->npar, hipMemcpyDeviceToHost, n->s);
     return hipStreamSynchronize(n->s) == hipSuccess ? 0 : -1;
 }
 
 int net_set_params(NetImpl *n, const float *h)
 {
-    long o = 0;
-    for (int l = 0; l < NET_NLAYER; l++) {
-        hipMemcpyAsync(n->L[l].W, h + o, sizeof(float) * n->L[l].nw, hipMemcpyHostToDevice, n->s);
-        o += n->L[l].nw;
-        hipMemcpyAsync(n->L[l].b, h + o, sizeof(float) * n->L[l].sp.cout, hipMemcpyHostToDevice, n->s);
-        o += n->L[l].sp.cout;
-    }
+    hipMemcpyAsync(n->par, h, sizeof(float) * n->npar, hipMemcpyHostToDevice, n->s);
     n->pack();
     return hipStreamSynchronize(n->s) == hipSuccess ? 0 : -1;
 }
@@ -1006,11 +1091,7 @@ static void adam_step(NetImpl *n, float lr)
     n->step++;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     const float c1 = 1.f - std::pow(b1, (float)n->step), c2 = 1.f - std::pow(b2, (float)n->step);
-    for (int l = 0; l < NET_NLAYER; l++) {
-        Layer &L = n->L[l];
-        hipLaunchKernelGGL(k_adam, dim3(nblk(L.nw)), dim3(256), 0, n->s, L.nw, L.W, L.gW, L.mW, L.vW, lr, b1, b2, eps, c1, c2);
-        hipLaunchKernelGGL(k_adam, dim3(nblk(L.sp.cout)), dim3(256), 0, n->s, (long)L.sp.cout, L.b, L.gb, L.mb, L.vb, lr, b1, b2, eps, c1, c2);
-    }
+    n->update(true, lr, b1, b2, eps, c1, c2);
     n->pack();
 }
 
@@ -1019,20 +1100,32 @@ int net_train(NetImpl *n, int epochs, float lr, double *loss)
     const int ns = net_num_samples(n);
     if (ns < 1) return -1;
     if (!n->scaled) set_scales(n);
-    double last = 0.0;
+    const unsigned nb = nblk(n->nv0);
     for (int e = 0; e < epochs; e++) {
-        double acc = 0.0;
         for (int q = 0; q < ns; q++) {
             hipLaunchKernelGGL(k_feat_pad, dim3(nblk(n->nv0 * 16)), dim3(256), 0, n->s, n->nv0, n->feat + (long)q * n->nv0 * 4, n->X0);
             hipLaunchKernelGGL(k_scale_targets, dim3(nblk(n->nv0 * 4)), dim3(256), 0, n->s, n->nv0 * 4, n->tgt_raw + (long)q * n->nv0 * 4, n->scale, n->tgt);
             n->forward();
-            acc += n->loss_of(n->tgt);
+            hipLaunchKernelGGL(k_loss, dim3(nb), dim3(256), 0, n->s, n->nv0, n->OUT, n->tgt, n->gOUT, n->lpart + (long)q * nb);
             n->backward();
             adam_step(n, lr);
         }
-        last = acc / ns;
     }
-    if (loss) *loss = last;
+    // the mean loss of the last epoch (read once here: a read per sample would drain the queue)
+    if (loss) {
+        std::vector<double> h((size_t)nb * ns);
+        double acc = 0.0;
+        if (epochs > 0) {
+            hipMemcpyAsync(h.data(), n->lpart, sizeof(double) * h.size(), hipMemcpyDeviceToHost, n->s);
+            hipStreamSynchronize(n->s);
+            for (int q = 0; q < ns; q++) {
+                double t = 0.0;
+                for (unsigned b = 0; b < nb; b++) t += h[(size_t)q * nb + b];
+                acc += t;
+            }
+        }
+        *loss = acc / ns;
+    }
     return hipStreamSynchronize(n->s) == hipSuccess ? 0 : -1;
 }
 
@@ -1055,15 +1148,10 @@ int net_grad_host(NetImpl *n, const float *feat, const float *tgt, double *loss,
     n->forward();
     double L = n->loss_of(dt);
     n->backward();
+    n->update(false, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f);
     if (loss) *loss = L;
     if (out) hipMemcpyAsync(out, n->OUT, sizeof(float) * n->nv0 * 16, hipMemcpyDeviceToHost, n->s);
-    long o = 0;
-    for (int l = 0; l < NET_NLAYER; l++) {
-        hipMemcpyAsync(grad + o, n->L[l].gW, sizeof(float) * n->L[l].nw, hipMemcpyDeviceToHost, n->s);
-        o += n->L[l].nw;
-        hipMemcpyAsync(grad + o, n->L[l].gb, sizeof(float) * n->L[l].sp.cout, hipMemcpyDeviceToHost, n->s);
-        o += n->L[l].sp.cout;
-    }
+    hipMemcpyAsync(grad, n->grd, sizeof(float) * n->npar, hipMemcpyDeviceToHost, n->s);
     return hipStreamSynchronize(n->s) == hipSuccess ? 0 : -1;
 }
 
@@ -1091,8 +1179,11 @@ int net_conv_test(int R, int ntap, int cin, int cout, int relu, int mode, const 
     float *part = (float *)A(nw * nsplit * 4);
     hipMemcpy(dw, w, nw * 4, hipMemcpyHostToDevice);
     if (bias) hipMemcpy(db, bias, cout * 4, hipMemcpyHostToDevice);
-    hipLaunchKernelGGL(k_pack_w, dim3(nblk(np)), dim3(256), 0, s, ntap, cin / 16, cout / 16, dw, Wp, 0);
-    hipLaunchKernelGGL(k_pack_w, dim3(nblk(np)), dim3(256), 0, s, ntap, cin / 16, cout / 16, dw, Wq, 1);
+    NetTab tb{};
+    tb.ntap[0] = ntap;
+    tb.ncib[0] = cin / 16;
+    tb.ncob[0] = cout / 16;
+    hipLaunchKernelGGL(k_pack_w, dim3(nblk(np), 2), dim3(256), 0, s, tb, dw, Wp, Wq);
     if (mode == 0 || mode == 2) {
         hipMemcpy(din, in, nv * cin * 4, hipMemcpyHostToDevice);
         hipLaunchKernelGGL((k_cvt_bf16<float>), dim3(nblk(nv * cin)), dim3(256), 0, s, nv * cin, (const float *)din, bin);
@@ -1103,20 +1194,22 @@ int net_conv_test(int R, int ntap, int cin, int cout, int relu, int mode, const 
     }
     if (mode == 0) {
         dim3 grid(nblk(nv, 64), cout / 16);
-        if (ntap == 27 && relu) hipLaunchKernelGGL((k_conv<27, 1, true>), grid, dim3(256), 0, s, R, bin, cin, 0, cin / 16, Wp, db, (void *)dout, cout, 0, cout / 16);
-        else if (ntap == 27) hipLaunchKernelGGL((k_conv<27, 1, false>), grid, dim3(256), 0, s, R, bin, cin, 0, cin / 16, Wp, db, (void *)dout, cout, 0, cout / 16);
-        else hipLaunchKernelGGL((k_conv<1, 1, false>), grid, dim3(256), 0, s, R, bin, cin, 0, cin / 16, Wp, db, (void *)dout, cout, 0, cout / 16);
+        if (ntap == 27 && relu) conv27<1, true>(grid, R, bin, cin, 0, cin / 16, Wp, db, dout, cout, 0, cout / 16, s);
+        else if (ntap == 27) conv27<1, false>(grid, R, bin, cin, 0, cin / 16, Wp, db, dout, cout, 0, cout / 16, s);
+        else hipLaunchKernelGGL((k_conv<1, 0, 1, false>), grid, dim3(256), 0, s, R, bin, cin, 0, cin / 16, Wp, db, (void *)dout, cout, 0, cout / 16);
         hipMemcpy(out, dout, nv * cout * 4, hipMemcpyDeviceToHost);
     } else if (mode == 1) {
         dim3 grid(nblk(nv, 64), cin / 16);
-        if (ntap == 27) hipLaunchKernelGGL((k_conv<27, 1, false>), grid, dim3(256), 0, s, R, bgo, cout, 0, cout / 16, Wq, (const float *)nullptr, (void *)dout, cin, 0, cin / 16);
-        else hipLaunchKernelGGL((k_conv<1, 1, false>), grid, dim3(256), 0, s, R, bgo, cout, 0, cout / 16, Wq, (const float *)nullptr, (void *)dout, cin, 0, cin / 16);
+        if (ntap == 27) conv27<1, false>(grid, R, bgo, cout, 0, cout / 16, Wq, nullptr, dout, cin, 0, cin / 16, s);
+        else hipLaunchKernelGGL((k_conv<1, 0, 1, false>), grid, dim3(256), 0, s, R, bgo, cout, 0, cout / 16, Wq, (const float *)nullptr, (void *)dout, cin, 0, cin / 16);
         hipMemcpy(out, dout, nv * cin * 4, hipMemcpyDeviceToHost);
     } else if (wg_staged_ok(R)) {
         bf16 *xs = (bf16 *)A(wg_xs_elems(R, cin) * 2), *gs = (bf16 *)A(nv * cout * 2);
-        float *wpart = (float *)A(wg_plan(R, cin, cout).nsplit * nw * 4);
-        float *wpart2 = (float *)A((long)WG_G * (nw > cout ? nw : cout) * 4);
-        wgrad_staged(R, ntap, cin, cout, bin, cin, 0, bgo, xs, gs, wpart, wpart2, dgw, dgb, s);
+        float *wpart2 = (float *)A((long)WG_G * (nw + cout) * 4), *dg = (float *)A((nw + cout) * 4);
+        wgrad_staged(R, ntap, cin, cout, bin, cin, 0, nullptr, 0, 0, dgo, cout, 0, 0, bgo, xs, gs, wpart2, s);
+        hipLaunchKernelGGL(k_update, dim3(nblk(nw + cout), 1), dim3(256), 0, s, tb, wpart2, dg, 0, dg, dg, dg, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f);
+        dgw = dg;
+        dgb = dg + nw;
         hipMemcpy(gw, dgw, nw * 4, hipMemcpyDeviceToHost);
         hipMemcpy(gb, dgb, cout * 4, hipMemcpyDeviceToHost);
     } else {

@@ -164,3 +164,10 @@ def test_residual_gate_never_loses_to_the_warm_start(make_solver):
             assert f["relres0"] <= sk["relres0"] * (1 + 1e-3) + 1e-7, (it, f["relres0"], sk["relres0"])
         a.record_sample()
         a.net_train(20, 1e-3)
+
+
+@pytest.mark.parametrize("R,cin,cout", [(12, 80, 16), (20, 48, 32), (5, 64, 16), (36, 16, 16)])
+def test_conv_layer_at_other_grids_and_channels(orc, R, cin, cout):
+    """Channel counts without a kernel of their own (80), grids whose last run of voxel
+    groups is short (20, 36: 1 to 64 runs a segment) or that are not staged (5)."""
+    test_conv_layer_matches_oracle(orc, R, 27, cin, cout, 1)
