@@ -101,7 +101,8 @@ void launch_oc_apply(long n, const double *rho, const double *base, const double
                      double rho_min, double *rn, double *part, hipStream_t);
 unsigned absmax_blocks(long n);
 void launch_absdiff_max(long n, const double *a, const double *b, double *part, hipStream_t);
-void launch_sum(int np, int nvec, const double *part, double *out, hipStream_t);
+void launch_sum(int np, int nvec, const double *part, double *out, hipStream_t s, double *hout = nullptr,
+                const double *hsrc = nullptr, double *hdst = nullptr);
 unsigned blas_blocks(long n);
 template <typename TA, typename TB> void launch_dot(long n, const TA *a, const TB *b, double *part, hipStream_t);
 template <typename TW, typename TV>

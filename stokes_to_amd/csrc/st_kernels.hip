@@ -817,14 +817,21 @@ __global__ void __launch_bounds__(256) k_absdiff_max(long n, const double *a, co
 
 // sum of partials in fixed order (one block)
 // out[v] = sum of the np partials of vector v; one workgroup per vector (grid nvec)
-__global__ void __launch_bounds__(1024) k_sum(int np, const double *part, double *out)
+// hout: a copy of out in pinned host memory; hsrc, hdst: one value per sum fetched from
+// there on the way (what a small transfer each way took 10 to 20 us for)
+__global__ void __launch_bounds__(1024) k_sum(int np, const double *part, double *out, double *hout, const double *hsrc,
+                                              double *hdst)
 {
     __shared__ double sh[16];
     const int v = blockIdx.x;
     double a = 0.0;
     for (int q = threadIdx.x; q < np; q += blockDim.x) a += part[(long)v * np + q];
     const double s = block_sum(a, sh);
-    if (threadIdx.x == 0) out[v] = s;
+    if (threadIdx.x == 0) {
+        out[v] = s;
+        if (hout) hout[v] = s;
+        if (hsrc) hdst[v] = hsrc[v];
+    }
 }
 
 template <typename TA, typename TB>
@@ -1246,10 +1253,11 @@ void launch_absdiff_max(long n, const double *a, const double *b, double *part, 
 {
     hipLaunchKernelGGL(k_absdiff_max, dim3(nb_grid(n)), dim3(256), 0, s, n, a, b, part);
 }
-void launch_sum(int np, int nvec, const double *part, double *out, hipStream_t s)
+void launch_sum(int np, int nvec, const double *part, double *out, hipStream_t s, double *hout, const double *hsrc,
+                double *hdst)
 {
     if (nvec < 1) return;
-    hipLaunchKernelGGL(k_sum, dim3((unsigned)nvec), dim3(1024), 0, s, np, part, out);
+    hipLaunchKernelGGL(k_sum, dim3((unsigned)nvec), dim3(1024), 0, s, np, part, out, hout, hsrc, hdst);
 }
 unsigned blas_blocks(long n) { return nb_grid(n); }
 template <typename TA, typename TB>

@@ -188,13 +188,12 @@ MmaDev *mma_create(long n, hipStream_t s)
         *arr[a] = (double *)p;
     }
     void *p = nullptr, *q = nullptr;
-    if (hipMalloc(&p, sizeof(double) * 2 * MMA_NB) != hipSuccess || hipMalloc(&q, sizeof(double) * 2) != hipSuccess) {
+    if (hipMalloc(&p, sizeof(double) * 2 * MMA_NB) != hipSuccess || hipHostMalloc(&q, sizeof(double) * 2, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
         if (p) hipFree(p);
         mma_destroy(m);
         return nullptr;
     }
     m->al.push_back(p);
-    m->al.push_back(q);
     m->part = (double *)p;
     m->red = (double *)q;
     return m;
@@ -204,6 +203,7 @@ void mma_destroy(MmaDev *m)
 {
     if (!m) return;
     for (void *p : m->al) hipFree(p);
+    if (m->red) hipHostFree(m->red);
     delete m;
 }
 
@@ -223,11 +223,9 @@ static int mma_nb(long n)
 static int mma_sums(MmaDev *m, double *g, double *h)
 {
     hipLaunchKernelGGL(k_mma_sum2, dim3(1), dim3(256), 0, m->s, mma_nb(m->n), m->part, m->red);
-    double r[2];
-    if (hipMemcpyAsync(r, m->red, sizeof(r), hipMemcpyDeviceToHost, m->s) != hipSuccess) return -1;
-    if (hipStreamSynchronize(m->s) != hipSuccess) return -1;
-    *g = r[0];
-    if (h) *h = r[1];
+    if (hipStreamSynchronize(m->s) != hipSuccess) return -1;  // red is pinned host memory
+    *g = m->red[0];
+    if (h) *h = m->red[1];
     return 0;
 }
 

@@ -11,11 +11,13 @@
 //    iteration cross PCIe (the reference copies two full vectors per iteration
 //    and orthogonalises on the host, CX/GMRES.cpp:46-95).
 #include "../../include/stokes_to.h"
+#include "st_hostcopy.h"
 #include "st_kernels.h"
 #include "st_mma.h"
 #include "st_net.h"
 
 #include <cmath>
+#include <limits>
 #include <cstdio>
 #include <cstring>
 #include <string>
@@ -55,7 +57,11 @@ struct st_ctx {
     long ndof = 0, ncell = 0, nvec = 0;  // ABI sizes and padded vector length
     double *X = nullptr, *B = nullptr, *XD = nullptr, *BODY = nullptr, *LAM = nullptr, *BA = nullptr, *ZERO = nullptr;
     double *Wv = nullptr, *V = nullptr, *Zb = nullptr;
-    double *part = nullptr, *red = nullptr, *h_dev = nullptr, *sig2_dev = nullptr;
+    double *part = nullptr, *h_dev = nullptr, *sig2_dev = nullptr;
+    // scalars in pinned host memory that kernels write and read: sums for the host, the
+    // Arnoldi column, the coefficients of the update and the squared scales of the basis
+    double *red = nullptr, *h_host = nullptr, *y_host = nullptr, *sig2_host = nullptr;
+    HostCopy hc;
     int npart = 0;
     // design
     double *rho = nullptr, *rhof = nullptr, *dj = nullptr, *dc = nullptr, *rn = nullptr, *fW = nullptr, *dv = nullptr;
@@ -204,8 +210,8 @@ static int dot64(st_ctx *c, const double *a, const double *b, long n, double *re
 {
     launch_dot<double, double>(n, a, b, c->part, c->s);
     launch_sum((int)blas_blocks(n), 1, c->part, c->red, c->s);
-    CK(hipMemcpyAsync(res, c->red, sizeof(double), hipMemcpyDeviceToHost, c->s));
     CK(hipStreamSynchronize(c->s));
+    *res = c->red[0];
     return ST_OK;
 }
 
@@ -508,8 +514,9 @@ template <typename TV, typename TW> static int fgmres(st_ctx *c, const double *b
     double bn = std::sqrt(bn2);
     if (!std::isfinite(bn)) return fail(c, ST_ENAN, "non-finite right-hand side");
     if (bn == 0.0) bn = 1.0;
-    std::vector<double> H((size_t)(m + 1) * m, 0.0), cs(m), sn(m), gv(m + 1), y(m), hh(m + 2);
-    std::vector<double> sig(m + 1, 1.0), sig2(m + 1, 1.0);
+    std::vector<double> H((size_t)(m + 1) * m, 0.0), cs(m), sn(m), gv(m + 1);
+    std::vector<double> sig(m + 1, 1.0);
+    double *const hh = c->h_host, *const y = c->y_host, *const sig2 = c->sig2_host;
     int it = 0;
     double rr = 0.0, rr0 = -1.0;
     const bool plain = std::is_same<TV, double>::value;
@@ -527,8 +534,8 @@ template <typename TV, typename TW> static int fgmres(st_ctx *c, const double *b
             else launch_residual<double>(g, c->fl[0], c->h64.al[0], b, x, r0, c->part, c->s);
             launch_sum(rb, 1, c->part, c->red, c->s);
             double r2 = 0.0;
-            CK(hipMemcpyAsync(&r2, c->red, sizeof(double), hipMemcpyDeviceToHost, c->s));
             CK(hipStreamSynchronize(c->s));
+            r2 = c->red[0];
             beta = std::sqrt(r2);
         }
         if (!std::isfinite(beta)) return fail(c, ST_ENAN, "non-finite residual");
@@ -538,7 +545,6 @@ template <typename TV, typename TW> static int fgmres(st_ctx *c, const double *b
         if (LAZY) {
             sig[0] = 1.0 / beta;
             sig2[0] = sig[0] * sig[0];
-            CK(hipMemcpyAsync(c->sig2_dev, sig2.data(), sizeof(double), hipMemcpyHostToDevice, c->s));
             if (!std::is_same<TV, double>::value && !r_f32) launch_axpby<double, TV>(nv, 1.0, r0, 0.0, Vb, c->s);
         } else {
             launch_axpby<double, TV>(nv, 1.0 / beta, r0, 0.0, Vb, c->s);
@@ -556,10 +562,9 @@ template <typename TV, typename TW> static int fgmres(st_ctx *c, const double *b
             prof_mark(c, ST_PROF_APPLY);
             const unsigned nbk = blas_blocks(nv);
             launch_multidot<TW, TV>(nv, w, Vb, nv, j + 1, c->part, c->s);
-            launch_sum((int)nbk, j + 1, c->part, c->h_dev, c->s);
+            launch_sum((int)nbk, j + 1, c->part, c->h_dev, c->s, hh, LAZY ? c->sig2_host : nullptr, c->sig2_dev);
             launch_multiaxpy<TW, TV>(nv, w, Vb, nv, j + 1, c->h_dev, LAZY ? c->sig2_dev : nullptr, c->part, c->s);
-            launch_sum((int)nbk, 1, c->part, c->h_dev + (j + 1), c->s);
-            CK(hipMemcpyAsync(hh.data(), c->h_dev, sizeof(double) * (j + 2), hipMemcpyDeviceToHost, c->s));
+            launch_sum((int)nbk, 1, c->part, hh + (j + 1), c->s);
             CK(hipStreamSynchronize(c->s));
             const double un = std::sqrt(hh[j + 1]);  // |u_{j+1}| (LAZY) or |w|
             if (!std::isfinite(un)) return fail(c, ST_ENAN, "non-finite Arnoldi vector");
@@ -573,7 +578,6 @@ template <typename TV, typename TW> static int fgmres(st_ctx *c, const double *b
                     sig[j + 1] = 1.0;
                 }
                 sig2[j + 1] = sig[j + 1] * sig[j + 1];
-                CK(hipMemcpyAsync(c->sig2_dev + (j + 1), &sig2[j + 1], sizeof(double), hipMemcpyHostToDevice, c->s));
             } else if (hn > 0) {
                 launch_axpby<TW, TV>(nv, 1.0 / hn, Wk, 0.0, Vb + (long)(j + 1) * nv, c->s);
             }
@@ -602,7 +606,7 @@ template <typename TV, typename TW> static int fgmres(st_ctx *c, const double *b
             y[i] = sacc / H[(size_t)i * m + i];
         }
         for (int i = 0; i < j; i++) y[i] = LAZY ? -y[i] * sig[i] : -y[i];
-        CK(hipMemcpyAsync(c->h_dev, y.data(), sizeof(double) * j, hipMemcpyHostToDevice, c->s));
+        CK(hipMemcpyAsync(c->h_dev, y, sizeof(double) * j, hipMemcpyHostToDevice, c->s));
         launch_multiaxpy<double, TV>(nv, x, Zs, nv, j, c->h_dev, nullptr, nullptr, c->s);
     }
     if (st) {
@@ -619,20 +623,23 @@ template <typename TV, typename TW> static int fgmres(st_ctx *c, const double *b
 
 static int stage_in(st_ctx *c, const double *h, long n)
 {
-    CK(hipMemcpyAsync(c->abi_a, h, sizeof(double) * n, hipMemcpyHostToDevice, c->s));
+    CK(c->hc.in(c->abi_a, h, sizeof(double) * n, c->s));
     return ST_OK;
 }
 static int stage_out(st_ctx *c, double *h, long n)
 {
-    CK(hipMemcpyAsync(h, c->abi_b, sizeof(double) * n, hipMemcpyDeviceToHost, c->s));
-    CK(hipStreamSynchronize(c->s));
+    CK(c->hc.out(h, c->abi_b, sizeof(double) * n, c->s));
     return ST_OK;
 }
 
 static int check_finite(st_ctx *c, const double *h, long n, const char *what)
 {
-    for (long q = 0; q < n; q++)
-        if (!std::isfinite(h[q])) return fail(c, ST_ENAN, std::string("non-finite value in ") + what);
+    for (long q0 = 0; q0 < n; q0 += 4096) {  // (without a branch per value the blocks vectorise)
+        const long q1 = std::min(n, q0 + 4096);
+        bool bad = false;
+        for (long q = q0; q < q1; q++) bad |= !(std::fabs(h[q]) <= std::numeric_limits<double>::max());
+        if (bad) return fail(c, ST_ENAN, std::string("non-finite value in ") + what);
+    }
     return ST_OK;
 }
 
@@ -763,7 +770,14 @@ int st_create(st_ctx **out, const st_params *p)
     // or of the objective (more than that from 512^3 and 2D 16384^2)
     c->npart = std::max(8192 * 33, (int)std::max(std::max(residual_blocks(g0), plain_residual_blocks(g0)), energy_blocks(g0)));
     if (rc == ST_OK) rc = dalloc(c, &c->part, c->npart);
-    if (rc == ST_OK) rc = dalloc(c, &c->red, 64);
+    if (rc == ST_OK && hipHostMalloc((void **)&c->red, sizeof(double) * 4 * 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
+        rc = fail(c, ST_EHIP, "cannot allocate pinned memory");
+    if (rc == ST_OK) {
+        c->h_host = c->red + 64;
+        c->y_host = c->red + 128;
+        c->sig2_host = c->red + 192;
+        c->hc.prepare(sizeof(double) * c->ndof);
+    }
     if (rc == ST_OK) rc = dalloc(c, &c->h_dev, 64);
     if (rc == ST_OK) rc = dalloc(c, &c->sig2_dev, 64);
     for (double **pp : {&c->rho, &c->rhof, &c->dj, &c->dc, &c->rn, &c->fW, &c->dv, &c->tmpc})
@@ -809,6 +823,7 @@ void st_destroy(st_ctx *c)
     if (c->net) net_destroy(c->net);
     if (c->mma) mma_destroy(c->mma);
     for (void *q : c->allocs) hipFree(q);
+    if (c->red) hipHostFree(c->red);
     if (c->e0) hipEventDestroy(c->e0);
     if (c->e1) hipEventDestroy(c->e1);
     if (c->e2) hipEventDestroy(c->e2);
@@ -891,7 +906,7 @@ int st_set_design(st_ctx *c, const double *rho)
     if (!c || !rho) return ST_EINVAL;
     if (!c->geom) return fail(c, ST_ESTATE, "st_set_geometry must precede st_set_design");
     CKR(check_finite(c, rho, c->ncell, "design"));
-    CK(hipMemcpyAsync(c->rho, rho, sizeof(double) * c->ncell, hipMemcpyHostToDevice, c->s));
+    CK(c->hc.in(c->rho, rho, sizeof(double) * c->ncell, c->s));
     design_to_alpha(c, c->rho);
     CK(hipStreamSynchronize(c->s));
     return ST_OK;
@@ -953,8 +968,7 @@ int st_profile_read(st_ctx *c, int kind, double *total_ms, long *launches, doubl
 int st_get_design(st_ctx *c, double *rho)
 {
     if (!c || !rho) return ST_EINVAL;
-    CK(hipMemcpyAsync(rho, c->rho, sizeof(double) * c->ncell, hipMemcpyDeviceToHost, c->s));
-    CK(hipStreamSynchronize(c->s));
+    CK(c->hc.out(rho, c->rho, sizeof(double) * c->ncell, c->s));
     return ST_OK;
 }
 
@@ -1087,8 +1101,8 @@ static int warm_mr(st_ctx *c, const double *b, double **xp, double **h, int &nh,
         launch_mr_gram(nd, nv, y, nv, u0, c->part, c->s);
         launch_sum(nbk, nq, c->part, c->red, c->s);
         double q[9];
-        CK(hipMemcpyAsync(q, c->red, sizeof(double) * nq, hipMemcpyDeviceToHost, c->s));
         CK(hipStreamSynchronize(c->s));
+        std::copy(c->red, c->red + nq, q);
         // G d = g (G symmetric positive semi-definite) by elimination in order; a pivot
         // below 1e-12 of the largest diagonal marks a (near-)dependent direction, which
         // gets a zero coefficient
@@ -1127,8 +1141,8 @@ static int warm_mr(st_ctx *c, const double *b, double **xp, double **h, int &nh,
             updated = true;
             launch_sum(nbk, 1, c->part, c->red, c->s);
             double rr = 0.0;
-            CK(hipMemcpyAsync(&rr, c->red, sizeof(double), hipMemcpyDeviceToHost, c->s));
             CK(hipStreamSynchronize(c->s));
+            rr = c->red[0];
             r0 = std::sqrt(rr);
             take = std::isfinite(r0) && r0 < r1;
         }
@@ -1267,8 +1281,8 @@ static int resid_norm_u0(st_ctx *c, const double *b, const double *x, double *nr
     march_residual_f32(g, c->fl[0], c->h64.al[0], b, x, reinterpret_cast<float *>(c->V), c->part, c->s);
     launch_sum((int)residual_blocks(g), 1, c->part, c->red, c->s);
     double r2 = 0.0;
-    CK(hipMemcpyAsync(&r2, c->red, sizeof(double), hipMemcpyDeviceToHost, c->s));
     CK(hipStreamSynchronize(c->s));
+    r2 = c->red[0];
     *nrm = std::sqrt(r2);
     return ST_OK;
 }
@@ -1280,8 +1294,8 @@ static int resid_norm(st_ctx *c, const double *b, const double *x, double *nrm)
     launch_residual<double>(g, c->fl[0], c->h64.al[0], b, x, (double *)nullptr, c->part, c->s);
     launch_sum((int)residual_blocks(g), 1, c->part, c->red, c->s);
     double r2 = 0.0;
-    CK(hipMemcpyAsync(&r2, c->red, sizeof(double), hipMemcpyDeviceToHost, c->s));
     CK(hipStreamSynchronize(c->s));
+    r2 = c->red[0];
     *nrm = std::sqrt(r2);
     return ST_OK;
 }
@@ -1430,8 +1444,7 @@ int st_get_gradient(st_ctx *c, double *dc)
 {
     if (!c || !dc) return ST_EINVAL;
     if (!c->have_grad) return fail(c, ST_ESTATE, "no design gradient yet (st_to_step)");
-    CK(hipMemcpyAsync(dc, c->dc, sizeof(double) * c->ncell, hipMemcpyDeviceToHost, c->s));
-    CK(hipStreamSynchronize(c->s));
+    CK(c->hc.out(dc, c->dc, sizeof(double) * c->ncell, c->s));
     return ST_OK;
 }
 
@@ -1477,8 +1490,8 @@ static int objective_dev(st_ctx *c, const double *x, double *y, double *J)
     launch_energy(g, c->fl[0], c->h64.al[0], x, y, c->part, c->s);
     launch_sum((int)energy_blocks(g), 1, c->part, c->red, c->s);
     double s = 0.0;
-    CK(hipMemcpyAsync(&s, c->red, sizeof(double), hipMemcpyDeviceToHost, c->s));
     CK(hipStreamSynchronize(c->s));
+    s = c->red[0];
     if (J) *J = 0.5 * s;
     return ST_OK;
 }
@@ -1507,14 +1520,13 @@ int st_sensitivity(st_ctx *c, const double *rho, const double *x, const double *
 {
     if (!c || !rho || !x || !lam || !dj) return ST_EINVAL;
     if (!c->geom) return fail(c, ST_ESTATE, "geometry must be set");
-    CK(hipMemcpyAsync(c->rn, rho, sizeof(double) * c->ncell, hipMemcpyHostToDevice, c->s));
+    CK(c->hc.in(c->rn, rho, sizeof(double) * c->ncell, c->s));
     CKR(stage_in(c, x, c->ndof));
     launch_pack<double>(c->lv[0], c->abi_a, c->Wv, 0, c->fl[0], 1.0, c->s);
     CKR(stage_in(c, lam, c->ndof));
     launch_pack<double>(c->lv[0], c->abi_a, c->BA, 0, c->fl[0], 1.0, c->s);
     launch_sensitivity(c->lv[0], c->rn, alpha_params(c), c->fl[0], c->Wv, c->BA, c->dj, c->s);
-    CK(hipMemcpyAsync(dj, c->dj, sizeof(double) * c->ncell, hipMemcpyDeviceToHost, c->s));
-    CK(hipStreamSynchronize(c->s));
+    CK(c->hc.out(dj, c->dj, sizeof(double) * c->ncell, c->s));
     return ST_OK;
 }
 
@@ -1530,10 +1542,9 @@ int st_filter(st_ctx *c, const double *in, double *out, int transpose)
 {
     if (!c || !in || !out) return ST_EINVAL;
     c->have_grad = false;  // c->dc is reused below
-    CK(hipMemcpyAsync(c->rn, in, sizeof(double) * c->ncell, hipMemcpyHostToDevice, c->s));
+    CK(c->hc.in(c->rn, in, sizeof(double) * c->ncell, c->s));
     filter_dev(c, c->rn, c->dc, transpose);
-    CK(hipMemcpyAsync(out, c->dc, sizeof(double) * c->ncell, hipMemcpyDeviceToHost, c->s));
-    CK(hipStreamSynchronize(c->s));
+    CK(c->hc.out(out, c->dc, sizeof(double) * c->ncell, c->s));
     return ST_OK;
 }
 
@@ -1588,8 +1599,8 @@ static int oc_dev(st_ctx *c, const double *rho, const double *dc, double volfrac
         }
         launch_oc_vols(n, rho, base, c->dv, f, move, rho_min, c->part, c->s);
         launch_sum(gb, OC_K, c->part, c->red, c->s);
-        CK(hipMemcpyAsync(vk, c->red, sizeof(double) * OC_K, hipMemcpyDeviceToHost, c->s));
         CK(hipStreamSynchronize(c->s));
+        std::copy(c->red, c->red + OC_K, vk);
         int k = 0;
         while (k < OC_K && vk[k] > volfrac) k++;
         if (k > 0) {
@@ -1607,12 +1618,11 @@ static int oc_dev(st_ctx *c, const double *rho, const double *dc, double volfrac
     c->oc_lambda = 0.5 * (l1 + l2);
     launch_oc_apply(n, rho, base, c->dv, std::pow(0.5 * (l1 + l2), -eta), move, rho_min, rn, c->part, c->s);
     launch_sum(gb, 1, c->part, c->red, c->s);
-    CK(hipMemcpyAsync(&vol, c->red, sizeof(double), hipMemcpyDeviceToHost, c->s));
-    CK(hipStreamSynchronize(c->s));
     launch_absdiff_max(n, rn, rho, c->part, c->s);
     std::vector<double> pm(absmax_blocks(n));
     CK(hipMemcpyAsync(pm.data(), c->part, sizeof(double) * pm.size(), hipMemcpyDeviceToHost, c->s));
     CK(hipStreamSynchronize(c->s));
+    vol = c->red[0];
     double ch = 0.0;
     for (double v : pm) ch = v > ch ? v : ch;
     if (change) *change = ch;
@@ -1625,11 +1635,10 @@ int st_oc_update(st_ctx *c, const double *rho, const double *dcp, double volfrac
 {
     if (!c || !rho || !dcp || !rho_new) return ST_EINVAL;
     c->have_grad = false;  // c->dc is reused below
-    CK(hipMemcpyAsync(c->rn, rho, sizeof(double) * c->ncell, hipMemcpyHostToDevice, c->s));
-    CK(hipMemcpyAsync(c->dc, dcp, sizeof(double) * c->ncell, hipMemcpyHostToDevice, c->s));
+    CK(c->hc.in(c->rn, rho, sizeof(double) * c->ncell, c->s));
+    CK(c->hc.in(c->dc, dcp, sizeof(double) * c->ncell, c->s));
     CKR(oc_dev(c, c->rn, c->dc, volfrac, move, eta, rho_min, c->dj, change, nullptr));
-    CK(hipMemcpyAsync(rho_new, c->dj, sizeof(double) * c->ncell, hipMemcpyDeviceToHost, c->s));
-    CK(hipStreamSynchronize(c->s));
+    CK(c->hc.out(rho_new, c->dj, sizeof(double) * c->ncell, c->s));
     return ST_OK;
 }
 
@@ -1654,16 +1663,15 @@ int st_mma_update(st_ctx *c, double *x, const double *dfdx, double g, const doub
     CKR(mma_ready(c));
     c->have_grad = false;  // c->dc is reused below
     const size_t nb = sizeof(double) * c->ncell;
-    CK(hipMemcpyAsync(c->rn, x, nb, hipMemcpyHostToDevice, c->s));
-    CK(hipMemcpyAsync(c->dc, dfdx, nb, hipMemcpyHostToDevice, c->s));
-    CK(hipMemcpyAsync(c->mdg, dgdx, nb, hipMemcpyHostToDevice, c->s));
-    CK(hipMemcpyAsync(c->mlo, xmin, nb, hipMemcpyHostToDevice, c->s));
-    CK(hipMemcpyAsync(c->mhi, xmax, nb, hipMemcpyHostToDevice, c->s));
+    CK(c->hc.in(c->rn, x, nb, c->s));
+    CK(c->hc.in(c->dc, dfdx, nb, c->s));
+    CK(c->hc.in(c->mdg, dgdx, nb, c->s));
+    CK(c->hc.in(c->mlo, xmin, nb, c->s));
+    CK(c->hc.in(c->mhi, xmax, nb, c->s));
     int r = mma_update(c->mma, c->rn, c->dc, g, c->mdg, c->mlo, c->mhi, newton_steps);
     if (r == -2) return fail(c, ST_ENAN, "MMA dual iteration produced a non-finite value");
     if (r != 0) return fail(c, ST_EHIP, "MMA update failed");
-    CK(hipMemcpyAsync(x, c->rn, nb, hipMemcpyDeviceToHost, c->s));
-    CK(hipStreamSynchronize(c->s));
+    CK(c->hc.out(x, c->rn, nb, c->s));
     return ST_OK;
 }
 
@@ -1687,8 +1695,8 @@ static int mma_dev(st_ctx *c, const double *rho, const double *dc, double volfra
     double vol = 0.0;
     launch_dot<double, double>(n, rho, c->dv, c->part, c->s);
     launch_sum((int)blas_blocks(n), 1, c->part, c->red, c->s);
-    CK(hipMemcpyAsync(&vol, c->red, sizeof(double), hipMemcpyDeviceToHost, c->s));
     CK(hipStreamSynchronize(c->s));
+    vol = c->red[0];
     const double coef = 1e4;
     launch_axpby<double, double>(n, coef, c->dv, 0.0, c->mdg, c->s);
     launch_mma_box(n, rho, move, rho_min, 1.0, c->mlo, c->mhi, c->s);
@@ -1702,8 +1710,8 @@ static int mma_dev(st_ctx *c, const double *rho, const double *dc, double volfra
     launch_dot<double, double>(n, rn, c->dv, c->part + pm.size(), c->s);
     launch_sum((int)blas_blocks(n), 1, c->part + pm.size(), c->red, c->s);
     double vn = 0.0;
-    CK(hipMemcpyAsync(&vn, c->red, sizeof(double), hipMemcpyDeviceToHost, c->s));
     CK(hipStreamSynchronize(c->s));
+    vn = c->red[0];
     double ch = 0.0;
     for (double v : pm) ch = v > ch ? v : ch;
     if (change) *change = ch;

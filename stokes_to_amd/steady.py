@@ -85,7 +85,7 @@ class FluidSteadyState:
         self._check(self.lib.st_set_design(self.h, dptr(rho)))
 
     def get_design(self):
-        out = np.zeros(self.ncell)
+        out = np.empty(self.ncell)
         self._check(self.lib.st_get_design(self.h, dptr(out)))
         return out
 
@@ -103,7 +103,7 @@ class FluidSteadyState:
         if mode == ST_INIT_HOST:
             x0 = _f64(x0)
             x0p = dptr(x0)
-        out = np.zeros(self.ndof) if fetch else None
+        out = np.empty(self.ndof) if fetch else None
         rc = self.lib.st_solve(self.h, mode, x0p, dptr(out) if fetch else None, ctypes.byref(st))
         self._check(rc, allow=(ST_ENOCONV,) if allow_noconv else ())
         self.stats = st.as_dict()
@@ -115,7 +115,7 @@ class FluidSteadyState:
 
     def gradient(self):
         """dJ/drho of the last to_step (filter chain rule applied)."""
-        out = np.zeros(self.ncell)
+        out = np.empty(self.ncell)
         self._check(self.lib.st_get_gradient(self.h, dptr(out)))
         return out
 
@@ -124,14 +124,14 @@ class FluidSteadyState:
         self._check(self.lib.st_reset_solution(self.h))
 
     def solution(self):
-        out = np.zeros(self.ndof)
+        out = np.empty(self.ndof)
         self._check(self.lib.st_get_solution(self.h, dptr(out)))
         return out
 
     # ---- CX/LinearMapping.h:4-14 ----
     def applyMapping(self, x):
         x = _f64(x)
-        y = np.zeros(self.ndof)
+        y = np.empty(self.ndof)
         self._check(self.lib.st_apply(self.h, dptr(x), dptr(y)))
         return y
 
@@ -144,23 +144,23 @@ class FluidSteadyState:
 
     def compute_gradient_x(self, x):
         x = _f64(x)
-        y = np.zeros(self.ndof)
+        y = np.empty(self.ndof)
         self._check(self.lib.st_energy_grad(self.h, dptr(x), dptr(y)))
         return y
 
     # ---- FT/FluidTopoOpt3D.cpp:170-198 ----
     def sensitivity(self, rho, x, lam):
-        out = np.zeros(self.ncell)
+        out = np.empty(self.ncell)
         self._check(self.lib.st_sensitivity(self.h, dptr(_f64(rho)), dptr(_f64(x)), dptr(_f64(lam)), dptr(out)))
         return out
 
     def filter(self, v, transpose=False):
-        out = np.zeros(self.ncell)
+        out = np.empty(self.ncell)
         self._check(self.lib.st_filter(self.h, dptr(_f64(v)), dptr(out), int(transpose)))
         return out
 
     def oc_update(self, rho, dc, volfrac, move=0.2, eta=0.5, rho_min=1e-3):
-        out = np.zeros(self.ncell)
+        out = np.empty(self.ncell)
         ch = ctypes.c_double()
         self._check(self.lib.st_oc_update(self.h, dptr(_f64(rho)), dptr(_f64(dc)), float(volfrac), float(move),
                                           float(eta), float(rho_min), dptr(out), ctypes.byref(ch)))

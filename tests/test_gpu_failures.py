@@ -171,3 +171,29 @@ def test_failed_solve_in_a_warm_started_sequence(make_solver):
     ref = solver_for(make_solver, P, rho * 0.8, rtol=1e-10, precision="fp32")
     xr, _ = ref.solve()
     assert st["converged"] and rel(x, xr) < 1e-7
+
+
+@pytest.mark.parametrize("dim,n", [(3, 64), (3, 128), (2, 1024)])
+def test_large_host_arrays_survive_the_trip(make_solver, dim, n):
+    """Arrays around and above the size at which host copies go through the pinned slots
+    (8.6, 68 and 25 MB; the last slot partly filled): bit-equal after up and down, also
+    when calls follow each other without a wait and after a call that failed."""
+    P = channel_problem(dim, n)
+    rng = np.random.default_rng(n)
+    s = solver_for(make_solver, P, np.full(n ** dim, 0.4), max_iter=2)
+    rho = rng.uniform(0.1, 0.9, n ** dim)
+    s.set_design(rho)
+    assert np.array_equal(s.get_design(), rho)
+    x = rng.standard_normal(P.fixed.size)
+    y = s.applyMapping(x)
+    for _ in range(3):
+        assert np.array_equal(s.applyMapping(x), y)
+        s.sensitivity(rho, x, y)
+    fixed = P.fixed.astype(bool)
+    assert np.array_equal(y[fixed], x[fixed])
+    bad = rho.copy()
+    bad[-1] = np.inf
+    with pytest.raises(StokesError):
+        s.set_design(bad)
+    out, _ = s.solve(init="host", x0=x, allow_noconv=True)
+    assert np.array_equal(out, s.solution())
