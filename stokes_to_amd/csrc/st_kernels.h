@@ -106,9 +106,9 @@ void launch_sum(int np, int nvec, const double *part, double *out, hipStream_t s
 unsigned blas_blocks(long n);
 template <typename TA, typename TB> void launch_dot(long n, const TA *a, const TB *b, double *part, hipStream_t);
 template <typename TW, typename TV>
-void launch_multidot(long n, const TW *w, const TV *V, long ld, int m, double *part, hipStream_t);
+unsigned launch_multidot(long n, const TW *w, const TV *V, long ld, int m, double *part, hipStream_t);
 template <typename TW, typename TV>
-void launch_multiaxpy(long n, TW *w, const TV *V, long ld, int m, const double *h, const double *sc, double *part,
+unsigned launch_multiaxpy(long n, TW *w, const TV *V, long ld, int m, const double *h, const double *sc, double *part,
                       hipStream_t);
 template <typename TX, typename TY> void launch_axpby(long n, double a, const TX *x, double b, TY *y, hipStream_t);
 void launch_lincomb3(long n, double a, const double *x, double b, const double *w, double c, double *y, hipStream_t);

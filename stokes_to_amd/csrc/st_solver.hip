@@ -560,10 +560,9 @@ template <typename TV, typename TW> static int fgmres(st_ctx *c, const double *b
             prof_mark(c, ST_PROF_APPLY);
             inner_apply(c, zj, w);
             prof_mark(c, ST_PROF_APPLY);
-            const unsigned nbk = blas_blocks(nv);
-            launch_multidot<TW, TV>(nv, w, Vb, nv, j + 1, c->part, c->s);
+            unsigned nbk = launch_multidot<TW, TV>(nv, w, Vb, nv, j + 1, c->part, c->s);
             launch_sum((int)nbk, j + 1, c->part, c->h_dev, c->s, hh, LAZY ? c->sig2_host : nullptr, c->sig2_dev);
-            launch_multiaxpy<TW, TV>(nv, w, Vb, nv, j + 1, c->h_dev, LAZY ? c->sig2_dev : nullptr, c->part, c->s);
+            nbk = launch_multiaxpy<TW, TV>(nv, w, Vb, nv, j + 1, c->h_dev, LAZY ? c->sig2_dev : nullptr, c->part, c->s);
             launch_sum((int)nbk, 1, c->part, hh + (j + 1), c->s);
             CK(hipStreamSynchronize(c->s));
             const double un = std::sqrt(hh[j + 1]);  // |u_{j+1}| (LAZY) or |w|
