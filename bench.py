@@ -129,13 +129,14 @@ def summary(stats):
 def roofline_of(prof, n, prec):
     """Roofline of the finest-level smoother from the solver's own HIP-event launch
     timings: the one-pass two-colour sweep (`k_sweep`) where the path runs it, else the
-    colour pass (`k_march<prec, SMOOTH>`)."""
+    colour pass (`k_march<prec, SMOOTH>`; `k_box<prec>` at 64^3, in FP64 at 128^3 too)."""
     ctype = {"fp64": "double", "fp32": "float", "bf16": "bf16"}[prec]
     if prof.get("sweep", {}).get("launches", 0) > 0:
         pr, kname = prof["sweep"], f"k_sweep<{ctype}> ({n}^3 finest-level two-colour sweep, {prec} storage)"
         traffic = SWEEP256_TRAFFIC_BYTES.get(prec) if n == 256 else None
     else:
-        pr, kname = prof["smooth"], f"k_march<{ctype},SMOOTH> ({n}^3 finest-level colour pass, {prec} storage)"
+        kern = f"k_box<{ctype}>" if n <= (128 if prec == "fp64" else 64) else f"k_march<{ctype},SMOOTH>"
+        pr, kname = prof["smooth"], f"{kern} ({n}^3 finest-level colour pass, {prec} storage)"
         traffic = SMOOTH256_TRAFFIC_BYTES.get(prec) if n == 256 else None
     avg_ms = pr["total_ms"] / max(pr["launches"], 1)
     achieved = pr["bytes"] / (avg_ms * 1e-3) / 1e9 if avg_ms > 0 else 0.0

@@ -197,8 +197,8 @@ int st_objective_noalloc(int dim, int n, const uint8_t *d_fixed, const double *d
 /* ---- kernel timing (HIP events around each launch on the context stream) ---- */
 enum { ST_PROF_SMOOTH = 0, ST_PROF_APPLY = 1, ST_PROF_RESIDUAL = 2, ST_PROF_SMOOTH0 = 3, ST_PROF_SWEEP = 4,
        ST_PROF_NKIND = 5 };
-/* ST_PROF_SMOOTH: smoother colour passes with x given (k_march<., SMOOTH>);
-   ST_PROF_SMOOTH0: the first pass of a V-cycle, from x = 0 (k_smooth0_pairs);
+/* ST_PROF_SMOOTH: smoother colour passes with x given (k_march<., SMOOTH>, k_box);
+   ST_PROF_SMOOTH0: the first pass of a V-cycle, from x = 0 (k_box);
    ST_PROF_SWEEP: one-pass two-colour sweeps (k_sweep, params.fused_sweep) */
 /* on != 0 starts recording the finest-level launches of each kind; 0 stops */
 int st_profile(st_ctx *c, int on);

@@ -323,7 +323,7 @@ template <typename TS> static void smooth(st_ctx *c, int l, const TS *b, TS *x, 
         }
     }
     for (int sw = 0; sw < nu; sw++) {
-        // the pass from x = 0 is another kernel (k_smooth0_pairs) with other bytes
+        // the pass from x = 0 is another kernel (k_box from zero) with other bytes
         const int k0 = (zero && sw == 0) ? ST_PROF_SMOOTH0 : ST_PROF_SMOOTH;
         if (pr) prof_mark(c, k0);
         launch_smooth<TS>(g, c->fl[l], h.al[l], b, x, t, first, om, zero && sw == 0, l > 0, c->s);
