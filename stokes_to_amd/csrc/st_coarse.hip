@@ -534,6 +534,34 @@ template <typename TS, int DIM, int N, bool M> struct LdsAcc {
     __device__ __forceinline__ C AL(int d, int di, int dj, int dk) const { return Cvt<TS>::ld(l.al[d * L::NODES + o(di, dj, dk)]); }
 };
 
+// What a colour cell of the lane keeps in registers over the level's passes of a cycle: its
+// right-hand side, penalties and the flags of its node and the neighbours along the axes,
+// half of what a pass reads from LDS and, with BF16 storage, converts (the cycle from 32^2
+// 50 -> 36 us BF16, 31 -> 29 FP32; from 8^3 35 -> 27 and 24 -> 23).  Not in FP64, where
+// they spill: 38 -> 47 us from 32^2, and read again on the way up 38 -> 38.
+template <typename TS, int DIM> struct TailCell {
+    typename Cvt<TS>::C b[1 + 2 * DIM], al[2 * DIM];
+    int fl, q;
+};
+template <typename TS> constexpr bool tail_keep() { return sizeof(typename Cvt<TS>::C) == 4; }
+template <typename TS, int DIM, int N, bool M> struct TailAcc {
+    typedef typename Cvt<TS>::C C;
+    static constexpr bool MASK = M, KEEP = tail_keep<TS>();
+    LdsAcc<TS, DIM, N, M> a;
+    TailCell<TS, DIM> c;
+    __device__ __forceinline__ int F(int di, int dj, int dk) const
+    {
+        const int s = di + dj + dk, ax = di ? 0 : (dj ? 1 : 2);
+        if (!KEEP || (di != 0) + (dj != 0) + (dk != 0) > 1 || s > 1 || s < -1) return a.F(di, dj, dk);
+        return (c.fl >> (s == 0 ? 0 : 4 * (1 + 2 * ax + (s > 0)))) & 15;
+    }
+    __device__ __forceinline__ C X(int f, int di, int dj, int dk) const { return a.X(f, di, dj, dk); }
+    __device__ __forceinline__ C B(int f, int di, int dj, int dk) const
+    { return KEEP ? c.b[di + dj + dk ? DIM + f : f] : a.B(f, di, dj, dk); }
+    __device__ __forceinline__ C AL(int d, int di, int dj, int dk) const
+    { return KEEP ? c.al[di + dj + dk ? DIM + d : d] : a.AL(d, di, dj, dk); }
+};
+
 constexpr int TAIL_NT = 512;  // 256 registers a lane: the FP64 block solve fits them
 
 // the node t of the (N + 1)^DIM nodes of a level
@@ -551,32 +579,55 @@ template <int DIM, int N> __device__ __forceinline__ void node_of(int t, int &i,
 }
 template <int DIM, int N> constexpr int n_nodes() { return (N + 1) * (N + 1) * (DIM == 3 ? N + 1 : 1); }
 
-// one colour pass in place: every lane reads what it needs, then every lane writes (the
-// first pass of the way down reads the zeros the launch starts with)
+// the lane's cell of a colour (the first half of the level's cells, one per lane)
 template <typename TS, int DIM, int N, bool MASK>
-__device__ __forceinline__ void tail_color(TLvl<TS, DIM, N> &l, int color, float omega)
+__device__ __forceinline__ TailCell<TS, DIM> tail_cell(const TLvl<TS, DIM, N> &l, int color)
 {
-    typedef typename Cvt<TS>::C C;
     typedef TLvl<TS, DIM, N> L;
     constexpr int NP = (DIM == 3 ? N * N * N : N * N) / 2, H = N / 2;
     static_assert(NP <= TAIL_NT, "one colour cell per lane");
-    const int t = threadIdx.x;
-    int q = 0;
+    const int t = (int)threadIdx.x < NP ? (int)threadIdx.x : 0;
+    int i, j, k;
+    const int pr = 2 * (t % H);
+    if (DIM == 3) {
+        j = (t / H) % N;
+        i = t / (H * N);
+        k = pr + ((i + j + color) & 1);
+    } else {
+        i = t / H;
+        j = pr + ((i + color) & 1);
+        k = 0;
+    }
+    TailCell<TS, DIM> c;
+    c.q = L::id(i, j, k);
+    if (!tail_keep<TS>()) return c;
+    const LdsAcc<TS, DIM, N, MASK> a{l, c.q};
+    c.fl = a.F(0, 0, 0) & 15;
+    c.b[0] = a.B(0, 0, 0, 0);
+#pragma unroll
+    for (int d = 0; d < DIM; d++) {
+        const int di = d == 0, dj = d == 1, dk = d == 2;
+        c.fl |= (a.F(-di, -dj, -dk) & 15) << (4 * (1 + 2 * d)) | (a.F(di, dj, dk) & 15) << (4 * (2 + 2 * d));
+        c.b[1 + d] = a.B(1 + d, 0, 0, 0);
+        c.b[1 + DIM + d] = a.B(1 + d, di, dj, dk);
+        c.al[d] = a.AL(d, 0, 0, 0);
+        c.al[DIM + d] = a.AL(d, di, dj, dk);
+    }
+    return c;
+}
+
+// one colour pass in place: every lane reads what it needs, then every lane writes (the
+// first pass of the way down reads the zeros the launch starts with)
+template <typename TS, int DIM, int N, bool MASK>
+__device__ __forceinline__ void tail_color(TLvl<TS, DIM, N> &l, const TailCell<TS, DIM> &c, float omega)
+{
+    typedef typename Cvt<TS>::C C;
+    typedef TLvl<TS, DIM, N> L;
+    constexpr int NP = (DIM == 3 ? N * N * N : N * N) / 2;
+    const int t = threadIdx.x, q = c.q;
     C pn, u0[3], u1[3];
     if (t < NP) {
-        int i, j, k;
-        const int pr = 2 * (t % H);
-        if (DIM == 3) {
-            j = (t / H) % N;
-            i = t / (H * N);
-            k = pr + ((i + j + color) & 1);
-        } else {
-            i = t / H;
-            j = pr + ((i + color) & 1);
-            k = 0;
-        }
-        q = L::id(i, j, k);
-        const LdsAcc<TS, DIM, N, MASK> a{l, q};
+        const TailAcc<TS, DIM, N, MASK> a{{l, q}, c};
         box_cell<C, DIM, false>(a, omega, pn, u0, u1);
     }
     __syncthreads();
@@ -593,10 +644,23 @@ __device__ __forceinline__ void tail_color(TLvl<TS, DIM, N> &l, int color, float
 }
 
 template <typename TS, int DIM, int N, bool MASK>
-__device__ __forceinline__ void tail_smooth(TLvl<TS, DIM, N> &l, int nu, int first, float omega)
+__device__ __forceinline__ void tail_smooth(TLvl<TS, DIM, N> &l, const TailCell<TS, DIM> &c0, const TailCell<TS, DIM> &c1,
+                                            int nu, int first, float omega)
 {
 #pragma unroll 1
-    for (int s = 0; s < 2 * nu; s++) tail_color<TS, DIM, N, MASK>(l, first ^ (s & 1), omega);
+    for (int s = 0; s < 2 * nu; s++) {
+        const bool odd = first ^ (s & 1);
+        TailCell<TS, DIM> c;
+        c.q = odd ? c1.q : c0.q;
+        if (tail_keep<TS>()) {
+            c.fl = odd ? c1.fl : c0.fl;
+#pragma unroll
+            for (int v = 0; v < 1 + 2 * DIM; v++) c.b[v] = odd ? c1.b[v] : c0.b[v];
+#pragma unroll
+            for (int v = 0; v < 2 * DIM; v++) c.al[v] = odd ? c1.al[v] : c0.al[v];
+        }
+        tail_color<TS, DIM, N, MASK>(l, c, omega);
+    }
 }
 
 // r = b - A x on the nodes of the level
@@ -741,10 +805,11 @@ __device__ __forceinline__ void tail_cycle(TailPool<TS, DIM, N> &p, int nu_pre, 
     } else {
         // way down, then way up: one loop, so that the passes of a level are compiled once
         // (the launch runs on one CU, and fetching its instructions is a good part of it)
+        const TailCell<TS, DIM> c0 = tail_cell<TS, DIM, N, MASK>(p.l, 0), c1 = tail_cell<TS, DIM, N, MASK>(p.l, 1);
 #pragma unroll 1
         for (int up = 0; up < 2; up++) {
             if (up) tail_prolong<TS, DIM, N>(p.l, p.next.l);
-            tail_smooth<TS, DIM, N, MASK>(p.l, up ? nu_post : nu_pre, up, om);
+            tail_smooth<TS, DIM, N, MASK>(p.l, c0, c1, up ? nu_post : nu_pre, up, om);
             if (!up) {
                 tail_residual<TS, DIM, N, MASK>(p.l);
                 tail_restrict<TS, DIM, N>(p.l, p.next.l);
@@ -761,9 +826,9 @@ __device__ __forceinline__ void tail_cycle(TailPool<TS, DIM, N> &p, int nu_pre, 
 // updated in place (a pass holds its results in registers over a barrier), so a level
 // needs x, b, alpha and r only and a 32^2 level fits in FP64; sides, pitches and loop
 // counts are compile-time constants, and the coarsest inverse is read into registers
-// while the levels are staged.  Per cycle, first level 8^3: 28 us FP64, 25 us FP32
+// while the levels are staged.  Per cycle, first level 8^3: 28 us FP64, 23 us FP32
 // (81 us both with 64-bit index arithmetic, run-time sides and the rows of a cell
-// evaluated one by one); from 32^2: 38 / 30 us (65 us from 16^2, and ten launches of
+// evaluated one by one); from 32^2: 38 / 29 us (65 us from 16^2, and ten launches of
 // 3-7 us for the 32^2 level).  One workgroup is a chain of ~20 passes of ~1 us each.
 template <typename TS, int DIM, int N, bool MASK>
 __global__ void __launch_bounds__(TAIL_NT) k_tail(TailArgs<TS> a, const TS *__restrict__ b0, TS *__restrict__ x0)
