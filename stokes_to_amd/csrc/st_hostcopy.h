@@ -14,8 +14,9 @@ class HostCopy {
 public:
     HostCopy() = default;
     ~HostCopy();
-    // slots and threads for arrays up to n bytes now (else on the first large copy)
-    void prepare(size_t n) { if (n >= MIN_OUT) ready(n); }
+    // the first half of the slots and threads now, for a context whose arrays have n bytes (the
+    // second half, and without this call the first, are made on the first copy that needs them)
+    void prepare(size_t n) { if (n >= MIN_OUT) ready(MIN_OUT); }
     // h may be read (out) or changed (in) by the caller when these return; the transfer of
     // in() may still run on s
     hipError_t out(void *h, const void *d, size_t n, hipStream_t s);
