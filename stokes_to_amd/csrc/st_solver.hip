@@ -20,6 +20,7 @@
 #include <limits>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -642,6 +643,15 @@ static int check_finite(st_ctx *c, const double *h, long n, const char *what)
     return ST_OK;
 }
 
+// The component entries (st_mg_smooth and the ones after it) use the solver's scratch vectors
+// in the layout of their level and precision.  They clear what they wrote: the padding
+// entries of a finest-level vector must hold 0 (the operator of st_fine.hip reads them as the
+// pressures outside the level), and most kernels never write those.
+static void clear_scratch(st_ctx *c, const Lvl &g, std::initializer_list<double *> used)
+{
+    for (double *v : used) launch_fill<double>((long)g.nfield * g.S, v, 0.0, c->s);
+}
+
 // one smoother colour step in FP32 / BF16 storage (test entry st_mg_smooth_mp)
 template <typename TS> static int mg_smooth_lowp(st_ctx *c, int l, int color, const double *b, const double *xin,
                                                  double *xout)
@@ -657,6 +667,7 @@ template <typename TS> static int mg_smooth_lowp(st_ctx *c, int l, int color, co
     launch_fill<TS>((long)g.nfield * g.S, xo, 0.0, c->s);
     launch_smooth<TS>(g, c->fl[l], hier<TS>(c).al[l], bb, xi, xo, color, (float)c->prm.omega, false, false, c->s);
     launch_unpack<TS>(g, xo, c->abi_b, c->s);
+    clear_scratch(c, g, {c->BA, c->Wv, c->V});
     return stage_out(c, xout, nd);
 }
 
@@ -1887,6 +1898,7 @@ int st_mg_level_desc(st_ctx *c, int l, uint8_t *fixed, double *alpha_faces)
         launch_fill<double>((long)g.nfield * g.S, c->Wv, 0.0, c->s);
         CK(hipMemcpyAsync(c->Wv + g.S, c->h64.al[l], sizeof(double) * g.dim * g.S, hipMemcpyDeviceToDevice, c->s));
         launch_unpack<double>(g, c->Wv, c->abi_b, c->s);
+        clear_scratch(c, g, {c->Wv});
         std::vector<double> tmp(nd);
         CKR(stage_out(c, tmp.data(), nd));
         long nc = (long)g.nx * g.ny * g.nz;
@@ -1908,6 +1920,7 @@ int st_mg_smooth(st_ctx *c, int l, int color, const double *b, const double *xin
     launch_fill<double>((long)g.nfield * g.S, c->V, 0.0, c->s);
     launch_smooth<double>(g, c->fl[l], c->h64.al[l], c->BA, c->Wv, c->V, color, (float)c->prm.omega, false, false, c->s);
     launch_unpack<double>(g, c->V, c->abi_b, c->s);
+    clear_scratch(c, g, {c->BA, c->Wv, c->V});
     return stage_out(c, xout, nd);
 }
 
@@ -1929,6 +1942,7 @@ int st_mg_restrict(st_ctx *c, int l, const double *rf, double *bc)
     launch_pack<double>(g, c->abi_a, c->BA, 0, c->fl[l], 1.0, c->s);
     launch_restrict<double>(g, gc, c->fl[l + 1], c->BA, c->Wv, c->s);
     launch_unpack<double>(gc, c->Wv, c->abi_b, c->s);
+    clear_scratch(c, g, {c->BA, c->Wv});
     return stage_out(c, bc, level_dofs(c, l + 1));
 }
 
@@ -1943,6 +1957,7 @@ int st_mg_prolong(st_ctx *c, int l, const double *ec, const double *xf, double *
     launch_pack<double>(g, c->abi_a, c->Wv, 0, c->fl[l], 1.0, c->s);
     launch_prolong<double>(g, gc, c->fl[l], c->BA, c->Wv, c->s);
     launch_unpack<double>(g, c->Wv, c->abi_b, c->s);
+    clear_scratch(c, g, {c->BA, c->Wv});
     return stage_out(c, xf_out, level_dofs(c, l));
 }
 

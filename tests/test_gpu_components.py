@@ -1,0 +1,46 @@
+"""Calls of the component entries (st_mg_*) and what they leave behind, and the coarsest
+inverse at the ends of its range, against the oracle."""
+import numpy as np
+import pytest
+
+from conftest import rel
+from helpers import oracle_desc, setup, solver_for
+from stokes_to_amd.problems import _split
+
+pytestmark = pytest.mark.gpu
+
+
+def open_low_sides(P, seed):
+    """P with 2% more fixed cells and interior faces and with free faces on the low side of
+    every axis, where a face's row reads a pressure outside the level."""
+    rng = np.random.default_rng(seed)
+    P.fixed[rng.integers(0, P.fixed.size, P.fixed.size // 50)] = 1
+    n, m = P.n, slice(P.n // 4, 3 * P.n // 4)
+    fx, fy, fz = _split(3, n, P.fixed)[1:]
+    fx[0, m, :] = 0
+    fy[:, 0, m] = 0
+    fz[m, :, 0] = 0
+
+
+@pytest.mark.parametrize("call", ["none", "smooth", "prolong", "restrict", "desc"])
+def test_vcycle_after_a_call_on_a_coarse_level(make_solver, orc, call):
+    """A component call on a coarser level must not change a later V-cycle on the finest
+    one (64^3, whose operator reads pressures outside the level from entries that hold 0):
+    1e-10 of the oracle, as without it."""
+    n = 64
+    P, rho = setup(3, n)
+    open_low_sides(P, n)
+    fixed, vol, pen = oracle_desc(orc, P, rho)
+    s = solver_for(make_solver, P, rho)
+    rng = np.random.default_rng(7)
+    v = [rng.standard_normal(orc.sizes(3, n >> l, n >> l, n >> l)[0]) for l in range(3)]
+    if call == "smooth":
+        s.mg_smooth(1, 0, v[1], v[1])
+    if call == "prolong":
+        s.mg_prolong(1, v[2], v[1])
+    if call == "restrict":
+        s.mg_restrict(0, v[0])
+    if call == "desc":
+        s.mg_level_desc(1)
+    mg = orc.MG(3, P.shape, fixed, pen, nu_pre=1, nu_post=2, omega=1.0, tang=0)
+    assert rel(s.mg_vcycle(v[0]), mg.vcycle(v[0])) < 1e-10
