@@ -327,9 +327,9 @@ __global__ void k_probe(Lvl g, const uint8_t *fl, const TS *al, const long *dofs
 // one workgroup, the matrix in LDS.  A step is one read and one write of the matrix:
 // every wave finds the pivot itself by shuffles, and every lane forms the new values of
 // its entries (row swap, scaling and elimination in one) before any is written.  The
-// 44 steps of 3D take 46 us, the 16 of 2D 15 us (194 and 58 us with the matrix in
-// memory, a tree of barriers per pivot and four passes per step).  info: 0 ok, k > 0 zero pivot at step k (singular), -1 a non-finite
-// entry (nothing is inverted)
+// 44 steps of 3D take 47 us, the 16 of 2D 17 us (194 and 58 us with the matrix in
+// memory, a tree of barriers per pivot and four passes per step).  info: 0 ok, k > 0 zero
+// pivot at step k (singular), -1 a non-finite entry (nothing is inverted)
 constexpr int GJ_MAX = 64, GJ_NT = 1024;
 // maximum over the wave, in every lane, by DPP row shifts and broadcasts
 __device__ __forceinline__ unsigned wave_max_u32(unsigned v)
@@ -369,25 +369,20 @@ __global__ void __launch_bounds__(GJ_NT) k_gauss_jordan(int n, double *A, int *i
         return;
     }
     for (int k = 0; k < n; k++) {
-        // pivot row: largest |M[r][k]|, r >= k, to 17 bits (any row that near the largest
-        // serves), the first of equals; magnitudes that vanish in FP32 are compared in full
+        // pivot row: largest |M[r][k]|, r >= k, the first of equals.  Magnitudes compare as
+        // their bits do: the high words first (1 more than the word, 0 for no candidate), the
+        // low words only among equals (in all 47 us in 3D and 17 in 2D; with the maximum of doubles
+        // 54 and 18, with a comparison of 17 bits 45 and 14)
         const double mag = (lane >= k && lane < n) ? fabs(M[lane][k]) : -1.0;
-        const unsigned fbits = mag > 0.0 ? __float_as_uint((float)mag) : 0u;
-        const unsigned key = wave_max_u32((fbits & ~63u) | (63u - (unsigned)lane));
-        int p = 63 - (int)(key & 63u);
-        if ((key & ~63u) == 0u) {
-            double best = mag;
-            p = lane;
-            for (int o = 32; o > 0; o >>= 1) {
-                const double ov = __shfl_xor(best, o, 64);
-                const int oi = __shfl_xor(p, o, 64);
-                if (ov > best || (ov == best && oi < p)) {
-                    best = ov;
-                    p = oi;
-                }
-            }
-            if (!(best >= 0.0)) p = k;
+        const unsigned hi = mag >= 0.0 ? (unsigned)__double2hiint(mag) + 1u : 0u;  // (no NaN)
+        const unsigned top = wave_max_u32(hi);
+        unsigned long long at = __ballot(hi == top);
+        if (at & (at - 1)) {
+            const unsigned lo = hi == top ? (unsigned)__double2loint(mag) : 0u;
+            const unsigned tl = wave_max_u32(lo);
+            at = __ballot(hi == top && lo == tl);
         }
+        const int p = top ? (int)__builtin_ctzll(at) : k;
         const double pv = M[p][k];
         const double pinv = (pv != 0.0) ? 1.0 / pv : 0.0;
         double nv[PER];

@@ -44,3 +44,29 @@ def test_vcycle_after_a_call_on_a_coarse_level(make_solver, orc, call):
         s.mg_level_desc(1)
     mg = orc.MG(3, P.shape, fixed, pen, nu_pre=1, nu_post=2, omega=1.0, tang=0)
     assert rel(s.mg_vcycle(v[0]), mg.vcycle(v[0])) < 1e-10
+
+
+@pytest.mark.parametrize("dim,share,seed", [(2, 0.3, 21), (3, 0.5, 21), (3, 0.5, 112)])
+def test_coarsest_inverse_pivots_in_full_precision(make_solver, orc, dim, share, seed):
+    """Penalties of 1e38 to 1e60, beyond the largest FP32 value: the pivot of the coarsest
+    inverse has to be the largest FP64 magnitude (a V-cycle without sweeps is that inverse
+    between transfers).  1e-10 of the oracle: eliminated with the largest pivot, these
+    matrices keep 1e-15 under any rounding; with a smaller one they can lose all digits."""
+    n = 8
+    rng = np.random.default_rng(seed)
+    nd = orc.sizes(dim, n, n, n if dim == 3 else 1)[0]
+    fixed, pen = np.zeros(nd, np.uint8), np.zeros(nd)
+    ff, pp = _split(dim, n, fixed), _split(dim, n, pen)
+    for d in range(dim):  # one value for the fine faces under each face of the 2^dim grid
+        c = 10.0 ** rng.uniform(38, 60, [3 if a == d else 2 for a in range(dim)])
+        off = rng.random(c.shape) < share
+        at = np.ix_(*[(np.arange(n + 1) + 1) // 4 if a == d else np.arange(n) // 4 for a in range(dim)])
+        pp[1 + d][...] = (c * ~off)[at].reshape(pp[1 + d].shape)
+        ff[1 + d][...] = off[at].reshape(pp[1 + d].shape)
+    ff[0][...] = (rng.random([2] * dim) < 0.3)[np.ix_(*[np.arange(n) // 4] * dim)].reshape(ff[0].shape)
+    s = make_solver(dim, n, nu_pre=0, nu_post=0)
+    s.init_boundary(fixed)
+    s.update_penalty(pen)
+    mg = orc.MG(dim, (n, n, n if dim == 3 else 1), fixed, pen, nu_pre=0, nu_post=0, omega=1.0, tang=0)
+    b = rng.standard_normal(nd)
+    assert rel(s.mg_vcycle(b), mg.vcycle(b)) < 1e-10
