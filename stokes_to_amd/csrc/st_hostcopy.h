@@ -48,7 +48,9 @@ private:
     bool open_ = false, stop_ = false;
     int in_job_ = 0;
     // the job: chunk k of h_ lies in slot sl(k); the threads copy the chunks below ready_
-    bool to_host_ = false, drop_ = false;
+    // (drop_: a transfer failed, copy no more; set while threads copy)
+    bool to_host_ = false;
+    std::atomic<bool> drop_{false};
     char *h_ = nullptr;
     size_t n_ = 0;
     long nchunk_ = 0;
