@@ -34,6 +34,7 @@ private:
     void work();
     void open(bool to_host, char *h, size_t n);
     void close();
+    void give_up(hipStream_t s);
     int sl(long k) const { return (int)(k % nslot_); }
     char *slot(long k) const { return pin_[sl(k) / (NSLOT / 2)] + (size_t)(sl(k) % (NSLOT / 2)) * SLOT; }
     size_t len(long k) const { return (size_t)(k + 1) * SLOT < n_ ? SLOT : n_ - (size_t)k * SLOT; }
@@ -42,6 +43,7 @@ private:
     int nslot_ = 0;
     hipEvent_t ev_[NSLOT] = {};
     bool used_[NSLOT] = {};  // ev_ recorded behind a transfer out of the slot
+    bool broken_ = false;    // the stream could not be waited for after a failure: slots stay unused
     std::vector<std::thread> th_;
     std::mutex m_;
     std::condition_variable go_, idle_;

@@ -40,6 +40,7 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 // second half); false: use the runtime's copy
 bool HostCopy::ready(size_t n)
 {
+    if (broken_) return false;
     const int half = n < BIG ? 1 : 2;
     for (int b = nslot_ / (NSLOT / 2); b < half; b++) {
         void *p = nullptr;
@@ -130,6 +131,16 @@ void HostCopy::close()
     idle_.wait(l, [this] { return in_job_ == 0; });
 }
 
+// after a failed transfer: the threads copy no more, and what is queued on s has left the
+// slots before they are used again
+void HostCopy::give_up(hipStream_t s)
+{
+    drop_ = true;
+    ready_.store(nchunk_, std::memory_order_release);
+    if (hipStreamSynchronize(s) != hipSuccess) broken_ = true;
+    for (bool &u : used_) u = false;
+}
+
 hipError_t HostCopy::out(void *h, const void *d, size_t n, hipStream_t s)
 {
     if (n < MIN_OUT || !aligned16(d) || !ready(n)) {
@@ -157,10 +168,7 @@ hipError_t HostCopy::out(void *h, const void *d, size_t n, hipStream_t s)
         if (e == hipSuccess) e = hipEventSynchronize(ev_[sl(j)]);
         if (e == hipSuccess) ready_.store(j + 1, std::memory_order_release);
     }
-    if (e != hipSuccess) {
-        drop_ = true;
-        ready_.store(nchunk_, std::memory_order_release);
-    }
+    if (e != hipSuccess) give_up(s);
     close();
     return e;
 }
@@ -190,10 +198,7 @@ hipError_t HostCopy::in(void *d, const void *h, size_t n, hipStream_t s)
         if (e == hipSuccess) e = hipEventRecord(ev_[q], s);
         if (e == hipSuccess) used_[q] = true;
     }
-    if (e != hipSuccess) {
-        drop_ = true;
-        ready_.store(nchunk_, std::memory_order_release);
-    }
+    if (e != hipSuccess) give_up(s);
     close();
     return e;
 }

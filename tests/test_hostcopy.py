@@ -35,3 +35,11 @@ def test_arrays_of_all_sizes_arrive(ring):
 @pytest.mark.parametrize("at", [1, 3, 12, 18])
 def test_a_copy_may_fail_while_threads_copy(ring, case, at):
     run(ring, case, at)
+
+
+@pytest.mark.parametrize("case", ["failed_out_then", "failed_in_then"])
+@pytest.mark.parametrize("at", [1, 3, 12, 18])
+def test_copies_after_a_failed_one_arrive(ring, case, at):
+    """A transfer that was queued before the failure must not reach a slot, or leave one, once
+    the next copy uses it."""
+    run(ring, case, at)
