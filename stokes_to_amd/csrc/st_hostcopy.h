@@ -17,8 +17,8 @@ public:
     // the first half of the slots and threads now, for a context whose arrays have n bytes (the
     // second half, and without this call the first, are made on the first copy that needs them)
     void prepare(size_t n) { if (n >= MIN_OUT) ready(MIN_OUT); }
-    // h may be read (out) or changed (in) by the caller when these return; the transfer of
-    // in() may still run on s
+    // h may be read (out) or, unless it is memory that the runtime knows, changed (in) by the
+    // caller when these return; the transfer of in() may still run on s
     hipError_t out(void *h, const void *d, size_t n, hipStream_t s);
     hipError_t in(void *d, const void *h, size_t n, hipStream_t s);
 

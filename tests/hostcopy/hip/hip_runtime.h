@@ -45,6 +45,18 @@ typedef struct SimEvent {
 } *hipEvent_t;
 
 inline int fail_record = 0, copies = 0;  // fail_record: the how many-th record from now on
+inline const void *pinned = nullptr;     // start of the one array that the runtime knows
+
+enum hipMemoryType { hipMemoryTypeUnregistered, hipMemoryTypeHost, hipMemoryTypeDevice, hipMemoryTypeManaged };
+struct hipPointerAttribute_t {
+    hipMemoryType type;
+};
+inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p)
+{
+    if (p != pinned) return hipErrorUnknown;
+    a->type = hipMemoryTypeHost;
+    return hipSuccess;
+}
 
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipHostMalloc(void **p, size_t n, unsigned)

@@ -44,6 +44,13 @@ int main(int argc, char **argv)
         for (size_t n : {MB / 2, 4 * MB, 4 * MB + 1, 5 * MB - 1, 32 * MB, 32 * MB + 3, 41 * MB + 7}) bad += both_ways(hc, s, n, n);
         return bad;
     }
+    if (c == "known") {  // by the runtime's own copy, whatever the size
+        Arr h = data(40 * MB, 1), d(40 * MB);
+        pinned = h.data();
+        bad += hc.in(d.data(), h.data(), h.size() * 8, &s) != hipSuccess || copies != 1;
+        bad += hc.out(h.data(), d.data(), h.size() * 8, &s) != hipSuccess || copies != 2;
+        return bad + check("known", h, data(40 * MB, 1));
+    }
     // a copy whose record of the at-th event fails
     const int at = argc > 2 ? std::atoi(argv[2]) : 1;
     const size_t n = 36 * MB + 5;

@@ -31,6 +31,10 @@ def test_arrays_of_all_sizes_arrive(ring):
     run(ring, "sizes")
 
 
+def test_pinned_arrays_take_the_runtime_s_copy(ring):
+    run(ring, "known")
+
+
 @pytest.mark.parametrize("case", ["failed_out", "failed_in"])
 @pytest.mark.parametrize("at", [1, 3, 12, 18])
 def test_a_copy_may_fail_while_threads_copy(ring, case, at):
