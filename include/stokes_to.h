@@ -199,12 +199,17 @@ enum { ST_PROF_SMOOTH = 0, ST_PROF_APPLY = 1, ST_PROF_RESIDUAL = 2, ST_PROF_SMOO
        ST_PROF_NKIND = 5 };
 /* ST_PROF_SMOOTH: smoother colour passes with x given (k_march<., SMOOTH>, k_box);
    ST_PROF_SMOOTH0: the first pass of a V-cycle, from x = 0 (k_box);
-   ST_PROF_SWEEP: one-pass two-colour sweeps (k_sweep, params.fused_sweep) */
+   ST_PROF_SWEEP: one-pass two-colour sweeps (k_sweep, params.fused_sweep); in 2D every
+   launch of the smoother (k_sweeps: one or two sweeps, with the prolongation before the
+   ones that follow it), so that SMOOTH and SMOOTH0 count none there;
+   ST_PROF_RESIDUAL: the residual of a V-cycle; in 2D and below 64^3 with its restriction.
+   A finest grid of 8^3 or of at most 32^2 cells runs its whole V-cycle in one launch that
+   is of no kind. */
 /* on != 0 starts recording the finest-level launches of each kind; 0 stops */
 int st_profile(st_ctx *c, int on);
 /* total device ms and launch count recorded for `kind` since st_profile(c, 1);
    bytes = algorithmic HBM bytes of one launch of that kind (FP64 unless the MG
-   precision applies) */
+   precision applies), the mean over those recorded where they differ */
 int st_profile_read(st_ctx *c, int kind, double *total_ms, long *launches, double *bytes_per_launch);
 
 /* ---- learned initial guess (no counterpart in the reference, whose GMRES starts

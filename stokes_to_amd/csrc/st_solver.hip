@@ -111,6 +111,8 @@ struct st_ctx {
     size_t evused[ST_PROF_NKIND] = {};
     double prof_ms[ST_PROF_NKIND] = {};
     long prof_n[ST_PROF_NKIND] = {};
+    double prof_bytes[ST_PROF_NKIND] = {};  // of the launches whose bytes differ by their path
+    long prof_nb[ST_PROF_NKIND] = {};
 };
 
 static void prof_mark(st_ctx *c, int kind)
@@ -123,6 +125,13 @@ static void prof_mark(st_ctx *c, int kind)
         pool.push_back(e);
     }
     hipEventRecord(pool[c->evused[kind]++], c->s);
+}
+// a launch of this kind that needs other bytes than kind_bytes
+static void prof_launch_bytes(st_ctx *c, int kind, double bytes)
+{
+    if (!c->prof) return;
+    c->prof_bytes[kind] += bytes;
+    c->prof_nb[kind]++;
 }
 
 // called after the stream is synchronised: fold recorded pairs into totals
@@ -363,6 +372,24 @@ template <typename TS> static TailArgs<TS> tail_args(st_ctx *c, int l0)
     return a;
 }
 
+// Bytes of the finest level's launches that do more than one step (k_sweeps,
+// k_resid_restrict), as kind_bytes counts them
+static double mg_bytes(const st_ctx *c) { return c->prm.precision == ST_FP64 ? 8.0 : (c->prm.precision == ST_FP32 ? 4.0 : 2.0); }
+static double coarse_dofs(const st_ctx *c) { return (double)abi_dofs(c->dim, c->n / 2); }
+// b, alpha read and x written, whatever the number of sweeps; x read unless it is zero, the
+// coarse correction where it is added
+static double sweeps_bytes(const st_ctx *c, bool zero, bool prol)
+{
+    const double nv = (double)c->ndof, nf = nv - (double)c->ncell;
+    return mg_bytes(c) * ((zero ? 2.0 : 3.0) * nv + nf + (prol ? coarse_dofs(c) : 0.0)) + nf / 8.0;
+}
+// x, b, alpha read and the coarse right-hand side written: the residual stays in LDS
+static double resid_restrict_bytes(const st_ctx *c)
+{
+    const double nv = (double)c->ndof, nf = nv - (double)c->ncell;
+    return mg_bytes(c) * (2.0 * nv + nf + coarse_dofs(c)) + nf / 8.0;
+}
+
 // The sweeps of a 2D level run up to ST_SWEEPS to a launch, each launch from one buffer to
 // the other (x and t).  Whether the cycle's first launch writes x, so that its last does:
 static bool first_writes_x(const st_ctx *c)
@@ -382,7 +409,10 @@ static void fused_sweeps(st_ctx *c, int l, const TS *b, TS *x, TS *&cur, int nu,
         if (l == 0) prof_mark(c, ST_PROF_SWEEP);
         launch_sweeps<TS>(g, c->lv[l + 1], c->fl[l], h.al[l], b, cur, done ? (const TS *)nullptr : ec, to, ns, first,
                           (float)c->prm.omega, zero && done == 0, l > 0, c->s);
-        if (l == 0) prof_mark(c, ST_PROF_SWEEP);
+        if (l == 0) {
+            prof_mark(c, ST_PROF_SWEEP);
+            prof_launch_bytes(c, ST_PROF_SWEEP, sweeps_bytes(c, zero && done == 0, ec && done == 0));
+        }
         cur = to;
         done += ns;
     }
@@ -415,7 +445,10 @@ template <typename TS> static void vcycle(st_ctx *c, const TS *b0, TS *x0)
             launch_restrict<TS>(g, c->lv[l + 1], c->fl[l + 1], h.r[l], h.b[l + 1], c->s);
         } else {
             launch_resid_restrict<TS>(g, c->lv[l + 1], c->fl[l], h.al[l], b, cur[l], c->fl[l + 1], h.b[l + 1], l > 0, c->s);
-            if (l == 0) prof_mark(c, ST_PROF_RESIDUAL);
+            if (l == 0) {
+                prof_mark(c, ST_PROF_RESIDUAL);
+                prof_launch_bytes(c, ST_PROF_RESIDUAL, resid_restrict_bytes(c));
+            }
         }
     }
     launch_vcycle_tail<TS>(tail_args<TS>(c, lt), c->dim, c->lv[lt].nx, lt == 0 ? b0 : h.b[lt], lt == 0 ? x0 : h.x[lt],
@@ -938,10 +971,37 @@ int st_profile(st_ctx *c, int on)
     CK(hipStreamSynchronize(c->s));
     prof_collect(c);
     if (on) {
-        for (int k = 0; k < ST_PROF_NKIND; k++) { c->prof_ms[k] = 0.0; c->prof_n[k] = 0; }
+        for (int k = 0; k < ST_PROF_NKIND; k++) {
+            c->prof_ms[k] = c->prof_bytes[k] = 0.0;
+            c->prof_n[k] = c->prof_nb[k] = 0;
+        }
     }
     c->prof = on != 0;
     return ST_OK;
+}
+
+// algorithmic HBM bytes of one finest-level launch over the valid DOFs, with the masks
+// counted as bit fields (n_f/8 bytes):
+//   operator apply      (s_x + s_y)(n_c + n_f) + s_a n_f + n_f/8  (x, alpha read, y write)
+//   residual            s(3 n_c + 4 n_f) + n_f/8   (x, b, alpha read, r write)
+//   smoother colour     half of a two-colour sweep s(3 n_c + 4 n_f) + n_f/8
+//                       (x, b, alpha read once, x written once per sweep)
+//   zero-start pass     s(2 n_c + 3 n_f) + n_f/8  (b, alpha read, x written; x = 0 is not
+//                       read)
+//   one-pass sweep      s(3 n_c + 4 n_f) + n_f/8  (both colours)
+// s: storage of the level-0 multigrid vectors; the Krylov operator of the FP32 path is
+// FP32, that of the BF16 path FP64 on FP32 vectors
+static double kind_bytes(const st_ctx *c, int kind)
+{
+    const double nc = (double)c->ncell, nf = (double)(c->ndof - c->ncell), sv = mg_bytes(c);
+    const int pr = c->prm.precision;
+    if (kind == ST_PROF_SMOOTH) return 0.5 * (sv * (3.0 * nc + 4.0 * nf) + nf / 8.0);
+    if (kind == ST_PROF_SMOOTH0) return sv * (2.0 * nc + 3.0 * nf) + nf / 8.0;
+    if (kind == ST_PROF_APPLY) {
+        const double sx = (pr == ST_FP64) ? 8.0 : 4.0, sa = (pr == ST_FP32) ? 4.0 : 8.0, sy = sa;
+        return (sx + sy) * (nc + nf) + sa * nf + nf / 8.0;
+    }
+    return sv * (3.0 * nc + 4.0 * nf) + nf / 8.0;
 }
 
 int st_profile_read(st_ctx *c, int kind, double *total_ms, long *launches, double *bytes)
@@ -949,29 +1009,7 @@ int st_profile_read(st_ctx *c, int kind, double *total_ms, long *launches, doubl
     if (!c || kind < 0 || kind >= ST_PROF_NKIND) return ST_EINVAL;
     if (total_ms) *total_ms = c->prof_ms[kind];
     if (launches) *launches = c->prof_n[kind];
-    if (bytes) {
-        // algorithmic HBM bytes of one finest-level launch over the valid DOFs, with the
-        // masks counted as bit fields (n_f/8 bytes):
-        //   operator apply      (s_x + s_y)(n_c + n_f) + s_a n_f + n_f/8  (x, alpha read, y write)
-        //   residual            s(3 n_c + 4 n_f) + n_f/8   (x, b, alpha read, r write)
-        //   smoother colour     half of a two-colour sweep s(3 n_c + 4 n_f) + n_f/8
-        //                       (x, b, alpha read once, x written once per sweep)
-        //   zero-start pass     s(2 n_c + 3 n_f) + n_f/8  (b, alpha read, x written; x = 0
-        //                       is not read)
-        //   one-pass sweep      s(3 n_c + 4 n_f) + n_f/8  (both colours)
-        // s: storage of the level-0 multigrid vectors; the Krylov operator of the FP32
-        // path is FP32, that of the BF16 path FP64 on FP32 vectors
-        const double nc = (double)c->ncell, nf = (double)(c->ndof - c->ncell);
-        const int pr = c->prm.precision;
-        const double sv = (pr == ST_FP32) ? 4.0 : (pr == ST_BF16 ? 2.0 : 8.0);
-        if (kind == ST_PROF_SMOOTH) *bytes = 0.5 * (sv * (3.0 * nc + 4.0 * nf) + nf / 8.0);
-        else if (kind == ST_PROF_SWEEP) *bytes = sv * (3.0 * nc + 4.0 * nf) + nf / 8.0;
-        else if (kind == ST_PROF_SMOOTH0) *bytes = sv * (2.0 * nc + 3.0 * nf) + nf / 8.0;
-        else if (kind == ST_PROF_APPLY) {
-            const double sx = (pr == ST_FP64) ? 8.0 : 4.0, sa = (pr == ST_FP32) ? 4.0 : 8.0, sy = sa;
-            *bytes = (sx + sy) * (nc + nf) + sa * nf + nf / 8.0;
-        } else *bytes = sv * (3.0 * nc + 4.0 * nf) + nf / 8.0;
-    }
+    if (bytes) *bytes = c->prof_nb[kind] ? c->prof_bytes[kind] / c->prof_nb[kind] : kind_bytes(c, kind);
     return ST_OK;
 }
 

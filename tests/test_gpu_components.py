@@ -1,11 +1,13 @@
 """Calls of the component entries (st_mg_*) and what they leave behind, and the coarsest
 inverse at the ends of its range, against the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 
 from conftest import rel
 from helpers import oracle_desc, setup, solver_for
-from stokes_to_amd.problems import _split
+from stokes_to_amd.problems import _split, dof_sizes
 
 pytestmark = pytest.mark.gpu
 
@@ -70,3 +72,27 @@ def test_coarsest_inverse_pivots_in_full_precision(make_solver, orc, dim, share,
     mg = orc.MG(dim, (n, n, n if dim == 3 else 1), fixed, pen, nu_pre=0, nu_post=0, omega=1.0, tang=0)
     b = rng.standard_normal(nd)
     assert rel(s.mg_vcycle(b), mg.vcycle(b)) < 1e-10
+
+
+@pytest.mark.parametrize("dim,n,prec", [(2, 64, "fp64"), (2, 128, "bf16"), (3, 16, "fp32"), (3, 32, "fp64")])
+def test_profiled_bytes_are_those_of_the_launches(make_solver, dim, n, prec):
+    """A V(1,2)-cycle's finest-level launches where they do more than one step: in 2D a launch
+    from x = 0 and one of two sweeps after the prolongation, and the residual that writes the
+    coarse right-hand side only."""
+    P, rho = setup(dim, n)
+    s = solver_for(make_solver, P, rho, precision=prec)
+    s.lib.st_profile(s.h, 1)
+    st = s.solve()[1]
+
+    def read(kind):
+        ms, cnt, by = ctypes.c_double(), ctypes.c_long(), ctypes.c_double()
+        assert s.lib.st_profile_read(s.h, kind, ctypes.byref(ms), ctypes.byref(cnt), ctypes.byref(by)) == 0
+        return cnt.value, by.value
+
+    sv, nv, nf = {"fp64": 8, "fp32": 4, "bf16": 2}[prec], s.ndof, s.ndof - s.ncell
+    coarse = dof_sizes(dim, n // 2)[-1]
+    assert read(2) == (st["iters"], sv * (2 * nv + nf + coarse) + nf / 8)
+    if dim == 2:
+        zero, prol = sv * (2 * nv + nf) + nf / 8, sv * (3 * nv + nf + coarse) + nf / 8
+        assert read(4) == (2 * st["iters"], (zero + prol) / 2)
+        assert read(0)[0] == read(3)[0] == 0
