@@ -1,12 +1,13 @@
 """Kernels that a converging solve would hide an error of, against the oracle: the marched
 smoother at the sizes that run it, the V-cycle in FP32 and BF16 storage and on every kind of
-level."""
+level, and the operator inside FGMRES."""
 import numpy as np
 import pytest
 
 from conftest import rel
 from helpers import oracle_desc, setup, solver_for
 from test_gpu_coarse import scattered
+from test_gpu_components import open_low_sides
 
 pytestmark = pytest.mark.gpu
 
@@ -53,3 +54,27 @@ def test_vcycle_through_a_padded_inner_level_matches_oracle(make_solver, orc):
     mg = orc.MG(3, P.shape, fixed, pen, nu_pre=1, nu_post=2, omega=1.0, tang=0)
     b = np.random.default_rng(7).standard_normal(fixed.size)
     assert rel(s.mg_vcycle(b), mg.vcycle(b)) < 1e-10
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-9), ("fp32", 1e-4)])
+def test_fgmres_steps_use_the_oracle_s_operator(make_solver, orc, prec, tol):
+    """Three steps of FGMRES from zero, with free faces on the low sides: the solution is that of
+    the same steps with the oracle's operator (k_fine inside the solver) and the library's
+    V-cycle, to rounding."""
+    P, rho = setup(3, 64)
+    open_low_sides(P, 64)
+    fixed, vol, pen = oracle_desc(orc, P, rho)
+    b = np.where(fixed.astype(bool), 0.0, np.random.default_rng(9).standard_normal(fixed.size))
+    s = solver_for(make_solver, P, rho, precision=prec, max_iter=3)
+    s.update_b(body=b)
+    x, _ = s.solve(allow_noconv=True)
+    V, Z, H = [b / np.linalg.norm(b)], [], np.zeros((4, 3))
+    for j in range(3):
+        Z.append(s.mg_vcycle(V[j]))
+        w = orc.apply(3, P.shape, fixed, vol, pen, Z[j])
+        H[:j + 1, j] = [v @ w for v in V]
+        w = w - sum(h * v for h, v in zip(H[:, j], V))
+        H[j + 1, j] = np.linalg.norm(w)
+        V.append(w / H[j + 1, j])
+    y = np.linalg.lstsq(H, np.r_[np.linalg.norm(b), 0, 0, 0], rcond=None)[0]
+    assert rel(x, sum(c * z for c, z in zip(y, Z))) < tol
