@@ -1,11 +1,12 @@
 """Kernels that a converging solve would hide an error of, against the oracle: the marched
 smoother at the sizes that run it, the V-cycle in FP32 and BF16 storage and on every kind of
-level, and the operator inside FGMRES."""
+level, the operator inside FGMRES, and large host arrays."""
 import numpy as np
 import pytest
 
 from conftest import rel
-from helpers import oracle_desc, setup, solver_for
+from helpers import DeviceArray, oracle_desc, setup, solver_for
+from stokes_to_amd.problems import channel_problem
 from test_gpu_coarse import scattered
 from test_gpu_components import open_low_sides
 
@@ -78,3 +79,22 @@ def test_fgmres_steps_use_the_oracle_s_operator(make_solver, orc, prec, tol):
         V.append(w / H[j + 1, j])
     y = np.linalg.lstsq(H, np.r_[np.linalg.norm(b), 0, 0, 0], rcond=None)[0]
     assert rel(x, sum(c * z for c, z in zip(y, Z))) < tol
+
+
+def test_large_host_arrays_reach_the_device_whole(make_solver, orc):
+    """128^3, where a vector goes up through the slots too (68 MB): the operator on a host array
+    gives the bits of the operator on a device vector copied there by the runtime, and the
+    sensitivity of two host vectors is the oracle's (1e-13)."""
+    P = channel_problem(3, 128)
+    rng = np.random.default_rng(1)
+    rho = rng.uniform(0.1, 0.9, 128 ** 3)
+    s = solver_for(make_solver, P, rho, restart=2, warm_order=0)
+    x, lam = rng.standard_normal(s.ndof), rng.standard_normal(s.ndof)
+    dx, dy = DeviceArray(x), DeviceArray(np.zeros(s.ndof))
+    assert s.lib.st_apply_device(s.h, dx.ptr, dy.ptr) == 0
+    assert np.array_equal(s.applyMapping(x), dy.get())
+    nc = 128 ** 3
+    ref = orc.sensitivity(3, P.shape, rho, P.alpha.array(), P.fixed[nc:], x[nc:], lam[nc:])
+    assert rel(s.sensitivity(rho, x, lam), ref) < 1e-13
+    dx.free()
+    dy.free()
