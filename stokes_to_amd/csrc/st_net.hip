@@ -686,7 +686,8 @@ long wg_xs_elems(int R, int cin)
     const long P = R + 2;
     return (long)(cin / 16) * 3 * 16 * P * P * R;
 }
-bool wg_staged_ok(int R) { return R >= 4 && R % 4 == 0 && R <= 128; }
+// (the staging kernel counts the gradient's values in 32 bits)
+bool wg_staged_ok(int R, int cout) { return R >= 4 && R % 4 == 0 && R <= 128 && (long)R * R * R * cout <= 1L << 30; }
 // segment sums of gW = sum over voxels of x(v + o_t) gz(v) for every tap (part2) and of
 // gb = sum over voxels of gz(v) (part2 + WG_G ntap cin cout), and gz itself from gy and
 // the activation y (xs, gs: staging buffers of wg_xs_elems(R, cin) and R^3 cout elements).
@@ -711,7 +712,8 @@ void wgrad_staged(int R, int ntap, int cin, int cout, const bf16 *x, int csx, in
     hipLaunchKernelGGL(k_rowsum_parts, dim3(WG_G, cout), dim3(256), 0, s, nv, gs, part2 + WG_G * nw);
 }
 
-// the convolution kernel for the layer's input channels
+// the convolution kernel for the layer's input channels (those with a kernel of their own
+// address the input in 32 bits)
 template <int OUTM, bool RELU>
 void conv27(dim3 grid, int R, const bf16 *in, int csi, int cio, int ncib, const bf4 *Wp, const float *bias, void *out,
             int cso, int coo, int ncob, hipStream_t s)
@@ -719,7 +721,7 @@ void conv27(dim3 grid, int R, const bf16 *in, int csi, int cio, int ncib, const 
 #define ST_CONV(N)                                                                                                    \
     hipLaunchKernelGGL((k_conv<27, N, OUTM, RELU>), grid, dim3(256), 0, s, R, in, csi, cio, ncib, Wp, bias, out, cso, \
                        coo, ncob)
-    switch (ncib) {
+    switch ((long)R * R * R * csi <= 1L << 31 ? ncib : 0) {
     case 1: ST_CONV(1); break;
     case 2: ST_CONV(2); break;
     case 3: ST_CONV(3); break;
@@ -801,7 +803,7 @@ struct NetImpl {
         const NetLayerSpec &p = L[l].sp;
         const int Rl = res(p.lvl);
         const long n = nv(p.lvl);
-        if (wg_staged_ok(Rl)) {
+        if (wg_staged_ok(Rl, p.cout)) {
             wgrad_staged(Rl, p.ntap, p.cin, p.cout, x, csx, cix, y, csy, cy, gy, csg, cg, p.relu, gz, wxs, wgs, L[l].part2, s);
             return;
         }
@@ -939,7 +941,7 @@ NetImpl *net_create(int R, int max_samples, unsigned seed, hipStream_t s)
         tb.p2[l] = -1;
         n->npar += L.nw + L.sp.cout;
         n->npk += L.nw / 4;
-        if (wg_staged_ok(Rl)) {
+        if (wg_staged_ok(Rl, L.sp.cout)) {
             tb.p2[l] = np2;
             np2 += WG_G * (L.nw + L.sp.cout);
             wgx = std::max(wgx, wg_xs_elems(Rl, L.sp.cin));
@@ -1203,7 +1205,7 @@ int net_conv_test(int R, int ntap, int cin, int cout, int relu, int mode, const 
         if (ntap == 27) conv27<1, false>(grid, R, bgo, cout, 0, cout / 16, Wq, nullptr, dout, cin, 0, cin / 16, s);
         else hipLaunchKernelGGL((k_conv<1, 0, 1, false>), grid, dim3(256), 0, s, R, bgo, cout, 0, cout / 16, Wq, (const float *)nullptr, (void *)dout, cin, 0, cin / 16);
         hipMemcpy(out, dout, nv * cin * 4, hipMemcpyDeviceToHost);
-    } else if (wg_staged_ok(R)) {
+    } else if (wg_staged_ok(R, cout)) {
         bf16 *xs = (bf16 *)A(wg_xs_elems(R, cin) * 2), *gs = (bf16 *)A(nv * cout * 2);
         float *wpart2 = (float *)A((long)WG_G * (nw + cout) * 4), *dg = (float *)A((nw + cout) * 4);
         wgrad_staged(R, ntap, cin, cout, bin, cin, 0, nullptr, 0, 0, dgo, cout, 0, 0, bgo, xs, gs, wpart2, s);
