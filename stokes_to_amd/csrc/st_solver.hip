@@ -394,7 +394,7 @@ static double resid_restrict_bytes(const st_ctx *c)
 // the other (x and t).  Whether the cycle's first launch writes x, so that its last does:
 static bool first_writes_x(const st_ctx *c)
 {
-    auto launches = [](int nu) { return (nu + ST_SWEEPS - 1) / ST_SWEEPS; };
+    auto launches = [](int nu) { return nu > 0 ? (nu + ST_SWEEPS - 1) / ST_SWEEPS : 0; };
     return (launches(c->prm.nu_pre) + launches(c->prm.nu_post)) % 2 == 1;
 }
 // nu sweeps of the 2D level l from cur (zero: from 0; ec: from cur + P ec); cur ends at the result

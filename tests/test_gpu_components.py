@@ -96,3 +96,15 @@ def test_profiled_bytes_are_those_of_the_launches(make_solver, dim, n, prec):
         zero, prol = sv * (2 * nv + nf) + nf / 8, sv * (3 * nv + nf + coarse) + nf / 8
         assert read(4) == (2 * st["iters"], (zero + prol) / 2)
         assert read(0)[0] == read(3)[0] == 0
+
+
+@pytest.mark.parametrize("dim,n", [(2, 64), (2, 128), (3, 16)])
+@pytest.mark.parametrize("nu,same", [((1, -3), (1, 0)), ((-3, 2), (0, 2)), ((-4, 1), (0, 1))])
+def test_negative_sweep_counts_mean_no_sweeps(make_solver, orc, dim, n, nu, same):
+    """st_create takes them; 1e-10 of the oracle's V-cycle without these sweeps."""
+    P, rho = setup(dim, n, sigma=4.0)
+    fixed, vol, pen = oracle_desc(orc, P, rho)
+    s = solver_for(make_solver, P, rho, nu_pre=nu[0], nu_post=nu[1])
+    mg = orc.MG(dim, P.shape, fixed, pen, nu_pre=same[0], nu_post=same[1], omega=1.0, tang=0)
+    b = np.random.default_rng(7).standard_normal(fixed.size)
+    assert rel(s.mg_vcycle(b), mg.vcycle(b)) < 1e-10
