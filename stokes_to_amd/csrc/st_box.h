@@ -1,8 +1,9 @@
 // One cell of the box-Vanka smoother and one node of the residual, written over an
 // accessor of the neighbouring nodes, for the levels that are not marched plane by
-// plane (st_coarse.hip).  The rows, their order of operations and the block solve are
-// those of Sten and smooth_cell in st_kernels.hip, so every kernel built on these
-// gives the same bits in FP32 and BF16.
+// plane (st_coarse.hip).  The rows and their order of operations are those of Sten in
+// st_kernels.hip (FINE: of the marching kernels in st_march.hip), the block solve is that
+// of the marched smoother, so every kernel built on these gives the same bits in FP32 and
+// BF16.
 //
 // An accessor A has, at node offsets (di, dj, dk) from its own node,
 //   X(f, di, dj, dk)   field f of x (0: p, 1 + d: velocity d), in the compute type
@@ -99,7 +100,8 @@ template <bool FINE, typename C> __device__ __forceinline__ C box_quo(C a, C b)
 }
 
 // new values of the cell's pressure and of its low (u0) and high (u1) faces after the
-// exact solve of its block (smooth_cell of st_kernels.hip); ZERO: x is zero and not read
+// exact solve of its block: the Schur complement of the pressure in a free cell,
+// Sherman-Morrison (K = E - b b^T) in a fixed one; ZERO: x is zero and not read
 template <typename C, int DIM, bool ZERO, bool FINE = false, typename A>
 __device__ __forceinline__ void box_cell(const A &a, float omega, C &pn, C *u0n, C *u1n)
 {

@@ -12,7 +12,8 @@
 //                     256^3 FP64  FP32   128^3 FP64  FP32   64^3 FP64  FP32
 //   y = A x           540 -> 443  262 -> 225   88 -> 66  35 -> 24   31 -> 10  24 -> 9
 //   r = b - A x       627 -> 528  316 -> 245  101 -> 73  44 -> 32   36 -> 13  28 -> 10
-// At 256^3 that is 3.7 to 4.6 TB/s of HBM traffic (FP32 0.83 / 1.14 GB, near the least).
+// At 256^3 the HBM traffic is 1.79 / 2.30 GB in FP64 and 0.84 / 1.13 GB in FP32, 1.1 to 1.2
+// times the least, at 3.5 to 4.4 TB/s.
 // Without the masks it gains 10% in FP64 and nothing in FP32, and with fewer registers
 // or other block orders nothing: the mix of 9 to 15 streams and short waves bounds it.
 #include "st_box.h"

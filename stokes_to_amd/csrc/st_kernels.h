@@ -140,8 +140,9 @@ void march_residual_f32(const Lvl &, const uint8_t *, const double *al, const do
 template <typename TS> void fine_apply(const Lvl &, const uint8_t *, const TS *, const TS *, TS *, hipStream_t);
 template <typename TS>
 void fine_residual(const Lvl &, const uint8_t *, const TS *, const TS *b, const TS *x, TS *r, double *part, hipStream_t);
-// FP64 operator applied to an FP32-stored vector (x float, alpha and y double)
+// FP64 operator on vectors in the caller's layout
 void user_apply(const Lvl &, const uint8_t *, const double *al, const double *x, double *y, hipStream_t);
+// FP64 operator applied to an FP32-stored vector (x float, alpha and y double)
 void fine_apply_mixed(const Lvl &, const uint8_t *, const double *al, const float *x, double *y, hipStream_t);
 unsigned fine_blocks(const Lvl &);
 // one red-black sweep (colour col0, then the other) in one pass (st_sweep.hip);

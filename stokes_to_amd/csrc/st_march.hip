@@ -387,7 +387,7 @@ __global__ void __launch_bounds__(BJ * 64) k_march(Lvl g, const uint8_t *__restr
                 a0[d] = m0[d] * (clo[d] + mc + C(4)) + al0 + (C(1) - m0[d]) + (C(1) - mc) * m0[d];
                 a1[d] = m1[d] * (mc + chi[d] + C(4)) + al1 + (C(1) - m1[d]) + (C(1) - mc) * m1[d];
             }
-            // block solve of st_kernels.hip smooth_cell: Schur complement in a free
+            // block solve of st_box.h box_cell: Schur complement in a free
             // cell, Sherman-Morrison (K = E - b b^T) in a fixed cell
             C beta = C(0), tb = C(0);
             C of[3], id[3];

@@ -810,7 +810,7 @@ int st_create(st_ctx **out, const st_params *p)
             if (rc == ST_OK) rc = dvec(c, pp, c->nvec, g0);
         }
     // partial sums: 33 vectors of the Krylov kernels' blocks, or one per block of a residual
-    // or of the objective (more than that from 512^3 and 2D 16384^2)
+    // or of the objective (more than that at 512^3)
     c->npart = std::max(8192 * 33, (int)std::max(std::max(residual_blocks(g0), plain_residual_blocks(g0)), energy_blocks(g0)));
     if (rc == ST_OK) rc = dalloc(c, &c->part, c->npart);
     if (rc == ST_OK && hipHostMalloc((void **)&c->red, sizeof(double) * 4 * 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)

@@ -14,7 +14,7 @@
 // it: the first colour is recomputed on that ring by every tile that needs it (and on
 // two planes before and after the chunk), so no workgroup waits for another.  Every
 // block update uses the arithmetic of the two-pass kernel (the exact closed-form block
-// solve of st_kernels.hip smooth_cell), so the result equals two colour passes; the
+// solve of st_box.h box_cell), so the result equals two colour passes; the
 // intermediate x' stays in FP32 in LDS (with BF16 storage it is not rounded to BF16
 // between the colours).
 //
@@ -43,7 +43,7 @@ __device__ __forceinline__ int m2(int p) { return p & 1; }
 __device__ __forceinline__ int m3(int p) { return (p + 9) % 3; }  // p >= -9
 __device__ __forceinline__ float rcpf_(float x) { return __builtin_amdgcn_rcpf(x); }
 
-// closed-form block solve of one cell (st_kernels.hip smooth_cell, st_march.hip), in
+// closed-form block solve of one cell (st_box.h box_cell, st_march.hip), in
 // the operation order of the two-pass kernel: inputs the 7 residuals, masks and
 // diagonal entries; outputs dp and the two face corrections per axis, times omega
 struct Blk {
